@@ -6,8 +6,9 @@ Every translation unit is compiled with packed FP32 disabled.  The ghost-fill /
 geometry and reduction units are compiled without floating-point contraction so
 that their results round exactly like the reference's float64 host arithmetic; the
 RHS unit contracts multiply-adds into FMAs.  The FP64 and Hybrid FP32-bulk flux kernels
-(flux_ilp.hip) are scheduled by LLVM's max-ILP machine scheduler.  The persistent stage
-kernel (stage.hip) and its bodies (stage_off.hip, stage_fast.hip) are relocatable device
+(flux_ilp.hip) are scheduled by LLVM's max-ILP machine scheduler.  The box flux kernels
+(fluxbox.hip) write their multiply-adds out and honour the contraction pragmas.  The persistent stage
+kernel (stage.hip) and its bodies (stage_off.hip, stage_fast.hip, stage_box.hip) are relocatable device
 code, device-linked into the same library.
 """
 import os
@@ -34,6 +35,7 @@ UNITS = {
     "flux.hip": ["-ffp-contract=fast"],
     "flux_ilp.hip": ["-ffp-contract=fast", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "flux3.hip": ["-ffp-contract=fast"],
+    "fluxbox.hip": ["-ffp-contract=fast-honor-pragmas"],
     "mlp.hip": ["-ffp-contract=fast"],
     "ops.hip": ["-ffp-contract=fast"],
     "capi.hip": [],
@@ -41,6 +43,7 @@ UNITS = {
     # with the FP contraction of the unit whose kernels it shares code with
     "stage_off.hip": ["-ffp-contract=off", "-fgpu-rdc"],
     "stage_fast.hip": ["-ffp-contract=fast", "-fgpu-rdc"],
+    "stage_box.hip": ["-ffp-contract=fast-honor-pragmas", "-fgpu-rdc"],
     "stage.hip": ["-fgpu-rdc"],
 }
 

@@ -120,7 +120,8 @@ struct wmx_plan {
   std::vector<InflowDev> inflows;
   // workspace
   size_t ws_bytes = 0;
-  std::vector<size_t> off_P, off_G, off_shell, off_sponge, off_geo32, off_sb;
+  std::vector<size_t> off_P, off_G, off_shell, off_sponge, off_geo32, off_sb, off_box;
+  bool box = false;                   // every block's metrics are tensor products (box.h)
   std::vector<std::vector<long long>> off_wall;   // per block, 6 faces (-1: none)
   size_t off_part = 0, off_scal = 0, off_stat = 0;
   double* d_stat = nullptr;           // plane-statistics partials
@@ -136,7 +137,7 @@ struct wmx_plan {
   Ptrs* d_pbuf = nullptr;
   int* d_fill_off = nullptr;
   int* d_fill_max = nullptr;
-  int stage_grid = 0, stage_grid_f = 0;   // persistent grids in use (0: not yet launched)
+  int stage_grid[3] = {0, 0, 0};      // persistent grids in use, per kernel form (0: not yet launched)
   // kernel-class event timing
   int prof_mask = 0;
   std::vector<hipEvent_t> ev_pool;
@@ -376,12 +377,48 @@ int auto_ci_len(int nb, const int* dims, int prec, int cu_count, long long* ntil
   return best;
 }
 
+// The flux launches of a plan run the box kernels (box.h): every block's metrics are tensor
+// products, and an FP32-bulk plan evaluates its gradients in the march.
+bool box_active(const wmx_plan* p) { return p->box && (p->nd.prec != WMX_PREC_FP32_BULK || p->fuse_grad); }
+
+// i-planes per tile of the box kernels when none is requested.  W workgroups share a CU (3 in
+// FP32, 2 in FP64), so T tiles are r full rounds of W CUs slots and a remainder.  A plane of a
+// full round takes one unit; with k workgroups on a CU it takes t(k), measured on the
+// 256 x 128 x 128 channel: 0.54 / 0.81 / 1 (FP32, 8.9 us), 0.62 / 1 (FP64, 11.8 us), between
+// them in proportion to the mean occupancy.  A tile costs its planes plus one.  Short chunks
+// are allowed down to one plane: below one workgroup per CU a launch is the serial march of
+// one tile (24 x 16 x 12 cells, FP64: 30.9 us at four planes, 15.5 us at one).  The shortest
+// estimate over ci in [1, 64] wins, ties to the shorter chunk (256 x 128 x 128, FP32: 8 planes,
+// three full rounds, 253 us; 26 planes, 267 us; 37 planes, 302 us).
+int box_ci_len(const wmx_plan* p) {
+  const bool f32 = p->nd.prec == WMX_PREC_FP32_BULK;
+  const double t32[4] = {0.54, 0.54, 0.81, 1.0}, t64[3] = {0.62, 0.62, 1.0};
+  const double* t = f32 ? t32 : t64;
+  const long long cus = std::max(1, p->cu_count), W = f32 ? 3 : 2;
+  int best = 1;
+  double best_cost = 1e300;
+  for (int ci = 1; ci <= 64; ++ci) {
+    long long T = 0;
+    for (const BlockDev& B : p->hb)
+      T += (long long)((B.n[0] + ci - 1) / ci) * ((B.n[1] + FLUX2_TILE_J - 1) / FLUX2_TILE_J) * ((B.n[2] + 15) / 16);
+    const long long r = T / (W * cus), m = T - r * W * cus;
+    const double x = (double)m / (double)cus;
+    const int k = (int)x;
+    const double rest = m == 0 ? 0.0 : (k >= W ? 1.0 : t[k] + (x - k) * (t[k + 1] - t[k]));
+    const double cost = ((double)r + rest) * (ci + 1);
+    if (cost < best_cost - 1e-9) { best_cost = cost; best = ci; }
+  }
+  return best;
+}
+
 void build_tiles(wmx_plan* p) {
   std::vector<int4> t;
-  // tile rows of both flux kernels
+  // tile rows of the flux kernels
   const int tjr = FLUX2_TILE_J;
   if (p->ci_req > 0) {
     p->ci_len = p->ci_req;
+  } else if (box_active(p)) {
+    p->ci_len = box_ci_len(p);
   } else {
     std::vector<int> dims;
     for (int b = 0; b < p->nb; ++b) dims.insert(dims.end(), p->hb[b].n, p->hb[b].n + 3);
@@ -405,6 +442,16 @@ void build_tiles(wmx_plan* p) {
     t.swap(o);
   }
   p->tiles.swap(t);
+}
+
+// the tile table rebuilt and uploaded (workspace bound, tiling or kernel form changed)
+int retile(wmx_plan* p) {
+  build_tiles(p);
+  (void)hipFree(p->d_tiles);
+  p->d_tiles = nullptr;
+  if (upload(p->tiles, &p->d_tiles)) return 1;
+  p->stage_dirty = true;
+  return 0;
 }
 
 NumDev make_numdev(const wmx_numerics_desc* nm) {
@@ -498,13 +545,14 @@ int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef,
                                p->d_case_off_all, p->d_part, nullptr, dt_out, s);
     }));
   }
-  // fused FP32-bulk plans: the flux kernel evaluates the gradient records itself; the
-  // gradient launch keeps only its head work (per-case dt min, Newton wall faces)
-  const bool grads = !(f32 && p->fuse_grad);
-  WMX_CHECK(timed(p, K_GRAD, s, [&] {
-    return launch_grad(p->d_blks, p->d_pre_box, p->nb, grads ? nwg_of(p->pre_box) : 0, p->nd,
-                       wall_in_grad ? p->d_wall : nullptr, (int)p->wall.size(), p->wall_max, q, gdt, s);
-  }));
+  // fused FP32-bulk plans and box plans: the flux kernel evaluates the gradient records
+  // itself; the gradient launch keeps only its head work (per-case dt min, Newton wall faces)
+  const bool grads = !((f32 && p->fuse_grad) || box_active(p));
+  if (grads || gdt.out || wall_in_grad)
+    WMX_CHECK(timed(p, K_GRAD, s, [&] {
+      return launch_grad(p->d_blks, p->d_pre_box, p->nb, grads ? nwg_of(p->pre_box) : 0, p->nd,
+                         wall_in_grad ? p->d_wall : nullptr, (int)p->wall.size(), p->wall_max, q, gdt, s);
+    }));
   if (!wall_in_grad && !wall_in_prim)
     WMX_CHECK(timed(p, K_WALL, s, [&] { return launch_wall(p->d_blks, p->d_wall, (int)p->wall.size(), p->wall_max, q, p->nd, s); }));
   if (p->nd.n_sponge > 0 && !p->d_sponge_pre)
@@ -518,6 +566,8 @@ int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef,
 hipError_t plan_flux(const wmx_plan* p, int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles,
                      int ci_len, const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
                      hipStream_t s) {
+  if (box_active(p))
+    return launch_box(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
   if (nd.prec == WMX_PREC_FP32_BULK && p->fuse_grad)
     return launch_flux3(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
   return launch_flux(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
@@ -765,6 +815,8 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
                                             (size_t)B.cells));
     p->off_sb.push_back(off);
     off = align_up(off + sizeof(double) * NSB_PLANES * (size_t)B.cells);
+    p->off_box.push_back(off);
+    off = align_up(off + sizeof(BoxEnt) * (size_t)(B.N[0] + B.N[1] + B.N[2]));
     p->off_shell.push_back(off);
     off = align_up(off + sizeof(double) * 5 * B.shell_cells);
     p->off_sponge.push_back(off);
@@ -793,7 +845,7 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
   p->ws_bytes = off;
   // device metadata
   std::vector<int> cdir(p->case_dir.begin(), p->case_dir.end());
-  if (upload(p->ops, &p->d_ops) || upload(p->wall, &p->d_wall) || upload(p->tiles, &p->d_tiles) ||
+  if (upload(p->ops, &p->d_ops) || upload(p->wall, &p->d_wall) ||
       upload(p->pre_all, &p->d_pre_all) || upload(p->pre_box, &p->d_pre_box) ||
       upload(p->pre_int, &p->d_pre_int) || upload(p->pre_shell, &p->d_pre_shell) ||
       upload(p->case_wg, &p->d_case_wg) || upload(p->case_off, &p->d_case_off) ||
@@ -874,6 +926,9 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
       B.volf = nullptr;
     }
     B.Sb = reinterpret_cast<double*>(p->ws + p->off_sb[b]);
+    B.box[0] = reinterpret_cast<const BoxEnt*>(p->ws + p->off_box[b]);
+    B.box[1] = B.box[0] + B.N[0];
+    B.box[2] = B.box[1] + B.N[1];
     B.shell = reinterpret_cast<double*>(p->ws + p->off_shell[b]);
     B.sponge_mean = reinterpret_cast<double*>(p->ws + p->off_sponge[b]);
     B.sponge_row = p->nd.n_sponge > 0
@@ -892,13 +947,20 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
   // loads the dt skips; the kernel ORs the non-zero planes into one word per block, kept in
   // the partials buffer (at least two doubles per block, unused until the first step).
   WMX_CHECK(hipDeviceSynchronize());
+  // The box check's word follows them.
   unsigned* d_nz = reinterpret_cast<unsigned*>(p->d_part);
-  WMX_CHECK(hipMemset(d_nz, 0, sizeof(unsigned) * p->nb));
-  for (int b = 0; b < p->nb; ++b) WMX_CHECK(launch_cell_sb(p->hb[b], d_nz + b, nullptr));
+  unsigned* d_bad = d_nz + p->nb;
+  WMX_CHECK(hipMemset(d_nz, 0, sizeof(unsigned) * (p->nb + 1)));
+  for (int b = 0; b < p->nb; ++b) {
+    WMX_CHECK(launch_cell_sb(p->hb[b], d_nz + b, nullptr));
+    WMX_CHECK(launch_box_check(p->hb[b], d_bad, nullptr));
+  }
   WMX_CHECK(hipDeviceSynchronize());
   {
-    std::vector<unsigned> nz(p->nb);
-    WMX_CHECK(hipMemcpy(nz.data(), d_nz, sizeof(unsigned) * p->nb, hipMemcpyDeviceToHost));
+    std::vector<unsigned> nz(p->nb + 1);
+    WMX_CHECK(hipMemcpy(nz.data(), d_nz, sizeof(unsigned) * (p->nb + 1), hipMemcpyDeviceToHost));
+    p->box = nz[p->nb] == 0;
+    if (retile(p)) return 1;
     for (int b = 0; b < p->nb; ++b)
       p->hb[b].sb_zero = p->hb[b].Sb ? (int)(~nz[b] & ((1u << NSB_PLANES) - 1u)) : 0;
     WMX_CHECK(hipMemcpy(p->d_blks, p->hb.data(), sizeof(BlockDev) * p->nb, hipMemcpyHostToDevice));
@@ -1234,7 +1296,8 @@ int advance_persistent(wmx_plan* p, double* const* q0, double* const* qout, doub
     c.d_dt = d_dt;
     c.dt_host = dt;
     WMX_CHECK(timed(p, K_FLUX, s, [&] {
-      return launch_stage(mode, sc, p->fuse_grad, p->d_stage, c, p->fuse_grad ? &p->stage_grid_f : &p->stage_grid, s);
+      const int form = box_active(p) ? 2 : (p->fuse_grad ? 1 : 0);
+      return launch_stage(mode, sc, form, p->d_stage, c, &p->stage_grid[form], s);
     }));
   }
   WMX_CHECK(launch_shell_finish(1, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), P0, PO, d_dt, dt, s));
@@ -1362,19 +1425,15 @@ int wmx_plan_set_tiling(wmx_plan* p, int32_t ci_len, int32_t order) {
   if (order != 0 && order != 1) return fail("order must be 0 or 1");
   p->ci_req = ci_len;
   p->tile_order = order;
-  build_tiles(p);
-  (void)hipFree(p->d_tiles);
-  p->d_tiles = nullptr;
-  if (upload(p->tiles, &p->d_tiles)) return 1;
+  if (retile(p)) return 1;
   drop_graphs(p);
-  p->stage_dirty = true;
   return 0;
 }
 
 int wmx_plan_set_fused_gradients(wmx_plan* p, int32_t on) {
   if (check_plan(p)) return 1;
   p->fuse_grad = on != 0;
-  p->stage_dirty = true;
+  if (retile(p)) return 1;
   drop_graphs(p);
   return 0;
 }

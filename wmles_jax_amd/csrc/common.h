@@ -26,6 +26,14 @@ struct Ptrs {
   double* p[WMX_MAX_BLOCKS];
 };
 
+// Metrics of a box (tensor-product) block along one axis, per ghosted index: cell width,
+// its reciprocal and cube root, centroid coordinate, reciprocal distance to the lower
+// neighbour's centroid (FP64, and as the FP32 faces form it).
+struct BoxEnt {
+  double w, iw, cb, x, id;
+  float idf, df;            // (df: the distance itself, signed)
+};
+
 struct BlockDev {
   int n[3];
   int N[3];
@@ -57,6 +65,7 @@ struct BlockDev {
   // e' = e_int - e_ref with e_ref = R T_gauge / (gamma - 1)
   double p_ref, T_gauge, e_ref;
   wmx_face_desc faces[6];
+  const BoxEnt* box[3];     // per-axis metrics (read by the kernels of box plans only)
 };
 
 // Learned wall model handed to the wall kernels; w == nullptr selects the Newton model.
@@ -165,6 +174,12 @@ hipError_t launch_flux(int mode, const BlockDev* d_blks, const int4* d_tiles, in
 hipError_t launch_flux3(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
                         const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
                         hipStream_t s);
+// the same for plans whose blocks are all boxes (box.h), both precisions; no gradient launch
+hipError_t launch_box(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
+                      const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
+                      hipStream_t s);
+// fills a block's BoxEnt tables; *d_bad becomes non-zero if the block is no box
+hipError_t launch_box_check(const BlockDev& hb, unsigned* d_bad, hipStream_t s);
 hipError_t launch_shell_save(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
                              hipStream_t s);
 hipError_t launch_shell_finish(int mode, const BlockDev* d_blks, const int* d_pre, int nblk, int nwg,
@@ -245,10 +260,10 @@ struct StageCall {
   const double* d_dt;
   double dt_host;
 };
-// fused: the fused kernel form (gradient records in the flux march, wall faces in the
-// primitive head).  grid: workgroups of the persistent grid (0: the co-resident maximum, a
+// form: 0 gradient launch and flux2 tiles, 1 the fused form (gradient records in the flux
+// march, wall faces in the primitive head), 2 the fused form with box tiles.  grid: workgroups of the persistent grid (0: the co-resident maximum, a
 // multiple of 8, returned in *grid_used)
-hipError_t launch_stage(int mode, int sc, bool fused, const StageStatic* d_st, const StageCall& c,
+hipError_t launch_stage(int mode, int sc, int form, const StageStatic* d_st, const StageCall& c,
                         int* grid_used, hipStream_t s);
 
 hipError_t launch_scheme_flux(const NumDev& nd, const int* n, int d, const double* w, const double* S,

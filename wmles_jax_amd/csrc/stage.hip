@@ -8,7 +8,7 @@
 // XCDs' L2 caches, so the phases see each other's stores).  Work item w of a phase is
 // taken by workgroup w mod grid, so with a grid that is a multiple of 8 it runs on XCD
 // w mod 8 as in the separate launches, whose XCD-span orderings (xcd_span, the tile order)
-// carry over.  The bodies are the separate kernels' own (stage_off.hip / stage_fast.hip,
+// carry over.  The bodies are the separate kernels' own (stage_off.hip / stage_fast.hip / stage_box.hip,
 // device-linked with their units' FP contraction), so the results are the same bits.
 #include <hip/hip_cooperative_groups.h>
 
@@ -27,10 +27,13 @@ template <int MODE, int SC>
 __device__ void st_flux(const StageStatic& s, const double* __restrict__ d_dt, double dt_host, int tile);
 template <int MODE, int SC>
 __device__ void st_flux3(const StageStatic& s, const double* __restrict__ d_dt, double dt_host, int tile);
+template <int MODE, int SC>
+__device__ void st_box(const StageStatic& s, const double* __restrict__ d_dt, double dt_host, int tile);
 
-// FUSED: the fused kernel form (flux3 tiles with the gradient records in the march, wall
-// faces in the primitive head, the gradient list only its dt head)
-template <int MODE, int SC, bool FUSED>
+// FORM 1: the fused kernel form (flux3 tiles with the gradient records in the march, wall
+// faces in the primitive head, the gradient list only its dt head); 2: the same with the box
+// tiles; 0: flux2 tiles after the gradient list
+template <int MODE, int SC, int FORM>
 __global__ __launch_bounds__(256, 2) void k_stage(const StageStatic* __restrict__ st, StageCall c) {
   cg::grid_group grid = cg::this_grid();
   const StageStatic& s = *st;
@@ -64,16 +67,17 @@ __global__ __launch_bounds__(256, 2) void k_stage(const StageStatic* __restrict_
   }
   grid.sync();
   for (int w = (int)blockIdx.x; w < s.ntiles; w += G) {
-    if (FUSED) st_flux3<MODE, SC>(s, c.d_dt, c.dt_host, w);
+    if (FORM == 2) st_box<MODE, SC>(s, c.d_dt, c.dt_host, w);
+    else if (FORM == 1) st_flux3<MODE, SC>(s, c.d_dt, c.dt_host, w);
     else st_flux<MODE, SC>(s, c.d_dt, c.dt_host, w);
     __syncthreads();
   }
 }
 
 namespace {
-template <int MODE, int SC, bool FUSED>
+template <int MODE, int SC, int FORM>
 hipError_t coop(const StageStatic* d_st, const StageCall& c, int grid, int* used, hipStream_t s) {
-  const void* fn = (const void*)k_stage<MODE, SC, FUSED>;
+  const void* fn = (const void*)k_stage<MODE, SC, FORM>;
   if (grid <= 0) {
     int per_cu = 0, dev = 0, cus = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, 0);
@@ -91,11 +95,13 @@ hipError_t coop(const StageStatic* d_st, const StageCall& c, int grid, int* used
 }
 }  // namespace
 
-hipError_t launch_stage(int mode, int sc, bool fused, const StageStatic* d_st, const StageCall& c,
+hipError_t launch_stage(int mode, int sc, int form, const StageStatic* d_st, const StageCall& c,
                         int* grid_used, hipStream_t s) {
   const int grid = grid_used && *grid_used > 0 ? *grid_used : 0;
 #define WMX_STAGE_F(M, C) \
-  return fused ? coop<M, C, true>(d_st, c, grid, grid_used, s) : coop<M, C, false>(d_st, c, grid, grid_used, s);
+  return form == 2   ? coop<M, C, 2>(d_st, c, grid, grid_used, s)  \
+         : form == 1 ? coop<M, C, 1>(d_st, c, grid, grid_used, s)  \
+                     : coop<M, C, 0>(d_st, c, grid, grid_used, s);
 #define WMX_STAGE_M(C)                 \
   switch (mode) {                      \
     case 1: WMX_STAGE_F(1, C)          \
