@@ -19,12 +19,21 @@
 // is off in the functions below and the fused multiply-adds are written out, so every
 // instance (kernel, mode, scheme, persistent stage) rounds the same way.
 //
-// March.  As flux3_tile: at plane I the tile evaluates the gradient records of plane I, the
-// j / k faces of plane I and the own i face I-1/2, and finishes cell I-1.  The i neighbours of
-// a gradient cell come from registers: a thread keeps the records of its own column at I-2 ..
-// I+1, the 46 threads that also own a ring cell keep that cell's (u, v, w, T) at I-1 .. I+1.
-// Thread row tj = 15 owns the column above the tile (its gradient cells and staged records are
-// the upper ring row), so the halo ring is 124 cells.
+// The state is read, not a primitive record: each thread forms the records of its column and
+// of a halo cell one plane ahead (rec_of), so no primitive launch writes 32 / 64 B per cell for
+// this one to read back with a halo.  Channel of 256 x 128 x 128 cells, Hybrid + Vreman, per
+// stage: FP32 307 us against 253 us on records and 78 us that wrote them; FP64 458 us against
+// 461 us + 137 us.  It is bound by vector issue (about 200 us of the FP32 launch) and by the
+// state loads' latency at three (FP64: two) waves per SIMD.
+//
+// March.  At plane I the tile evaluates the gradient records of plane I, the own i face I-1/2,
+// which completes cell I-1, and then the j / k faces of plane I.  The records of planes I-1 and
+// I are in LDS (FP64: I, with I-1 in registers), that of I+1 in registers, I-2 of the own column
+// too.  46 threads evaluate a ring cell's gradient besides their own; thread row tj = 15 owns
+// the column above the tile (the upper ring row), so the halo ring is 124 cells.  Two barriers
+// per plane (FP64: three): the gradient records, and the face exchange together with the next
+// plane's staging.  sched_barriers keep the scheduler from hoisting a phase's LDS loads into
+// the one before: without them the kernels spill 18 to 60 registers and run 1.3 times as long.
 #pragma once
 #include <type_traits>
 
@@ -321,27 +330,22 @@ __device__ __forceinline__ void face_axis(const NumDev& nd, const BCell<R>& L2, 
 }
 
 // Gradient record of a cell from its own (u, v, w, T) c, its six neighbours m / p per axis,
-// the three face areas S, the volume and the filter width: GB planes.  FP32: the Green-Gauss
-// face sums of the general kernels in their rounding; FP64: the central difference itself
-// (S[d] = 1 / width there).
+// S[d] half the face area of axis d, the volume and the filter width: GB planes.  FP32: the
+// Green-Gauss face sums of the general kernels in their rounding (the 1/2 of the face averages
+// taken with the area is exact); FP64: the central difference itself (S[d] = 1 / (2 width)).
 template <class R>
 __device__ __forceinline__ void grad_axis(const NumDev& nd, const R* c, const R (*m)[4], const R (*p)[4],
                                           const R* S, R vol, R delta, R rho, R mu, R* G) {
   R g[9];
   {
 #pragma clang fp contract(off)
-    const R h = R(0.5);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
       for (int v = 0; v < GB<R>::NV; ++v) {
         R x;
-        if constexpr (sizeof(R) == 4) {
-          const R lo = h * (m[d][v] + c[v]), hi = h * (c[v] + p[d][v]);
-          x = fdiv<R>(fm(hi, S[d], -(lo * S[d])), vol);
-        } else {
-          x = (h * (p[d][v] - m[d][v])) * S[d];
-        }
+        if constexpr (sizeof(R) == 4) x = fdiv<R>(fm(c[v] + p[d][v], S[d], -((m[d][v] + c[v]) * S[d])), vol);
+        else x = (p[d][v] - m[d][v]) * S[d];
         G[3 * v + d] = x;
         if (v < 3) g[3 * v + d] = x;
       }
@@ -374,7 +378,7 @@ template <class R, int MODE, int SC>
 __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, const int4* __restrict__ tiles,
                                          int ci_len, const NumDev& nd, const Ptrs& qin, const Ptrs& q0,
                                          const Ptrs& out, const double* __restrict__ d_dt, double dt_host,
-                                         int tile) {
+                                         int zfuse, int tile) {
 #pragma clang fp contract(off)
   constexpr bool F32 = sizeof(R) == 4;
   constexpr int NF = F32 ? 6 : 5;                // exchanged values per face
@@ -412,27 +416,6 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     return jj >= ng - 1 && jj <= ng + n1 && kk >= ng - 1 && kk <= ng + n2;
   };
   const int I0 = ng + i0, Iend = ng + i1;
-  auto load_a = [&](unsigned c, R* a) {          // (u, v, w, T)
-    if constexpr (F32) {
-      const float4 v = ld4((const float*)B.Pf + 4 * (size_t)c);
-      a[0] = v.x; a[1] = v.y; a[2] = v.z; a[3] = v.w;
-    } else {
-#pragma unroll
-      for (int x = 0; x < 3; ++x) a[x] = ldu(B.P + (P_U + x) * (size_t)cells, c);
-      a[3] = ldu(B.P + P_T * (size_t)cells, c);
-    }
-  };
-  auto load_b = [&](unsigned c, R* b) {          // (rho, p, mu, e)
-    if constexpr (F32) {
-      const float4 v = ld4((const float*)B.Pf + 4 * ((size_t)cells + c));
-      b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
-    } else {
-      b[0] = ldu((const double*)B.P, c);
-      b[1] = ldu(B.P + P_P * (size_t)cells, c);
-      b[2] = ldu(B.P + P_MU * (size_t)cells, c);
-      b[3] = ldu(B.P + P_E * (size_t)cells, c);
-    }
-  };
   auto energy = [&](const R* a, R e) {           // E (KEEP: e)
 #pragma clang fp contract(off)
     return keep ? e : fm(R(0.5), fm(a[2], a[2], fm(a[1], a[1], a[0] * a[0])), e);
@@ -448,21 +431,36 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     P[0][s] = c.r; P[1][s] = c.u[0]; P[2][s] = c.u[1]; P[3][s] = c.u[2];
     P[4][s] = c.p; P[5][s] = c.T; P[6][s] = c.E;
   };
+  // a k ghost of a fused side is read at its periodic image
+  const int zf = zfuse ? B.zfuse : 0;
+  auto kcol = [&](int kk) {
+    if ((zf & 1) && kk < ng) return kk + n2;
+    if ((zf & 2) && kk >= ng + n2) return kk - n2;
+    return kk;
+  };
+  const double* qi = qin.p[t.x];
+  auto load_q = [&](unsigned c, double* q) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v] = ldu(qi + v * (size_t)cells, c);
+  };
   // own column (clamped into the array) and its slots
-  const unsigned cb = (unsigned)min(J, N[1] - 1) * N[2] + min(K, N[2] - 1);
+  const unsigned cb = (unsigned)min(J, N[1] - 1) * N[2] + kcol(min(K, N[2] - 1));
   const bool own_p = p_ok(J, K), own_g = g_ok(J, K);
   const int sp_own = (tj + 2) * H2K + (tk + 2), sg_own = (tj + 1) * GB<R>::P + (tk + 1);
-  // halo job: threads 0..45 a ring cell whose gradient record they also evaluate (row -1,
-  // columns -1 and 16), threads 64..141 a cell that is only staged
+  // halo job by ht, the thread index turned by a multiple of 64 that changes from one of an
+  // XCD's workgroups to the next (the jobs of two wavefronts would otherwise fall on the same
+  // two SIMDs of every CU): 0..45 a ring cell whose gradient record the thread also evaluates
+  // (row -1, columns -1 and 16), 46..123 a cell that is only staged
+  const int ht = (tid + 64 * ((tile >> 3) & 3)) & (NT - 1);
   int hj = 0, hk = 0, halo = 0;
-  if (tid < NGRB) {
+  if (ht < NGRB) {
     halo = 2;
-    if (tid < TK) { hj = -1; hk = tid; }
-    else if (tid < TK + C2J) { hj = tid - TK; hk = -1; }
-    else { hj = tid - TK - C2J; hk = TK; }
-  } else if (tid >= 64 && tid < 64 + NHB - NGRB) {
+    if (ht < TK) { hj = -1; hk = ht; }
+    else if (ht < TK + C2J) { hj = ht - TK; hk = -1; }
+    else { hj = ht - TK - C2J; hk = TK; }
+  } else if (ht < NHB) {
     halo = 1;
-    const int x = tid - 64;                      // rows -2 and 16 (20 each), corners of row -1 (4),
+    const int x = ht - NGRB;                     // rows -2 and 16 (20 each), corners of row -1 (4),
     if (x < H2K) { hj = -2; hk = x - 2; }        // columns -2 and 17 of rows 0..15, -1 and 16 of row 15
     else if (x < 2 * H2K) { hj = BJ; hk = x - H2K - 2; }
     else if (x < 2 * H2K + 4) { const int y = x - 2 * H2K; hj = -1; hk = y < 2 ? y - 2 : TK + y - 2; }
@@ -471,7 +469,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
   }
   if (halo && !p_ok(J - tj + hj, K - tk + hk)) halo = 0;
   const bool ring_g = halo == 2 && g_ok(J - tj + hj, K - tk + hk);
-  const unsigned hoff = halo ? (unsigned)(J - tj + hj) * N[2] + (unsigned)(K - tk + hk) : 0;
+  const unsigned hoff = halo ? (unsigned)(J - tj + hj) * N[2] + (unsigned)kcol(K - tk + hk) : 0;
   const int hs = (hj + 2) * H2K + (hk + 2);
   // metric tables of the tile's rows and columns (index 0: row j0 - 1 / column k0 - 1)
   if (tid < 2 * G2K) {
@@ -495,34 +493,38 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
   double iwi_p = iwi;                            // 1 / width of plane I-1
   BCell<R> W0, W1;                               // own records of I-2 and (FP64; FP32: staged) I-1
   R mu0, Hr = R(0), Hm = R(0);                   // mu of the own cell I, rho and mu of the ring cell
-  R na[4], nb[4], Hx[4], Hn[4];                  // records in flight: own column, halo cell
+  double qn[5], hq[5];                           // states in flight: own column, halo cell
+  R mu1, Hx[4], Hn[4];                           // own mu of the next plane, the halo cell's record there
 #pragma unroll
   for (int x = 0; x < 4; ++x) Hx[x] = Hn[x] = R(0);
-  auto request = [&](int p) {                    // the records of plane p
-    load_a((unsigned)p * sI + cb, na);
-    load_b((unsigned)p * sI + cb, nb);
-    if (halo) {
-      load_a((unsigned)p * sI + hoff, Hx);
-      load_b((unsigned)p * sI + hoff, Hn);
-    }
+  auto request = [&](int p) {                    // the states of plane p
+    load_q((unsigned)p * sI + cb, qn);
+    if (halo) load_q((unsigned)p * sI + hoff, hq);
   };
-  auto stage_plane = [&](R (*P)[NP2], const BCell<R>& c) {     // the records in flight
+  auto arrive = [&]() {                          // their records
+    R a[4], b[4];
+    rec_of(nd, qn, B.p_ref, B.T_gauge, B.e_ref, a, b);
+    mu1 = b[2];
+    if (halo) rec_of(nd, hq, B.p_ref, B.T_gauge, B.e_ref, Hx, Hn);
+    return cell_of(a, b);
+  };
+  auto stage_plane = [&](R (*P)[NP2], const BCell<R>& c) {
     if (own_p) stage(P, sp_own, c);
     if (halo) stage(P, hs, cell_of(Hx, Hn));
-    mu0 = nb[2];
+    mu0 = mu1;
     Hr = Hn[0];
     Hm = Hn[2];
   };
   request(I0 - 2);
-  W0 = W1 = cell_of(na, nb);
+  W0 = W1 = arrive();
   if constexpr (F32) {
     stage_plane(sP[NB - 1], W1);
   } else if (halo == 2) {
 #pragma unroll
-    for (int x = 0; x < 3; ++x) sH0[x][tid] = Hx[x];
+    for (int x = 0; x < 3; ++x) sH0[x][ht] = Hx[x];
   }
   request(I0 - 1);
-  stage_plane(sP[0], cell_of(na, nb));
+  stage_plane(sP[0], arrive());
   request(I0);
   // partial outward sum of the own cell I-1 in FP64: its lower i face minus its j / k face sums
   double Cp[NF];
@@ -551,7 +553,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     const bool inner = I >= I0 && I < Iend;      // plane owned by the tile: j / k faces
     const bool fin = act && I >= I0 + 1;         // cell I-1 is finished at this plane
     R (*P)[NP2] = sP[buf];
-    const BCell<R> Pn = cell_of(na, nb);         // own record of I+1
+    const BCell<R> Pn = arrive();                // own record of I+1
     auto cell = [&](const R (*Q)[NP2], int s) {
       BCell<R> w;
       w.r = Q[0][s]; w.u[0] = Q[1][s]; w.u[1] = Q[2][s]; w.u[2] = Q[3][s];
@@ -565,11 +567,11 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       o.mu = sG[GB<R>::MU][g]; o.k = sG[GB<R>::K][g];
       return o;
     };
+    __builtin_amdgcn_sched_barrier(0);
     // ---- cell I-1: its state loads go out first, covered by the gradients and the i face
     const unsigned c = (unsigned)(I - 1) * sI + (unsigned)J * N[2] + K;
     // the stage is base + a1 dt r with base = a0 q0 + a1 q: one value per component is kept
     const double a0 = MODE == 2 ? 0.75 : 1.0 / 3.0, a1 = MODE == 1 ? 1.0 : (MODE == 2 ? 0.25 : 2.0 / 3.0);
-    const double* qi = qin.p[t.x];
     double base[5], vz[5];
     if (MODE >= 1 && fin) {
 #pragma unroll
@@ -594,11 +596,11 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       }
       if constexpr (F32) {
         const double a = sW[0][wj_], b = sW[1][wk_];
-        const R S[3] = {R(a * b), R(wi * b), R(wi * a)}, vol = R((wi * a) * b);
+        const R h = R(0.5), S[3] = {h * R(a * b), h * R(wi * b), h * R(wi * a)}, vol = R((wi * a) * b);
         grad_axis<R>(nd, u, m, p, S, vol, cbrtf(vol), rho, mu, G);
       } else {
         const R delta = R((cbi * sCb[0][wj_]) * sCb[1][wk_]);
-        const R S[3] = {R(iwi), R(sIw[0][wj_]), R(sIw[1][wk_])};
+        const R S[3] = {R(0.5 * iwi), R(0.5 * sIw[0][wj_]), R(0.5 * sIw[1][wk_])};
         grad_axis<R>(nd, u, m, p, S, R(0), delta, rho, mu, G);
       }
     };
@@ -673,7 +675,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
 #pragma unroll
       for (int x = 0; x < GB<R>::NV; ++x) {
         if constexpr (F32) m[x] = sP[NB - 1 - buf][x < 3 ? 1 + x : 5][hs];
-        else m[x] = sH0[x][tid];
+        else m[x] = sH0[x][ht];
       }
       grads(m, Hx, hs, hj + 1, hk + 1, Hr, Hm, Gr);
       const int sg = (hj + 1) * GB<R>::P + (hk + 1);
@@ -730,7 +732,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     if (!F32) {                                  // FP64: one buffer, free after the exchange barrier
       if (ring_g) {
 #pragma unroll
-        for (int x = 0; x < 3; ++x) sH0[F32 ? 0 : x][F32 ? 0 : tid] = P[1 + x][hs];
+        for (int x = 0; x < 3; ++x) sH0[F32 ? 0 : x][F32 ? 0 : ht] = P[1 + x][hs];
       }
       stage_plane(sP[0], Pn);
       request(I + 2);

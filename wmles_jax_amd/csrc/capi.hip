@@ -382,17 +382,18 @@ int auto_ci_len(int nb, const int* dims, int prec, int cu_count, long long* ntil
 bool box_active(const wmx_plan* p) { return p->box && (p->nd.prec != WMX_PREC_FP32_BULK || p->fuse_grad); }
 
 // i-planes per tile of the box kernels when none is requested.  W workgroups share a CU (3 in
-// FP32, 2 in FP64), so T tiles are r full rounds of W CUs slots and a remainder.  A plane of a
-// full round takes one unit; with k workgroups on a CU it takes t(k), measured on the
-// 256 x 128 x 128 channel: 0.54 / 0.81 / 1 (FP32, 8.9 us), 0.62 / 1 (FP64, 11.8 us), between
-// them in proportion to the mean occupancy.  A tile costs its planes plus one.  Short chunks
-// are allowed down to one plane: below one workgroup per CU a launch is the serial march of
-// one tile (24 x 16 x 12 cells, FP64: 30.9 us at four planes, 15.5 us at one).  The shortest
-// estimate over ci in [1, 64] wins, ties to the shorter chunk (256 x 128 x 128, FP32: 8 planes,
-// three full rounds, 253 us; 26 planes, 267 us; 37 planes, 302 us).
+// FP32, 2 in FP64), so T tiles are r full rounds of W CUs slots and a remainder.  A full round
+// of ci planes takes ci + 1 units (11.3 us FP32, 12.1 us FP64); a remainder that puts at most k
+// workgroups on a CU takes t(k) of one: 0.55 / 0.78 / 1 (FP32), 0.6 / 1 (FP64).  Fitted to the
+// 256 x 128 x 128-cell, 128 x 96 x 96-cell and ensemble launches at ci of 2..64 (within 13%).
+// Short chunks are allowed down to one plane: below one workgroup per CU a launch is the
+// serial march of one tile (24 x 16 x 12 cells, FP64: 29.4 us at four planes, 15.0 us at one).
+// The shortest estimate over ci in [1, 64] wins, ties to the shorter chunk, whose tiles leave
+// and refill the slots more often (256 planes, FP32: 8 per tile, three full rounds, 307 us; 26
+// per tile, one round, 319 us; 24 per tile, one round and 24 tiles, 422 us).
 int box_ci_len(const wmx_plan* p) {
   const bool f32 = p->nd.prec == WMX_PREC_FP32_BULK;
-  const double t32[4] = {0.54, 0.54, 0.81, 1.0}, t64[3] = {0.62, 0.62, 1.0};
+  const double t32[4] = {0.0, 0.55, 0.78, 1.0}, t64[3] = {0.0, 0.6, 1.0};
   const double* t = f32 ? t32 : t64;
   const long long cus = std::max(1, p->cu_count), W = f32 ? 3 : 2;
   int best = 1;
@@ -402,10 +403,7 @@ int box_ci_len(const wmx_plan* p) {
     for (const BlockDev& B : p->hb)
       T += (long long)((B.n[0] + ci - 1) / ci) * ((B.n[1] + FLUX2_TILE_J - 1) / FLUX2_TILE_J) * ((B.n[2] + 15) / 16);
     const long long r = T / (W * cus), m = T - r * W * cus;
-    const double x = (double)m / (double)cus;
-    const int k = (int)x;
-    const double rest = m == 0 ? 0.0 : (k >= W ? 1.0 : t[k] + (x - k) * (t[k + 1] - t[k]));
-    const double cost = ((double)r + rest) * (ci + 1);
+    const double cost = ((double)r + t[(m + cus - 1) / cus]) * (ci + 1);
     if (cost < best_cost - 1e-9) { best_cost = cost; best = ci; }
   }
   return best;
@@ -460,7 +458,8 @@ NumDev make_numdev(const wmx_numerics_desc* nm) {
   nd.gas = GasC{nm->gamma, nm->R, nm->Pr, nm->Pr_t, nm->mu_ref, nm->T_ref, nm->S_suth,
                 nm->gamma * nm->R / (nm->gamma - 1.0)};
   nd.rc = RecC{1.0 / nm->R, 1.0 / (nm->gamma - 1.0), (float)(1.0 / nm->T_ref),
-               (float)(nm->mu_ref * (nm->T_ref + nm->S_suth)), (float)nm->S_suth};
+               (float)(nm->mu_ref * (nm->T_ref + nm->S_suth)), (float)nm->S_suth,
+               1.0 / nm->T_ref, nm->mu_ref * (nm->T_ref + nm->S_suth)};
   nd.wm = WallModelC{nm->kappa, nm->B, nm->wm_ekb, nm->wm_pr13, nm->wm_pr3, nm->wm_beta, nm->n_iter};
   nd.scheme = nm->scheme;
   nd.central = nm->central;
@@ -504,6 +503,72 @@ int run_fill(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, 
   return 0;
 }
 
+// The stage-2 state of a box plan: its gradient records' region, which the box kernels do not
+// use (64 or 120 B per cell for the 40 of a state).
+Ptrs stage_buffer(const wmx_plan* p) {
+  static_assert(sizeof(float) * 4 * G32_GROUPS >= 5 * sizeof(double) && NGR >= 5, "a state fits the gradient records");
+  Ptrs r;
+  std::memset(&r, 0, sizeof(r));
+  for (int b = 0; b < p->nb; ++b) r.p[b] = p->hb[b].G;
+  return r;
+}
+
+// ghost fill, wall faces and (dt_out != nullptr) the CFL dt of one RHS evaluation of a box plan,
+// whose flux launch reads the state itself; the arguments of run_cells
+int run_pre(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, hipStream_t s, double* dt_out,
+            bool zfuse, bool fill) {
+  const int nph = fill ? (int)p->phase_max.size() - (zfuse && p->fuse_last ? 1 : 0) : 0;
+  bool launched = false, dt_due = false;       // dt_due: the partials are taken, the mins are not
+  GradDt fin;
+  fin.ncases = p->n_cases;
+  fin.list = p->case_wg_ident ? nullptr : p->d_case_wg;
+  fin.off = p->d_case_off;
+  fin.part = p->d_part;
+  fin.out = dt_out;
+  for (int ph = 0; ph < std::max(nph, 1); ++ph) {
+    PreWork w;
+    if (ph < nph && p->phase_ext[ph].blk < 0) {
+      w.ops = p->d_ops + p->phase_off[ph];
+      w.nops = p->phase_off[ph + 1] - p->phase_off[ph];
+      w.per = (p->phase_max[ph] + 255) / 256;
+    }
+    if (!launched && !p->nd.net.w && !p->wall.empty()) {
+      w.wall = p->d_wall;
+      w.nwall = (int)p->wall.size();
+      w.wall_wgx = (p->wall_max + 255) / 256;
+    }
+    if (dt_due) w.fin = fin;
+    dt_due = !launched && dt_out;
+    if (dt_due) {
+      w.dt_pre = p->d_pre_int;
+      w.ndt = nwg_of(p->pre_int);
+      w.part = p->d_part;
+    }
+    WMX_CHECK(timed(p, K_FILL, s, [&] { return launch_pre(p->d_blks, p->nb, q, p->nd, w, s); }));
+    launched = true;
+    if (ph < nph)
+      for (int blk : p->phase_inflow[ph]) {
+        const BlockDev& B = p->hb[blk];
+        WMX_CHECK(timed(p, K_INFLOW, s, [&] {
+          return launch_inflow(p->d_blks, blk, B.N[1], B.N[2], B.ng, p->inflows[B.faces[0].inflow_id], q, p->nd.gas,
+                               time, d_dt, coef, s);
+        }));
+      }
+  }
+  if (dt_due)
+    WMX_CHECK(timed(p, K_DT, s, [&] {
+      return launch_case_final(0, p->n_cases, fin.list, fin.off, p->d_part, nullptr, dt_out, s);
+    }));
+  if (p->nd.net.w)
+    WMX_CHECK(timed(p, K_WALL, s, [&] { return launch_wall(p->d_blks, p->d_wall, (int)p->wall.size(), p->wall_max, q, p->nd, s); }));
+  if (p->nd.n_sponge > 0)
+    for (int b = 0; b < p->nb; ++b)
+      WMX_CHECK(timed(p, K_SPONGE, s, [&] {
+        return launch_sponge_mean(p->d_blks, b, (long long)p->hb[b].n[0] * p->hb[b].n[1], q, s);
+      }));
+  return 0;
+}
+
 // ghost fill + cell-level fields of one RHS evaluation
 // dt_out != nullptr: the primitive launch also takes the CFL partials of the (unchanged)
 // interior state and the per-case minimum goes to dt_out before the gradients
@@ -511,6 +576,7 @@ int run_fill(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, 
 int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, hipStream_t s,
               double* dt_out = nullptr, bool zfuse = false, bool fill = true) {
   zfuse = zfuse && p->fuse_last && fill;
+  if (box_active(p)) return run_pre(p, q, time, d_dt, coef, s, dt_out, zfuse, fill);
   if (fill && run_fill(p, q, time, d_dt, coef, s, zfuse)) return 1;
   SpongeHead sh;
   if (p->d_sponge_pre) {
@@ -545,9 +611,9 @@ int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef,
                                p->d_case_off_all, p->d_part, nullptr, dt_out, s);
     }));
   }
-  // fused FP32-bulk plans and box plans: the flux kernel evaluates the gradient records
-  // itself; the gradient launch keeps only its head work (per-case dt min, Newton wall faces)
-  const bool grads = !((f32 && p->fuse_grad) || box_active(p));
+  // fused FP32-bulk plans: the flux kernel evaluates the gradient records itself; the
+  // gradient launch keeps only its head work (per-case dt min, Newton wall faces)
+  const bool grads = !(f32 && p->fuse_grad);
   if (grads || gdt.out || wall_in_grad)
     WMX_CHECK(timed(p, K_GRAD, s, [&] {
       return launch_grad(p->d_blks, p->d_pre_box, p->nb, grads ? nwg_of(p->pre_box) : 0, p->nd,
@@ -565,9 +631,9 @@ int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef,
 
 hipError_t plan_flux(const wmx_plan* p, int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles,
                      int ci_len, const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
-                     hipStream_t s) {
+                     bool zfuse, hipStream_t s) {
   if (box_active(p))
-    return launch_box(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
+    return launch_box(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, zfuse && p->fuse_last, s);
   if (nd.prec == WMX_PREC_FP32_BULK && p->fuse_grad)
     return launch_flux3(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
   return launch_flux(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
@@ -960,6 +1026,20 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
     std::vector<unsigned> nz(p->nb + 1);
     WMX_CHECK(hipMemcpy(nz.data(), d_nz, sizeof(unsigned) * (p->nb + 1), hipMemcpyDeviceToHost));
     p->box = nz[p->nb] == 0;
+    // the box kernels read a fused side's k ghosts at their periodic images: a side that is no
+    // plain periodic face of its own block is filled by a launch
+    bool image = true;
+    for (int b = 0; b < p->nb; ++b)
+      for (int sd = 0; sd < 2; ++sd)
+        if ((p->hb[b].zfuse >> sd) & 1) {
+          const wmx_face_desc& f = p->hb[b].faces[4 + sd];
+          image = image && f.kind == WMX_FACE_INTERFACE && f.nb == b && f.src_axis == 2 && f.src_side == 1 - sd &&
+                  f.mapping[0] == 0 && f.mapping[1] == 1 && !f.flip[0] && !f.flip[1];
+        }
+    if (p->box && !image) {
+      p->fuse_last = false;
+      for (BlockDev& B : p->hb) B.zfuse = 0;
+    }
     if (retile(p)) return 1;
     for (int b = 0; b < p->nb; ++b)
       p->hb[b].sb_zero = p->hb[b].Sb ? (int)(~nz[b] & ((1u << NSB_PLANES) - 1u)) : 0;
@@ -1184,7 +1264,7 @@ int wmx_rhs_filled(wmx_plan* p, double* const* q, double* const* r, void* stream
   Ptrs pq = make_ptrs(p, q), pr = make_ptrs(p, r);
   if (run_cells(p, pq, 0.0, nullptr, 0.0, s, nullptr, false, false)) return 1;
   WMX_CHECK(plan_flux(p, 0, p->d_blks, p->d_tiles, (int)p->tiles.size(), p->ci_len, p->nd, pq, pq, pr,
-                        nullptr, 0.0, s));
+                        nullptr, 0.0, false, s));
   WMX_CHECK(launch_shell_finish(0, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), pq, pr,
                                 nullptr, 0.0, s));
   return 0;
@@ -1196,7 +1276,7 @@ int wmx_rhs(wmx_plan* p, double* const* q, double* const* r, double time, void* 
   Ptrs pq = make_ptrs(p, q), pr = make_ptrs(p, r);
   if (run_cells(p, pq, time, nullptr, 0.0, s)) return 1;
   WMX_CHECK(plan_flux(p, 0, p->d_blks, p->d_tiles, (int)p->tiles.size(), p->ci_len, p->nd, pq, pq, pr,
-                        nullptr, 0.0, s));
+                        nullptr, 0.0, false, s));
   WMX_CHECK(launch_shell_finish(0, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), pq, pr,
                                 nullptr, 0.0, s));
   return 0;
@@ -1259,6 +1339,12 @@ int upload_stage(wmx_plan* p) {
   if (p->fuse_grad) st.ngrad = 0;                 // the gradient list keeps only its dt head
   st.dt_list = p->case_wg_all_ident ? nullptr : p->d_case_wg_all;
   st.dt_off = p->d_case_off_all;
+  if (box_active(p)) {                            // CFL partials by the interior cells
+    st.pre_all = p->d_pre_int;
+    st.nprim = nwg_of(p->pre_int);
+    st.dt_list = p->case_wg_ident ? nullptr : p->d_case_wg;
+    st.dt_off = p->d_case_off;
+  }
   st.tiles = p->d_tiles;
   st.ntiles = (int)p->tiles.size();
   st.ci_len = p->ci_len;
@@ -1278,15 +1364,16 @@ int advance_persistent(wmx_plan* p, double* const* q0, double* const* qout, doub
   hipStream_t s = as_stream(stream);
   Ptrs P0 = make_ptrs(p, q0), PO = make_ptrs(p, qout);
   WMX_CHECK(launch_shell_save(p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), P0, s));
+  const Ptrs P2 = box_active(p) ? stage_buffer(p) : PO;
   const int sc = scheme_config(p->nd);
   const int nph = (int)p->phase_max.size();
   const int wx = !p->wall.empty() && p->wall_max > 0 ? (p->wall_max + 255) / 256 : 0;
   for (int mode = 1; mode <= 3; ++mode) {
     StageCall c;
     std::memset(&c, 0, sizeof(c));
-    c.qin = mode == 1 ? P0 : PO;
+    c.qin = mode == 1 ? P0 : (mode == 2 ? PO : P2);
     c.q0 = P0;
-    c.out = PO;
+    c.out = mode == 2 ? P2 : PO;
     c.nfill = nph - (p->fuse_last ? 1 : 0);
     c.zfuse = p->fuse_last ? 1 : 0;
     c.ndt = mode == 1 && dt_out ? p->n_cases : 0;
@@ -1315,12 +1402,14 @@ int advance_impl(wmx_plan* p, double* const* q0, double* const* qout, double dt,
   WMX_CHECK(timed(p, K_SHELL, s, [&] { return launch_shell_save(p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), P0, s); }));
   // stage times t, t + dt, t + dt/2 (solver.py:125-129)
   const double t1 = d_dt ? time : time + dt, t2 = d_dt ? time : time + 0.5 * dt;
+  // a box plan's flux launch reads its neighbours' states: stage 2 goes to a second buffer
+  const Ptrs P2 = box_active(p) ? stage_buffer(p) : PO;
   if (run_cells(p, P0, time, nullptr, 0.0, s, dt_out, true)) return 1;
-  WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 1, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, P0, P0, PO, d_dt, dt, s); }));
+  WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 1, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, P0, P0, PO, d_dt, dt, true, s); }));
   if (run_cells(p, PO, t1, d_dt, 1.0, s, nullptr, true)) return 1;
-  WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 2, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, PO, P0, PO, d_dt, dt, s); }));
-  if (run_cells(p, PO, t2, d_dt, 0.5, s, nullptr, true)) return 1;
-  WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 3, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, PO, P0, PO, d_dt, dt, s); }));
+  WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 2, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, PO, P0, P2, d_dt, dt, true, s); }));
+  if (run_cells(p, P2, t2, d_dt, 0.5, s, nullptr, true)) return 1;
+  WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 3, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, P2, P0, PO, d_dt, dt, true, s); }));
   WMX_CHECK(timed(p, K_SHELL, s, [&] {
     return launch_shell_finish(1, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), P0, PO, d_dt, dt, s);
   }));

@@ -84,6 +84,7 @@ struct WallNetDev {
 struct RecC {
   double iR, igm1;          // 1 / R, 1 / (gamma - 1)
   float iTref, muc, S;      // 1 / T_ref, mu_ref (T_ref + S_suth), S_suth
+  double iTref64, muc64;    // the first two in FP64
 };
 
 struct NumDev {
@@ -152,7 +153,7 @@ struct SpongeHead {
 // launch is skipped) instead of read from q
 hipError_t launch_prim(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
                        const NumDev& nd, double* d_part, int zfuse, SpongeHead sh, hipStream_t s);
-// per-case dt mins taken inside the gradient launch (out == nullptr: none)
+// per-case dt mins taken inside another launch (out == nullptr: none)
 struct GradDt {
   int ncases = 0;
   const int* list = nullptr;       // per-case workgroup list (nullptr: identity)
@@ -160,6 +161,21 @@ struct GradDt {
   const double* part = nullptr;    // CFL partials
   double* out = nullptr;           // dt per case
 };
+// What a stage of a box plan does before its flux launch, as one launch per sweep phase: the
+// phase's ghost fills and, where they are given, the Newton wall faces, the CFL partials (both
+// read interior states only) and the per-case dt mins of partials that an earlier launch took.
+struct PreWork {
+  const GhostOp* ops = nullptr;    // the phase's fill ops, `per` workgroups each
+  int nops = 0, per = 0;
+  const WallOp* wall = nullptr;    // wall ops, `wall_wgx` workgroups each
+  int nwall = 0, wall_wgx = 0;
+  const int* dt_pre = nullptr;     // CFL partials: workgroups per block (prefix)
+  int ndt = 0;
+  double* part = nullptr;
+  GradDt fin;                      // the dt mins (ncases 0: none)
+  int head = 0;                    // set by the launcher
+};
+hipError_t launch_pre(const BlockDev* d_blks, int nblk, Ptrs q, const NumDev& nd, PreWork w, hipStream_t s);
 // FP32-bulk plans: d_wall != nullptr also evaluates those Newton wall faces in the launch,
 // gdt.out != nullptr the per-case dt mins
 hipError_t launch_grad(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, const NumDev& nd,
@@ -174,10 +190,12 @@ hipError_t launch_flux(int mode, const BlockDev* d_blks, const int4* d_tiles, in
 hipError_t launch_flux3(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
                         const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
                         hipStream_t s);
-// the same for plans whose blocks are all boxes (box.h), both precisions; no gradient launch
+// the same for plans whose blocks are all boxes (box.h), both precisions, from the state itself:
+// no primitive or gradient launch.  Tiles read their neighbours' states, so out must not alias
+// qin.  zfuse: the k ghosts flagged in BlockDev::zfuse are read at their periodic images.
 hipError_t launch_box(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
                       const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
-                      hipStream_t s);
+                      int zfuse, hipStream_t s);
 // fills a block's BoxEnt tables; *d_bad becomes non-zero if the block is no box
 hipError_t launch_box_check(const BlockDev& hb, unsigned* d_bad, hipStream_t s);
 hipError_t launch_shell_save(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
@@ -239,7 +257,7 @@ struct StageStatic {
   const GhostOp* ops;          // sweep phases: ops[fill_off[ph] .. fill_off[ph + 1])
   const int* fill_off;
   const int* fill_max;         // cells of the phase's largest op
-  const int* pre_all;          // primitive workgroups per block (prefix)
+  const int* pre_all;          // primitive (box form: CFL partial) workgroups per block (prefix)
   int nblk, nprim;
   const int* pre_box;          // gradient workgroups per block (prefix)
   int ngrad;
@@ -332,15 +350,24 @@ __device__ __forceinline__ void st4(float* rec, float4 v) {
   *(__attribute__((address_space(1))) wmx_f4*)__builtin_assume_aligned(rec, 16) = w;
 }
 
+// 1 / x within an ulp: the hardware reciprocal and two Newton steps (no scaling: x is a density
+// or a sum of its size, far from the ends of the range; 0, infinities and NaN give NaN)
+__device__ __forceinline__ double rcp64(double x) {
+#pragma clang fp contract(off)
+  double y = __builtin_amdgcn_rcp(x);
+  y = __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+  return __builtin_fma(__builtin_fma(-x, y, 1.0), y, y);
+}
+
 // FP32-bulk primitive record of a cell from its conserved state q, with the block gauge
 // (p' = p - p_ref, T' = T - T_gauge, e' = e_int - e_ref): cons_to_prim (reference
 // gas.py:28-33) in FP64 with one reciprocal of rho, and Sutherland's mu (gas.py:24-26)
-// from the float temperature (the record holds it as a float), stored as the two 16-byte
-// groups (u, v, w, T') and (rho, p', mu, e').  The arithmetic is not contracted (callers are
-// built with contraction off or, where fast, honour the pragma), so every caller stores the
+// from the float temperature (the record holds it as a float), as the two groups
+// a = (u, v, w, T') and b = (rho, p', mu, e').  The arithmetic is not contracted (callers are
+// built with contraction off or, where fast, honour the pragma), so every caller forms the
 // same bits.
-__device__ __forceinline__ void rec32_store(float* Pb, size_t cells, size_t c, const NumDev& nd, const double* q,
-                                            double p_ref, double T_gauge, double e_ref) {
+__device__ __forceinline__ void rec_of(const NumDev& nd, const double* q, double p_ref, double T_gauge,
+                                       double e_ref, float* a, float* b) {
 #pragma clang fp contract(off)
   const RecC& rc = nd.rc;
   const double r = q[0];
@@ -352,9 +379,35 @@ __device__ __forceinline__ void rec32_store(float* Pb, size_t cells, size_t c, c
   const double T = pr * rc.iR;
   const float Tf = (float)T;
   const float t = Tf * rc.iTref;
-  const float mu = (rc.muc * (t * __builtin_amdgcn_sqrtf(t))) * __builtin_amdgcn_rcpf(Tf + rc.S);
-  st4(Pb + 4 * c, make_float4((float)u, (float)v, (float)w, (float)(T - T_gauge)));
-  st4(Pb + 4 * (cells + c), make_float4((float)r, (float)(p - p_ref), mu, (float)(pr * rc.igm1 - e_ref)));
+  b[2] = (rc.muc * (t * __builtin_amdgcn_sqrtf(t))) * __builtin_amdgcn_rcpf(Tf + rc.S);
+  a[0] = (float)u; a[1] = (float)v; a[2] = (float)w; a[3] = (float)(T - T_gauge);
+  b[0] = (float)r; b[1] = (float)(p - p_ref); b[3] = (float)(pr * rc.igm1 - e_ref);
+}
+
+__device__ __forceinline__ void rec32_store(float* Pb, size_t cells, size_t c, const NumDev& nd, const double* q,
+                                            double p_ref, double T_gauge, double e_ref) {
+  float a[4], b[4];
+  rec_of(nd, q, p_ref, T_gauge, e_ref, a, b);
+  st4(Pb + 4 * c, make_float4(a[0], a[1], a[2], a[3]));
+  st4(Pb + 4 * (cells + c), make_float4(b[0], b[1], b[2], b[3]));
+}
+
+// The same record in FP64, without gauge (box kernels): one reciprocal of rho, within an ulp
+// or two of k_prim's divisions.
+__device__ __forceinline__ void rec_of(const NumDev& nd, const double* q, double, double, double, double* a,
+                                       double* b) {
+#pragma clang fp contract(off)
+  const RecC& rc = nd.rc;
+  const double r = q[0];
+  const double ir = rcp64(r);
+  a[0] = q[1] * ir; a[1] = q[2] * ir; a[2] = q[3] * ir;
+  const double k = (a[0] * a[0] + a[1] * a[1]) + a[2] * a[2];
+  const double p = (nd.gas.gamma - 1.0) * (q[4] - (0.5 * r) * k);
+  const double pr = p * ir;
+  const double T = pr * rc.iR, t = T * rc.iTref64;
+  a[3] = T;
+  b[0] = r; b[1] = p; b[3] = pr * rc.igm1;
+  b[2] = (rc.muc64 * (t * sqrt(t))) * rcp64(T + nd.gas.S_suth);
 }
 
 // SmoothRampSponge weight at a cell centre x (smooth_ramp.py:212-221); pr = (x_start_l,

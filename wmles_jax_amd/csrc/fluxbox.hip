@@ -13,16 +13,16 @@ namespace wmx {
 template <class R, int MODE, int SC>
 __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : 2) void k_box(
     const BlockDev* __restrict__ blks, const int4* __restrict__ tiles, int ci_len, NumDev nd, Ptrs qin, Ptrs q0,
-    Ptrs out, const double* __restrict__ d_dt, double dt_host) {
-  box_tile<R, MODE, SC>(blks, tiles, ci_len, nd, qin, q0, out, d_dt, dt_host, (int)blockIdx.x);
+    Ptrs out, const double* __restrict__ d_dt, double dt_host, int zfuse) {
+  box_tile<R, MODE, SC>(blks, tiles, ci_len, nd, qin, q0, out, d_dt, dt_host, zfuse, (int)blockIdx.x);
 }
 
 hipError_t launch_box(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
                       const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
-                      hipStream_t s) {
+                      int zfuse, hipStream_t s) {
   if (ntiles <= 0) return hipSuccess;
   dim3 grid(ntiles), block(NT);
-#define WMX_BX(R, M, C) hipLaunchKernelGGL((k_box<R, M, C>), grid, block, 0, s, d_blks, d_tiles, ci_len, nd, qin, q0, out, d_dt, dt)
+#define WMX_BX(R, M, C) hipLaunchKernelGGL((k_box<R, M, C>), grid, block, 0, s, d_blks, d_tiles, ci_len, nd, qin, q0, out, d_dt, dt, zfuse)
 #define WMX_BXM(R, C)               \
   switch (mode) {                   \
     case 0: WMX_BX(R, 0, C); break; \

@@ -141,6 +141,75 @@ __device__ __forceinline__ double cell_dt(const BlockDev& B, const NumDev& nd, u
   return cell_dt_eval(nd, w, m, vol);
 }
 
+// CFL partial of workgroup wgx of nwg: INT_CELLS interior cells per thread, blockDim.x apart
+// (solver.py:139-150).  XCD-contiguous spans.
+__device__ __forceinline__ void dt_partial_block(const BlockDev* __restrict__ blks, const int* __restrict__ wg_prefix,
+                                                 int nblk, const Ptrs& q, const NumDev& nd,
+                                                 double* __restrict__ part, int wgx, int nwg) {
+  const int wg = xcd_span(wgx, nwg);
+  const int b = find_block_r(wg_prefix, nblk, wg);
+  const BlockDev& B = blks[b];
+  const unsigned base = (unsigned)(wg - wg_prefix[b]) * (INT_CELLS * blockDim.x) + threadIdx.x;
+  const unsigned nint = (unsigned)B.n[0] * B.n[1] * B.n[2];
+  double dtc = __builtin_huge_val();
+  for (int u = 0; u < INT_CELLS; ++u) {
+    const unsigned l = base + (unsigned)u * blockDim.x;
+    if (l < nint) {
+      int I, J, K;
+      const unsigned c = interior_cell(B, l, &I, &J, &K);
+      const unsigned cells = (unsigned)B.cells;
+      const double* qb = q.p[b];
+      double qv[5];
+#pragma unroll
+      for (int v = 0; v < 5; ++v) qv[v] = ldu(qb + v * cells, c);
+      const Prim w = cons_to_prim(nd.gas, qv[0], qv[1], qv[2], qv[3], qv[4]);
+      dtc = nmin(dtc, cell_dt(B, nd, c, I, J, K, w));
+    }
+  }
+  const double r = block_reduce<true>(dtc);
+  if (threadIdx.x == 0) part[wg] = r;
+}
+
+// Workgroup wgx of nwg of the work before a box plan's stage (PreWork): the dt mins, the wall
+// faces and the ghost fills first (w.head workgroups, a multiple of 8), then the CFL partials.
+__device__ __forceinline__ void pre_block(const BlockDev* __restrict__ blks, int nblk, const Ptrs& q,
+                                          const NumDev& nd, const PreWork& w, int wgx, int nwg) {
+  if (wgx >= w.head) {
+    dt_partial_block(blks, w.dt_pre, nblk, q, nd, w.part, wgx - w.head, nwg - w.head);
+    return;
+  }
+  if (wgx < w.fin.ncases) {
+    const int lo = w.fin.off[wgx], hi = w.fin.off[wgx + 1];
+    double a = __builtin_huge_val();
+    for (int t0 = lo + (int)threadIdx.x; t0 < hi; t0 += 16 * (int)blockDim.x) {
+      double va[16];                             // clamped: a repeated element leaves a min unchanged
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int t = min(t0 + u * (int)blockDim.x, hi - 1);
+        va[u] = w.fin.part[w.fin.list ? w.fin.list[t] : t];
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a = nmin(a, va[u]);
+    }
+    a = block_reduce<true>(a);
+    if (threadIdx.x == 0) w.fin.out[wgx] = a;
+    return;
+  }
+  int h = wgx - w.fin.ncases;
+  if (h < w.wall_wgx * w.nwall) {
+    const int i = h / w.wall_wgx;
+    const WallOp op = w.wall[i];
+    const int idx = (h - i * w.wall_wgx) * (int)blockDim.x + (int)threadIdx.x;
+    if (idx < op.count) wall_face<false>(blks, op, idx, q, nd, nullptr, nullptr);
+    return;
+  }
+  h -= w.wall_wgx * w.nwall;
+  if (h < w.nops * w.per) {
+    const int i = h / w.per;
+    fill_cell(blks, w.ops[i], q, nd.gas, (h - i * w.per) * (int)blockDim.x + (int)threadIdx.x);
+  }
+}
+
 // Spanwise mean of sponge row `row` for rows of 9..129 cells (numpy's pairwise order for
 // the elements 1..nk-1 by eight lanes u of the row, combined by shuffles in that order);
 // every lane of the 8-lane group calls it.  smooth_ramp.py:214-216.

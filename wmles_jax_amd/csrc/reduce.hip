@@ -13,29 +13,13 @@ namespace wmx {
 __global__ __launch_bounds__(256) void k_dt_partial(const BlockDev* __restrict__ blks,
                                                     const int* __restrict__ wg_prefix, int nblk,
                                                     Ptrs q, NumDev nd, double* __restrict__ part) {
-  const int wg = xcd_span(blockIdx.x, gridDim.x);
-  const int b = find_block_r(wg_prefix, nblk, wg);
-  const BlockDev& B = blks[b];
-  // INT_CELLS interior cells per thread, blockDim.x apart
-  const unsigned base = (unsigned)(wg - wg_prefix[b]) * (INT_CELLS * blockDim.x) + threadIdx.x;
-  const unsigned nint = (unsigned)B.n[0] * B.n[1] * B.n[2];
-  double dtc = __builtin_huge_val();
-  for (int u = 0; u < INT_CELLS; ++u) {
-    const unsigned l = base + (unsigned)u * blockDim.x;
-    if (l < nint) {
-      int I, J, K;
-      const unsigned c = interior_cell(B, l, &I, &J, &K);
-      const unsigned cells = (unsigned)B.cells;
-      const double* qb = q.p[b];
-      double qv[5];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) qv[v] = ldu(qb + v * cells, c);
-      const Prim w = cons_to_prim(nd.gas, qv[0], qv[1], qv[2], qv[3], qv[4]);
-      dtc = nmin(dtc, cell_dt(B, nd, c, I, J, K, w));
-    }
-  }
-  const double r = block_reduce<true>(dtc);
-  if (threadIdx.x == 0) part[wg] = r;
+  dt_partial_block(blks, wg_prefix, nblk, q, nd, part, (int)blockIdx.x, (int)gridDim.x);
+}
+
+// The work before a box plan's stage (pre_block)
+__global__ __launch_bounds__(256) void k_pre(const BlockDev* __restrict__ blks, int nblk, Ptrs q, NumDev nd,
+                                             PreWork w) {
+  pre_block(blks, nblk, q, nd, w, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // FP64 record (r, u, v, w, p, T, mu, e_int)
@@ -334,6 +318,14 @@ hipError_t launch_dt_partial(const BlockDev* d_blks, const int* d_pre, int nblk,
                              const NumDev& nd, double* d_part, hipStream_t s) {
   if (nwg <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_dt_partial, dim3(nwg), dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part);
+  return hipGetLastError();
+}
+
+hipError_t launch_pre(const BlockDev* d_blks, int nblk, Ptrs q, const NumDev& nd, PreWork w, hipStream_t s) {
+  if (!w.fin.out) w.fin.ncases = 0;
+  w.head = (w.fin.ncases + w.wall_wgx * w.nwall + w.nops * w.per + 7) / 8 * 8;   // (keeps the XCD spans)
+  if (w.head + w.ndt <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_pre, dim3(w.head + w.ndt), dim3(256), 0, s, d_blks, nblk, q, nd, w);
   return hipGetLastError();
 }
 

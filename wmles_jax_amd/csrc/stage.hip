@@ -21,6 +21,7 @@ namespace wmx {
 __device__ void st_fill(const StageStatic& s, int opi, int idx);
 template <bool DT>
 __device__ void st_prim(const StageStatic& s, double* __restrict__ part, int zfuse, int wgx);
+__device__ void st_pre(const StageStatic& s, double* __restrict__ part, int wgx);
 __device__ void st_grad(const StageStatic& s, int head, int ndt, const double* __restrict__ part,
                         double* __restrict__ dt_out, int wgx);
 template <int MODE, int SC>
@@ -28,11 +29,11 @@ __device__ void st_flux(const StageStatic& s, const double* __restrict__ d_dt, d
 template <int MODE, int SC>
 __device__ void st_flux3(const StageStatic& s, const double* __restrict__ d_dt, double dt_host, int tile);
 template <int MODE, int SC>
-__device__ void st_box(const StageStatic& s, const double* __restrict__ d_dt, double dt_host, int tile);
+__device__ void st_box(const StageStatic& s, const double* __restrict__ d_dt, double dt_host, int zfuse, int tile);
 
 // FORM 1: the fused kernel form (flux3 tiles with the gradient records in the march, wall
-// faces in the primitive head, the gradient list only its dt head); 2: the same with the box
-// tiles; 0: flux2 tiles after the gradient list
+// faces in the primitive head, the gradient list only its dt head); 2: box plans (box tiles,
+// which read the state: the primitive list holds the wall faces and the CFL partials); 0: flux2 tiles after the gradient list
 template <int MODE, int SC, int FORM>
 __global__ __launch_bounds__(256, 2) void k_stage(const StageStatic* __restrict__ st, StageCall c) {
   cg::grid_group grid = cg::this_grid();
@@ -53,9 +54,10 @@ __global__ __launch_bounds__(256, 2) void k_stage(const StageStatic* __restrict_
     for (int w = (int)blockIdx.x; w < nwork; w += G) st_fill(s, o + w / per, (w % per) * 256 + (int)threadIdx.x);
     grid.sync();
   }
-  const int npr = s.prim_head + s.nprim;
+  const int npr = s.prim_head + (FORM == 2 && !c.part ? 0 : s.nprim);
   for (int w = (int)blockIdx.x; w < npr; w += G) {
-    if (c.part) st_prim<true>(s, c.part, c.zfuse, w);          // (uniform: a kernel argument)
+    if (FORM == 2) st_pre(s, c.part, w);
+    else if (c.part) st_prim<true>(s, c.part, c.zfuse, w);          // (uniform: a kernel argument)
     else st_prim<false>(s, c.part, c.zfuse, w);
     __syncthreads();                                            // LDS reuse by the next item
   }
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(256, 2) void k_stage(const StageStatic* __restrict_
   }
   grid.sync();
   for (int w = (int)blockIdx.x; w < s.ntiles; w += G) {
-    if (FORM == 2) st_box<MODE, SC>(s, c.d_dt, c.dt_host, w);
+    if (FORM == 2) st_box<MODE, SC>(s, c.d_dt, c.dt_host, c.zfuse, w);
     else if (FORM == 1) st_flux3<MODE, SC>(s, c.d_dt, c.dt_host, w);
     else st_flux<MODE, SC>(s, c.d_dt, c.dt_host, w);
     __syncthreads();

@@ -19,6 +19,18 @@ __device__ void st_prim(const StageStatic& s, double* __restrict__ part, int zfu
   sh.head = s.prim_head;
   prim32_block<DT>(s.blks, s.pre_all, s.nblk, s.pbuf[0], s.nd, part, zfuse, sh, wgx, s.prim_head + s.nprim);
 }
+
+// Box form: the wall faces and (part != nullptr) the CFL partials of the stage.
+__device__ void st_pre(const StageStatic& s, double* __restrict__ part, int wgx) {
+  PreWork w;
+  w.wall = s.wall_ops;
+  w.wall_wgx = s.prim_wall_wgx;
+  w.nwall = s.prim_wall_wgx > 0 ? s.nwall_ops : 0;
+  w.head = s.prim_head;
+  w.dt_pre = s.pre_all;
+  w.part = part;
+  pre_block(s.blks, s.nblk, s.pbuf[0], s.nd, w, wgx, s.prim_head + s.nprim);
+}
 template __device__ void st_prim<true>(const StageStatic&, double*, int, int);
 template __device__ void st_prim<false>(const StageStatic&, double*, int, int);
 
