@@ -460,11 +460,15 @@ struct WallModelC {      // reference wall_model.py:15-17 + host-evaluated const
 // Spalding u_tau by safeguarded fixed-count Newton, reference wall_model.py:19-40.  The
 // iteration map depends on up alone, so once an update returns its input exactly the
 // remaining iterations would repeat it: stopping there gives the fixed-count result bit
-// for bit.
+// for bit.  One face in eight ends in a pair of neighbouring values instead, each the update
+// of the other (so nearly every wave held one and ran all 30 iterations; both cases end
+// within 12): an update that returns the value before its input stops too, at the member of
+// the pair that the iteration count would stop at.  The launch of 768 wall faces, a serial
+// chain: 13.9 us to 6.6 us.
 WMX_HD double spalding_utau(const WallModelC& m, double h, double U, double rho_w, double mu_w) {
   double k = m.kappa, ekb = m.ekb;
   double Reh = ((h * U) * rho_w) / mu_w;
-  double up = fmin(fmax(sqrt(Reh), 1.0), 25.0);
+  double up = fmin(fmax(sqrt(Reh), 1.0), 25.0), before = -1.0;
   for (int it = 0; it < m.n_iter; ++it) {
     double ku = k * up;
     double ex = exp(ku);
@@ -475,6 +479,11 @@ WMX_HD double spalding_utau(const WallModelC& m, double h, double U, double rho_
     double nw = up - F / dF;
     const double upn = fmin(fmax(nw, 0.5 * up), 100.0);
     if (upn == up) break;
+    if (upn == before) {
+      if (((m.n_iter - 1 - it) & 1) == 0) up = upn;
+      break;
+    }
+    before = up;
     up = upn;
   }
   return U / up;
