@@ -472,11 +472,10 @@ class Solver:
         """{(block, face): (tau_w, q_w)} for all wall-modelled faces (solver.py:163-179)."""
         Q = self._as_state(Q)
         tot = sum(r[3] * r[4] for r in self._wall_faces)
-        tau = torch.empty(max(tot, 1), dtype=torch.float64, device=self._dev)
-        qw = torch.empty_like(tau)
-        _lib.check(_lib.lib.wmx_wall_stats(self._plan, _lib.ptr_array(Q), C.c_void_p(tau.data_ptr()),
-                                           C.c_void_p(qw.data_ptr()), _lib.stream_ptr()))
-        tau, qw = tau.cpu().numpy(), qw.cpu().numpy()
+        both = torch.empty((2, max(tot, 1)), dtype=torch.float64, device=self._dev)
+        _lib.check(_lib.lib.wmx_wall_stats(self._plan, _lib.ptr_array(Q), C.c_void_p(both[0].data_ptr()),
+                                           C.c_void_p(both[1].data_ptr()), _lib.stream_ptr()))
+        tau, qw = both.cpu().numpy()                 # (one copy to the host for both)
         out, off = {}, 0
         for b, a, s, n1, n2 in self._wall_faces:
             cnt = n1 * n2

@@ -24,7 +24,8 @@ class PlaneStats:
     def __init__(self, mesh, solver):
         self.mesh, self.solver = mesh, solver
         blk, geom = mesh.blocks[0], solver.geoms[0]
-        self.y = np.asarray(torch.as_tensor(blk.interior(geom.xc[1])).cpu())[0, :, 0]
+        # (the line alone goes to the host: the whole field took 1.1 ms at 192 x 96 x 96 cells)
+        self.y = np.asarray(torch.as_tensor(blk.interior(geom.xc[1])[0, :, 0]).cpu())
         self.n = 0
         self.tau_w_sum = 0.0
         self._acc = torch.zeros((len(KEYS), blk.n[1]), dtype=torch.float64, device=solver._dev)
