@@ -811,7 +811,7 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
         int t1, t2;
         tangents(f / 2, &t1, &t2);
         int cnt = p->hb[b].n[t1] * p->hb[b].n[t2];
-        p->wall.push_back(WallOp{b, f / 2, f % 2, cnt});
+        p->wall.push_back(WallOp{b, f / 2, f % 2, cnt, p->wall.empty() ? 0 : p->wall.back().off + p->wall.back().count});
         p->wall_max = std::max(p->wall_max, cnt);
       }
   {
@@ -1601,16 +1601,7 @@ int wmx_wall_stats(wmx_plan* p, double* const* q, double* d_tau, double* d_qw, v
   if (check_plan(p)) return 1;
   hipStream_t s = as_stream(stream);
   Ptrs pq = make_ptrs(p, q);
-  WMX_CHECK(launch_wall(p->d_blks, p->d_wall, (int)p->wall.size(), p->wall_max, pq, p->nd, s));
-  size_t off = 0;
-  for (const WallOp& w : p->wall) {
-    const double* W = p->hb[w.blk].wall[2 * w.axis + w.side];
-    WMX_CHECK(hipMemcpyAsync(d_tau + off, W + 5 * (size_t)w.count, sizeof(double) * w.count,
-                             hipMemcpyDeviceToDevice, s));
-    WMX_CHECK(hipMemcpyAsync(d_qw + off, W + 6 * (size_t)w.count, sizeof(double) * w.count,
-                             hipMemcpyDeviceToDevice, s));
-    off += w.count;
-  }
+  WMX_CHECK(launch_wall(p->d_blks, p->d_wall, (int)p->wall.size(), p->wall_max, pq, p->nd, s, d_tau, d_qw));
   return 0;
 }
 

@@ -114,6 +114,7 @@ struct GhostOp {
 
 struct WallOp {
   int blk, axis, side, count;
+  long long off;            // faces of the operations before it
 };
 
 struct InflowDev {
@@ -182,7 +183,7 @@ hipError_t launch_grad(const BlockDev* d_blks, const int* d_pre, int nblk, int n
                        const WallOp* d_wall, int nwall_ops, int wall_max, Ptrs q, const GradDt& gdt,
                        hipStream_t s);
 hipError_t launch_wall(const BlockDev* d_blks, const WallOp* d_ops, int nops, int maxcount, Ptrs q,
-                       const NumDev& nd, hipStream_t s);
+                       const NumDev& nd, hipStream_t s, double* tau = nullptr, double* qw = nullptr);
 hipError_t launch_flux(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
                        const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt,
                        double dt, hipStream_t s);

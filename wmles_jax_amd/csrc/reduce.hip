@@ -181,24 +181,28 @@ __global__ __launch_bounds__(256) void k_mf_apply(const BlockDev* __restrict__ b
 
 // Plane statistics of one block (wmles/channel5200.py:139-157): per interior j plane the
 // (i, k) means of rho, u, v, w, uu, vv, ww, uv, uw, vw, T, p.  Partial sums per
-// (plane, chunk) workgroup, then one thread per plane sums its chunks in order and adds
-// the means to the accumulator acc[NSTAT][n1].
+// (plane, chunk) workgroup, then one thread per plane and quantity sums its chunks in order
+// and adds the mean to the accumulator acc[NSTAT][n1].  Bound by the state's 40 B per cell
+// (15 us at 192 x 96 x 96); the index division is 32-bit and the twelve block sums share one
+// barrier (25 -> 20.7 us), a thread has one quantity (one thread per plane was a serial chain
+// of 192 loads: 30 -> 4.1 us).
 __global__ __launch_bounds__(256) void k_plane_partial(const BlockDev* __restrict__ blks, int blk,
                                                        Ptrs q, GasC gas, int chunk,
                                                        double* __restrict__ part) {
+  __shared__ double red[4][NSTAT];
   const BlockDev& B = blks[blk];
   const int j = blockIdx.y, ch = blockIdx.x, nch = gridDim.x;
-  const int n0 = B.n[0], n2 = B.n[2], ng = B.ng;
+  const unsigned n2 = (unsigned)B.n[2], ng = (unsigned)B.ng;
   const long long cells = B.cells;
-  const long long tot = (long long)n0 * n2;
-  const long long l0 = (long long)ch * chunk, l1 = l0 + chunk < tot ? l0 + chunk : tot;
+  const unsigned tot = (unsigned)B.n[0] * n2;
+  const unsigned l0 = (unsigned)ch * (unsigned)chunk, l1 = min(l0 + (unsigned)chunk, tot);
   const double* qb = q.p[blk];
   double a[NSTAT];
 #pragma unroll
   for (int v = 0; v < NSTAT; ++v) a[v] = 0.0;
-  for (long long l = l0 + threadIdx.x; l < l1; l += blockDim.x) {
-    const int i = (int)(l / n2), k = (int)(l % n2);
-    const long long c = cidx(B.N, ng + i, ng + j, ng + k);
+  for (unsigned l = l0 + threadIdx.x; l < l1; l += blockDim.x) {
+    const unsigned i = l / n2, k = l - i * n2;
+    const long long c = cidx(B.N, (int)(ng + i), (int)ng + j, (int)(ng + k));
     const Prim w = cons_to_prim(gas, qb[c], qb[cells + c], qb[2 * cells + c], qb[3 * cells + c],
                                 qb[4 * cells + c]);
     a[0] += w.r;
@@ -214,21 +218,29 @@ __global__ __launch_bounds__(256) void k_plane_partial(const BlockDev* __restric
     a[10] += w.T;
     a[11] += w.p;
   }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
   for (int v = 0; v < NSTAT; ++v) {
-    const double r = block_reduce<false>(a[v]);
-    if (threadIdx.x == 0) part[((long long)j * nch + ch) * NSTAT + v] = r;
+    for (int o = 32; o > 0; o >>= 1) a[v] = a[v] + __shfl_xor(a[v], o, 64);
+    if (lane == 0) red[wave][v] = a[v];
   }
+  __syncthreads();
+  const int v = threadIdx.x;
+  if (v < NSTAT) part[((long long)j * nch + ch) * NSTAT + v] = ((red[0][v] + red[1][v]) + red[2][v]) + red[3][v];
 }
 
-__global__ void k_plane_final(int n1, int nch, double inv_count, const double* __restrict__ part,
-                              double* __restrict__ acc) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n1) return;
-  for (int v = 0; v < NSTAT; ++v) {
-    double s = 0.0;
-    for (int ch = 0; ch < nch; ++ch) s += part[((long long)j * nch + ch) * NSTAT + v];
-    acc[(long long)v * n1 + j] += s * inv_count;
-  }
+__global__ __launch_bounds__(64) void k_plane_final(int n1, double inv_count, const double* __restrict__ part,
+                                                    double* __restrict__ acc) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n1 * NSTAT) return;
+  const int j = t / NSTAT, v = t - j * NSTAT;
+  double p[PLANE_CHUNKS];
+#pragma unroll
+  for (int ch = 0; ch < PLANE_CHUNKS; ++ch) p[ch] = part[((long long)j * PLANE_CHUNKS + ch) * NSTAT + v];
+  double s = 0.0;
+#pragma unroll
+  for (int ch = 0; ch < PLANE_CHUNKS; ++ch) s += p[ch];
+  acc[(long long)v * n1 + j] += s * inv_count;
 }
 
 // Rows that need the sponge mean: some cell of the (i, j) row has a weight > 0 under
@@ -355,7 +367,7 @@ hipError_t launch_plane_stats(const BlockDev* d_blks, const BlockDev& hb, int bl
                      chunk, d_part);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_plane_final, dim3((hb.n[1] + 63) / 64), dim3(64), 0, s, hb.n[1], PLANE_CHUNKS,
+  hipLaunchKernelGGL(k_plane_final, dim3((hb.n[1] * NSTAT + 63) / 64), dim3(64), 0, s, hb.n[1],
                      1.0 / (double)tot, d_part, d_acc);
   return hipGetLastError();
 }

@@ -124,9 +124,12 @@ template __global__ void k_grad32<WMX_SGS_VREMAN>(const BlockDev*, const int*, i
 // ------------------------------------------------------------------------------ wall
 // NET: the learned model (wave-cooperative network + Newton polish) replaces the
 // Newton solve; whole waves past the face count leave, the others clamp their index.
+// tau, qw: where wall_stats wants the stresses and heat fluxes (null in a stage); each thread
+// reads back what it wrote.
 template <bool NET>
 __global__ __launch_bounds__(256) void k_wall(const BlockDev* __restrict__ blks,
-                                              const WallOp* __restrict__ ops, Ptrs q, NumDev nd) {
+                                              const WallOp* __restrict__ ops, Ptrs q, NumDev nd,
+                                              double* __restrict__ tau, double* __restrict__ qw) {
   __shared__ unsigned short sW[NET ? MLP_LDS_BF16 : 1];
   __shared__ float sF[NET ? MLP_NF32 : 1];
   const WallOp op = ops[blockIdx.y];
@@ -139,6 +142,11 @@ __global__ __launch_bounds__(256) void k_wall(const BlockDev* __restrict__ blks,
     return;
   }
   wall_face<NET>(blks, op, idx0, q, nd, sW, sF);
+  if (tau && idx0 < op.count) {                  // the caller's copy, all faces one after the other
+    const double* W = blks[op.blk].wall[2 * op.axis + op.side];
+    tau[op.off + idx0] = W[5 * (size_t)op.count + idx0];
+    qw[op.off + idx0] = W[6 * (size_t)op.count + idx0];
+  }
 }
 
 // ------------------------------------------------------------------- shells / sponge
@@ -286,13 +294,13 @@ hipError_t launch_grad(const BlockDev* d_blks, const int* d_pre, int nblk, int n
 }
 
 hipError_t launch_wall(const BlockDev* d_blks, const WallOp* d_ops, int nops, int maxcount, Ptrs q,
-                       const NumDev& nd, hipStream_t s) {
+                       const NumDev& nd, hipStream_t s, double* tau, double* qw) {
   if (nops <= 0 || maxcount <= 0) return hipSuccess;
   dim3 grid((maxcount + 255) / 256, nops);
   if (nd.net.w)
-    hipLaunchKernelGGL(k_wall<true>, grid, dim3(256), 0, s, d_blks, d_ops, q, nd);
+    hipLaunchKernelGGL(k_wall<true>, grid, dim3(256), 0, s, d_blks, d_ops, q, nd, tau, qw);
   else
-    hipLaunchKernelGGL(k_wall<false>, grid, dim3(256), 0, s, d_blks, d_ops, q, nd);
+    hipLaunchKernelGGL(k_wall<false>, grid, dim3(256), 0, s, d_blks, d_ops, q, nd, tau, qw);
   return hipGetLastError();
 }
 
