@@ -118,3 +118,29 @@ def test_a_mesh_that_is_nearly_a_box_takes_the_general_kernels():
     blk = mesh.blocks[0]
     R = s.rhs(Q)[0].cpu().numpy()
     assert golden_io.rel_err(blk.interior(R), blk.interior(ref.rhs(Q)[0])) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [(3, 3, 3), (8, 16, 8), (11, 31, 13)])
+def test_box_cfl_step_is_the_oracles(n):
+    """The filtered CFL minimum of a box block (less than, exactly and several workgroups of
+    1024 cells): fields with one fastest cell at either end, equal cells, and states whose
+    minimum is no number, zero or negative."""
+    spec, arrays = box_spec(n, (None, WM, None), HYB, "vreman")
+    mesh, s = cases.build(wmx, spec, arrays)
+    _, ref = cases.build(oracle, spec, arrays)
+    blk = mesh.blocks[0]
+    noise = state(mesh, s)[0]
+    prim = np.array([1.2, 0.0, 0.0, 0.0, 1e5])
+    flat = np.asarray(s.init_state(lambda xc: prim[:, None, None, None] + 0.0 * xc[:1])[0].cpu())
+    tests = {"noise": noise, "equal cells": flat}
+    for name, at, v, val in (("first", 0, 4, 2e6), ("last", -1, 4, 2e6), ("nan", -1, 2, np.nan), ("inf", 0, 4, np.inf),
+                             ("negative density", 0, 0, -1.0), ("negative pressure", -1, 4, -1.0),
+                             ("huge", 0, 1, 1e200), ("zero density", -1, 0, 0.0)):
+        q = noise.copy()
+        blk.interior(q)[(v,) + (at,) * 3] = val
+        tests[name] = q
+    for name, q in tests.items():
+        with np.errstate(all="ignore"):
+            want = float(np.asarray(ref.max_dt([q])))
+        got = float(s.max_dt([q]))
+        assert got == want or (np.isnan(got) and np.isnan(want)) or abs(got - want) <= 1e-13 * abs(want), (name, got, want)

@@ -1430,7 +1430,7 @@ int wmx_max_dt(wmx_plan* p, double* const* q, double* d_dt, void* stream) {
   Ptrs pq = make_ptrs(p, q);
   WMX_CHECK(timed(p, K_DT, s, [&] {
     hipError_t e = launch_dt_partial(p->d_blks, p->d_pre_int, p->nb, nwg_of(p->pre_int), pq, p->nd,
-                                     p->d_part, s);
+                                     p->d_part, p->box, s);
     if (e == hipSuccess)
       e = launch_case_final(0, p->n_cases, p->case_wg_ident ? nullptr : p->d_case_wg, p->d_case_off,
                             p->d_part, nullptr, d_dt, s);
@@ -1485,7 +1485,7 @@ int wmx_max_dt_noalloc(wmx_plan* p, double* const* q, double* d_dt, void* stream
   hipStream_t s = as_stream(stream);
   Ptrs pq = make_ptrs(p, q);
   // the same two launches as wmx_max_dt, with the partials in the static scratch
-  WMX_CHECK(launch_dt_partial(p->d_blks, p->d_pre_int, p->nb, npart, pq, p->nd, part, s));
+  WMX_CHECK(launch_dt_partial(p->d_blks, p->d_pre_int, p->nb, npart, pq, p->nd, part, p->box, s));
   WMX_CHECK(launch_case_final(0, p->n_cases, p->case_wg_ident ? nullptr : p->d_case_wg, p->d_case_off,
                               part, nullptr, d_dt, s));
   return 0;

@@ -10,10 +10,11 @@
 namespace wmx {
 
 // Per-cell CFL time step, min over interiors; solver.py:139-150.
+template <bool BOX>
 __global__ __launch_bounds__(256) void k_dt_partial(const BlockDev* __restrict__ blks,
                                                     const int* __restrict__ wg_prefix, int nblk,
                                                     Ptrs q, NumDev nd, double* __restrict__ part) {
-  dt_partial_block(blks, wg_prefix, nblk, q, nd, part, (int)blockIdx.x, (int)gridDim.x);
+  dt_partial_block<BOX>(blks, wg_prefix, nblk, q, nd, part, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The work before a box plan's stage (pre_block)
@@ -327,9 +328,10 @@ hipError_t launch_cell_sb(const BlockDev& hb, unsigned* d_nz, hipStream_t s) {
 }
 
 hipError_t launch_dt_partial(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
-                             const NumDev& nd, double* d_part, hipStream_t s) {
+                             const NumDev& nd, double* d_part, bool box, hipStream_t s) {
   if (nwg <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_dt_partial, dim3(nwg), dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part);
+  hipLaunchKernelGGL(box ? k_dt_partial<true> : k_dt_partial<false>, dim3(nwg), dim3(256), 0, s, d_blks, d_pre, nblk, q,
+                     nd, d_part);
   return hipGetLastError();
 }
 
