@@ -36,6 +36,7 @@ UNITS = {
     "flux_ilp.hip": ["-ffp-contract=fast", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "flux3.hip": ["-ffp-contract=fast"],
     "fluxbox.hip": ["-ffp-contract=fast-honor-pragmas"],
+    "fluxcurv.hip": ["-ffp-contract=fast"],
     "mlp.hip": ["-ffp-contract=fast"],
     "ops.hip": ["-ffp-contract=fast"],
     "capi.hip": [],

@@ -2,7 +2,7 @@
 // one non-zero component, every centroid coordinate depends on one index, so the metrics of a
 // block are three one-dimensional tables (BoxEnt: width, its reciprocal and cube root, the
 // reciprocal centroid distance across the lower face).  The reference composition is that of
-// flux3_tile / k_flux1 (viscous.py:6-51, sgs.py, schemes.py, solver.py:78-121); what the
+// flux3_tile (viscous.py:6-51, sgs.py, schemes.py, solver.py:78-121); what the
 // metrics' zeros remove from it:
 //  * no geometry is read per cell (28 face-vector, centroid and volume words per cell and
 //    stage in the general form): the tables of a tile sit in LDS, those of the marching
@@ -369,6 +369,25 @@ __device__ __forceinline__ void grad_axis(const NumDev& nd, const R* c, const R 
   }
 }
 
+// halo job ht: 0..45 a ring cell whose gradient record the thread also evaluates (halo 2: row -1,
+// columns -1 and 16), 46..123 a cell that is only staged (halo 1)
+__device__ __forceinline__ void box_halo_job(int ht, int* hj, int* hk, int* halo) {
+  if (ht < NGRB) {
+    *halo = 2;
+    if (ht < TK) { *hj = -1; *hk = ht; }
+    else if (ht < TK + C2J) { *hj = ht - TK; *hk = -1; }
+    else { *hj = ht - TK - C2J; *hk = TK; }
+  } else if (ht < NHB) {
+    *halo = 1;
+    const int x = ht - NGRB;                     // rows -2 and 16 (20 each), corners of row -1 (4),
+    if (x < H2K) { *hj = -2; *hk = x - 2; }        // columns -2 and 17 of rows 0..15, -1 and 16 of row 15
+    else if (x < 2 * H2K) { *hj = BJ; *hk = x - H2K - 2; }
+    else if (x < 2 * H2K + 4) { const int y = x - 2 * H2K; *hj = -1; *hk = y < 2 ? y - 2 : TK + y - 2; }
+    else if (x < 2 * H2K + 4 + 2 * BJ) { const int y = x - 2 * H2K - 4; *hj = y >> 1; *hk = y & 1 ? TK + 1 : -2; }
+    else { *hj = C2J; *hk = x - (2 * H2K + 4 + 2 * BJ) ? TK : -1; }
+  }
+}
+
 }  // namespace
 
 // One marching tile (tiles[tile]) of a box plan's flux launch; called by every thread of a
@@ -449,24 +468,10 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
   const int sp_own = (tj + 2) * H2K + (tk + 2), sg_own = (tj + 1) * GB<R>::P + (tk + 1);
   // halo job by ht, the thread index turned by a multiple of 64 that changes from one of an
   // XCD's workgroups to the next (the jobs of two wavefronts would otherwise fall on the same
-  // two SIMDs of every CU): 0..45 a ring cell whose gradient record the thread also evaluates
-  // (row -1, columns -1 and 16), 46..123 a cell that is only staged
+  // two SIMDs of every CU)
   const int ht = (tid + 64 * ((tile >> 3) & 3)) & (NT - 1);
   int hj = 0, hk = 0, halo = 0;
-  if (ht < NGRB) {
-    halo = 2;
-    if (ht < TK) { hj = -1; hk = ht; }
-    else if (ht < TK + C2J) { hj = ht - TK; hk = -1; }
-    else { hj = ht - TK - C2J; hk = TK; }
-  } else if (ht < NHB) {
-    halo = 1;
-    const int x = ht - NGRB;                     // rows -2 and 16 (20 each), corners of row -1 (4),
-    if (x < H2K) { hj = -2; hk = x - 2; }        // columns -2 and 17 of rows 0..15, -1 and 16 of row 15
-    else if (x < 2 * H2K) { hj = BJ; hk = x - H2K - 2; }
-    else if (x < 2 * H2K + 4) { const int y = x - 2 * H2K; hj = -1; hk = y < 2 ? y - 2 : TK + y - 2; }
-    else if (x < 2 * H2K + 4 + 2 * BJ) { const int y = x - 2 * H2K - 4; hj = y >> 1; hk = y & 1 ? TK + 1 : -2; }
-    else { hj = C2J; hk = x - (2 * H2K + 4 + 2 * BJ) ? TK : -1; }
-  }
+  box_halo_job(ht, &hj, &hk, &halo);
   if (halo && !p_ok(J - tj + hj, K - tk + hk)) halo = 0;
   const bool ring_g = halo == 2 && g_ok(J - tj + hj, K - tk + hk);
   const unsigned hoff = halo ? (unsigned)(J - tj + hj) * N[2] + (unsigned)kcol(K - tk + hk) : 0;

@@ -377,9 +377,10 @@ int auto_ci_len(int nb, const int* dims, int prec, int cu_count, long long* ntil
   return best;
 }
 
-// The flux launches of a plan run the box kernels (box.h): every block's metrics are tensor
-// products, and an FP32-bulk plan evaluates its gradients in the march.
-bool box_active(const wmx_plan* p) { return p->box && (p->nd.prec != WMX_PREC_FP32_BULK || p->fuse_grad); }
+// The flux launches of a plan read the state itself and form records and gradients in the march:
+// every FP64 plan (box.h where its blocks' metrics are tensor products, else curv.h), and an
+// FP32-bulk plan of box blocks that evaluates its gradients in the march (box.h).
+bool direct(const wmx_plan* p) { return p->nd.prec != WMX_PREC_FP32_BULK || (p->box && p->fuse_grad); }
 
 // i-planes per tile of the box kernels when none is requested.  W workgroups share a CU (3 in
 // FP32, 2 in FP64), so T tiles are r full rounds of W CUs slots and a remainder.  A full round
@@ -415,7 +416,7 @@ void build_tiles(wmx_plan* p) {
   const int tjr = FLUX2_TILE_J;
   if (p->ci_req > 0) {
     p->ci_len = p->ci_req;
-  } else if (box_active(p)) {
+  } else if (direct(p)) {
     p->ci_len = box_ci_len(p);
   } else {
     std::vector<int> dims;
@@ -503,18 +504,18 @@ int run_fill(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, 
   return 0;
 }
 
-// The stage-2 state of a box plan: its gradient records' region, which the box kernels do not
-// use (64 or 120 B per cell for the 40 of a state).
+// The stage-2 state of a plan whose flux launch reads the state: its G region (FP32-bulk: the
+// unfused form's gradient records, 64 B per cell for the 40 of a state).
 Ptrs stage_buffer(const wmx_plan* p) {
-  static_assert(sizeof(float) * 4 * G32_GROUPS >= 5 * sizeof(double) && NGR >= 5, "a state fits the gradient records");
+  static_assert(sizeof(float) * 4 * G32_GROUPS >= 5 * sizeof(double), "a state fits the gradient records");
   Ptrs r;
   std::memset(&r, 0, sizeof(r));
   for (int b = 0; b < p->nb; ++b) r.p[b] = p->hb[b].G;
   return r;
 }
 
-// ghost fill, wall faces and (dt_out != nullptr) the CFL dt of one RHS evaluation of a box plan,
-// whose flux launch reads the state itself; the arguments of run_cells
+// ghost fill, wall faces and (dt_out != nullptr) the CFL dt of one RHS evaluation of a plan whose
+// flux launch reads the state itself; the arguments of run_cells
 int run_pre(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, hipStream_t s, double* dt_out,
             bool zfuse, bool fill) {
   const int nph = fill ? (int)p->phase_max.size() - (zfuse && p->fuse_last ? 1 : 0) : 0;
@@ -537,12 +538,17 @@ int run_pre(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, h
       w.nwall = (int)p->wall.size();
       w.wall_wgx = (p->wall_max + 255) / 256;
     }
+    if (!launched && p->d_sponge_pre) {
+      w.sponge = p->d_sponge_pre;
+      w.nsponge = p->sponge_pre.back();
+    }
     if (dt_due) w.fin = fin;
     dt_due = !launched && dt_out;
     if (dt_due) {
       w.dt_pre = p->d_pre_int;
       w.ndt = nwg_of(p->pre_int);
       w.part = p->d_part;
+      w.box = p->box ? 1 : 0;
     }
     WMX_CHECK(timed(p, K_FILL, s, [&] { return launch_pre(p->d_blks, p->nb, q, p->nd, w, s); }));
     launched = true;
@@ -561,7 +567,7 @@ int run_pre(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, h
     }));
   if (p->nd.net.w)
     WMX_CHECK(timed(p, K_WALL, s, [&] { return launch_wall(p->d_blks, p->d_wall, (int)p->wall.size(), p->wall_max, q, p->nd, s); }));
-  if (p->nd.n_sponge > 0)
+  if (p->nd.n_sponge > 0 && !p->d_sponge_pre)
     for (int b = 0; b < p->nb; ++b)
       WMX_CHECK(timed(p, K_SPONGE, s, [&] {
         return launch_sponge_mean(p->d_blks, b, (long long)p->hb[b].n[0] * p->hb[b].n[1], q, s);
@@ -569,23 +575,22 @@ int run_pre(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, h
   return 0;
 }
 
-// ghost fill + cell-level fields of one RHS evaluation
+// ghost fill + cell-level fields of one RHS evaluation (run_pre, or an FP32-bulk plan's records)
 // dt_out != nullptr: the primitive launch also takes the CFL partials of the (unchanged)
 // interior state and the per-case minimum goes to dt_out before the gradients
 // zfuse: a step's stage (the sweep's last phase evaluated by the primitive launch)
 int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef, hipStream_t s,
               double* dt_out = nullptr, bool zfuse = false, bool fill = true) {
   zfuse = zfuse && p->fuse_last && fill;
-  if (box_active(p)) return run_pre(p, q, time, d_dt, coef, s, dt_out, zfuse, fill);
+  if (direct(p)) return run_pre(p, q, time, d_dt, coef, s, dt_out, zfuse, fill);
   if (fill && run_fill(p, q, time, d_dt, coef, s, zfuse)) return 1;
   SpongeHead sh;
   if (p->d_sponge_pre) {
     sh.pre = p->d_sponge_pre;
     sh.nwg = p->sponge_pre.back();
   }
-  // fused FP32-bulk plans: the Newton wall faces ride in the primitive launch's head
-  const bool f32 = p->nd.prec == WMX_PREC_FP32_BULK;
-  const bool wall_in_prim = f32 && p->fuse_grad && !p->nd.net.w && !p->wall.empty() && p->wall_max > 0;
+  // fused plans: the Newton wall faces ride in the primitive launch's head
+  const bool wall_in_prim = p->fuse_grad && !p->nd.net.w && !p->wall.empty() && p->wall_max > 0;
   if (wall_in_prim) {
     sh.wall = p->d_wall;
     sh.wall_wgx = (p->wall_max + 255) / 256;
@@ -595,25 +600,20 @@ int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef,
     return launch_prim(p->d_blks, p->d_pre_all, p->nb, nwg_of(p->pre_all), q, p->nd,
                        dt_out ? p->d_part : nullptr, zfuse ? 1 : 0, sh, s);
   }));
-  // FP32-bulk plans take the per-case dt mins and (Newton model, unfused) the wall faces into
-  // the gradient launch; the flux kernel after it is the first reader of both
-  const bool wall_in_grad = f32 && !p->nd.net.w && !wall_in_prim;
+  // the per-case dt mins and (Newton model, unfused) the wall faces go into the gradient launch;
+  // the flux kernel after it is the first reader of both
+  const bool wall_in_grad = !p->nd.net.w && !wall_in_prim;
   GradDt gdt;
-  if (dt_out && f32) {
+  if (dt_out) {
     gdt.ncases = p->n_cases;
     gdt.list = p->case_wg_all_ident ? nullptr : p->d_case_wg_all;
     gdt.off = p->d_case_off_all;
     gdt.part = p->d_part;
     gdt.out = dt_out;
-  } else if (dt_out) {
-    WMX_CHECK(timed(p, K_DT, s, [&] {
-      return launch_case_final(0, p->n_cases, p->case_wg_all_ident ? nullptr : p->d_case_wg_all,
-                               p->d_case_off_all, p->d_part, nullptr, dt_out, s);
-    }));
   }
-  // fused FP32-bulk plans: the flux kernel evaluates the gradient records itself; the
+  // fused plans: the flux kernel evaluates the gradient records itself; the
   // gradient launch keeps only its head work (per-case dt min, Newton wall faces)
-  const bool grads = !(f32 && p->fuse_grad);
+  const bool grads = !p->fuse_grad;
   if (grads || gdt.out || wall_in_grad)
     WMX_CHECK(timed(p, K_GRAD, s, [&] {
       return launch_grad(p->d_blks, p->d_pre_box, p->nb, grads ? nwg_of(p->pre_box) : 0, p->nd,
@@ -632,9 +632,10 @@ int run_cells(wmx_plan* p, Ptrs q, double time, const double* d_dt, double coef,
 hipError_t plan_flux(const wmx_plan* p, int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles,
                      int ci_len, const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
                      bool zfuse, hipStream_t s) {
-  if (box_active(p))
-    return launch_box(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, zfuse && p->fuse_last, s);
-  if (nd.prec == WMX_PREC_FP32_BULK && p->fuse_grad)
+  if (direct(p))
+    return (p->box ? launch_box : launch_curv)(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt,
+                                               zfuse && p->fuse_last, s);
+  if (p->fuse_grad)
     return launch_flux3(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
   return launch_flux(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
 }
@@ -825,8 +826,7 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
   std::vector<long long> c_all, c_box, c_int, c_shell;
   for (auto& B : p->hb) {
     c_all.push_back(B.cells);
-    const int run = grad_run(nd.prec == WMX_PREC_FP32_BULK ? sizeof(float) : sizeof(double));
-    c_box.push_back((long long)((B.n[0] + 2 + run - 1) / run) * (B.n[1] + 2) * (B.n[2] + 2));
+    c_box.push_back((long long)((B.n[0] + 2 + GRAD_RUN - 1) / GRAD_RUN) * (B.n[1] + 2) * (B.n[2] + 2));
     c_int.push_back(((long long)B.n[0] * B.n[1] * B.n[2] + INT_CELLS - 1) / INT_CELLS);   // thread slots
     c_shell.push_back(B.shell_cells);
   }
@@ -870,11 +870,11 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
   p->off_wall.assign(nblocks, std::vector<long long>(6, -1));
   for (int b = 0; b < nblocks; ++b) {
     const BlockDev& B = p->hb[b];
-    const size_t rec = nd.prec == WMX_PREC_FP32_BULK ? sizeof(float) : sizeof(double);
+    const bool f32 = nd.prec == WMX_PREC_FP32_BULK;
     p->off_P.push_back(off);
-    off = align_up(off + rec * NP * B.cells);
+    off = align_up(off + (f32 ? sizeof(float) * NP : sizeof(double) * NCURV) * B.cells);
     p->off_G.push_back(off);
-    off = align_up(off + rec * (nd.prec == WMX_PREC_FP32_BULK ? 4 * G32_GROUPS : NGR) * B.cells);
+    off = align_up(off + (f32 ? sizeof(float) * 4 * G32_GROUPS : sizeof(double) * 5) * B.cells);
     p->off_geo32.push_back(off);
     if (nd.prec == WMX_PREC_FP32_BULK)
       off = align_up(off + sizeof(float) * (3 * (size_t)(fcount(B.N, 0) + fcount(B.N, 1) + fcount(B.N, 2)) +
@@ -1026,7 +1026,10 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
     std::vector<unsigned> nz(p->nb + 1);
     WMX_CHECK(hipMemcpy(nz.data(), d_nz, sizeof(unsigned) * (p->nb + 1), hipMemcpyDeviceToHost));
     p->box = nz[p->nb] == 0;
-    // the box kernels read a fused side's k ghosts at their periodic images: a side that is no
+    // (half reciprocal volumes and filter widths of the curvilinear FP64 kernel)
+    if (!p->box && p->nd.prec != WMX_PREC_FP32_BULK)
+      for (int b = 0; b < p->nb; ++b) WMX_CHECK(launch_curv_geo(p->hb[b], nullptr));
+    // those kernels and the box kernels read a fused side's k ghosts at their periodic images: a side that is no
     // plain periodic face of its own block is filled by a launch
     bool image = true;
     for (int b = 0; b < p->nb; ++b)
@@ -1036,7 +1039,7 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
           image = image && f.kind == WMX_FACE_INTERFACE && f.nb == b && f.src_axis == 2 && f.src_side == 1 - sd &&
                   f.mapping[0] == 0 && f.mapping[1] == 1 && !f.flip[0] && !f.flip[1];
         }
-    if (p->box && !image) {
+    if ((p->box || p->nd.prec != WMX_PREC_FP32_BULK) && !image) {
       p->fuse_last = false;
       for (BlockDev& B : p->hb) B.zfuse = 0;
     }
@@ -1339,7 +1342,7 @@ int upload_stage(wmx_plan* p) {
   if (p->fuse_grad) st.ngrad = 0;                 // the gradient list keeps only its dt head
   st.dt_list = p->case_wg_all_ident ? nullptr : p->d_case_wg_all;
   st.dt_off = p->d_case_off_all;
-  if (box_active(p)) {                            // CFL partials by the interior cells
+  if (direct(p)) {                            // CFL partials by the interior cells
     st.pre_all = p->d_pre_int;
     st.nprim = nwg_of(p->pre_int);
     st.dt_list = p->case_wg_ident ? nullptr : p->d_case_wg;
@@ -1364,7 +1367,7 @@ int advance_persistent(wmx_plan* p, double* const* q0, double* const* qout, doub
   hipStream_t s = as_stream(stream);
   Ptrs P0 = make_ptrs(p, q0), PO = make_ptrs(p, qout);
   WMX_CHECK(launch_shell_save(p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), P0, s));
-  const Ptrs P2 = box_active(p) ? stage_buffer(p) : PO;
+  const Ptrs P2 = direct(p) ? stage_buffer(p) : PO;
   const int sc = scheme_config(p->nd);
   const int nph = (int)p->phase_max.size();
   const int wx = !p->wall.empty() && p->wall_max > 0 ? (p->wall_max + 255) / 256 : 0;
@@ -1383,7 +1386,7 @@ int advance_persistent(wmx_plan* p, double* const* q0, double* const* qout, doub
     c.d_dt = d_dt;
     c.dt_host = dt;
     WMX_CHECK(timed(p, K_FLUX, s, [&] {
-      const int form = box_active(p) ? 2 : (p->fuse_grad ? 1 : 0);
+      const int form = direct(p) ? 2 : (p->fuse_grad ? 1 : 0);
       return launch_stage(mode, sc, form, p->d_stage, c, &p->stage_grid[form], s);
     }));
   }
@@ -1402,8 +1405,8 @@ int advance_impl(wmx_plan* p, double* const* q0, double* const* qout, double dt,
   WMX_CHECK(timed(p, K_SHELL, s, [&] { return launch_shell_save(p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), P0, s); }));
   // stage times t, t + dt, t + dt/2 (solver.py:125-129)
   const double t1 = d_dt ? time : time + dt, t2 = d_dt ? time : time + 0.5 * dt;
-  // a box plan's flux launch reads its neighbours' states: stage 2 goes to a second buffer
-  const Ptrs P2 = box_active(p) ? stage_buffer(p) : PO;
+  // a flux launch that reads its neighbours' states: stage 2 goes to a second buffer
+  const Ptrs P2 = direct(p) ? stage_buffer(p) : PO;
   if (run_cells(p, P0, time, nullptr, 0.0, s, dt_out, true)) return 1;
   WMX_CHECK(timed(p, K_FLUX, s, [&] { return plan_flux(p, 1, p->d_blks, p->d_tiles, ntiles, p->ci_len, p->nd, P0, P0, PO, d_dt, dt, true, s); }));
   if (run_cells(p, PO, t1, d_dt, 1.0, s, nullptr, true)) return 1;

@@ -8,18 +8,15 @@
 
 namespace wmx {
 
-constexpr int NP = 8;    // prim planes: rho u v w p T mu e_int
-constexpr int NGR = 15;  // gradient record planes: g[4][3], mu_eff, k_eff, theta
+constexpr int NP = 8;    // FP32-bulk primitive record: rho u v w p T mu e_int
+constexpr int NCURV = 2; // FP64 planes that curv.h keeps: half the reciprocal volume, filter width
 constexpr int WALL_PLANES = 7;  // Fw[5], tau, qw
 
-enum PrimPlane { P_R = 0, P_U, P_V, P_W, P_P, P_T, P_MU, P_E };
-enum GradPlane { G_MU = 12, G_K = 13, G_TH = 14 };
-// FP64 records are plane-major (plane v of cell c at v * cells + c).  FP32-bulk records
-// move in 16-byte groups: the primitive record is two planes of float4,
+// FP32-bulk records move in 16-byte groups: the primitive record is two planes of float4,
 // Pf[4 c ..] = (u, v, w, T') and Pf[4 cells + 4 c ..] = (rho, p', mu, e'), so the
 // gradient kernel reads one group per neighbour; the gradient record is four planes of
-// float4, Gf[4 (q cells + c) ..] for q = 0..3 holding GradPlane entries 4q..4q+3 (the last
-// group (mu_eff, k_eff, theta, 0)).  Every 16-byte access of a wavefront is contiguous.
+// float4, Gf[4 (q cells + c) ..] for q = 0..3 holding the components 4q..4q+3 of (g[4][3],
+// mu_eff, k_eff, theta, 0).  Every 16-byte access of a wavefront is contiguous.
 constexpr int G32_GROUPS = 4;
 
 struct Ptrs {
@@ -44,10 +41,10 @@ struct BlockDev {
   const double* xc;
   const double* S[3];
   const double* xf[3];
-  double* P;                // NP planes (FP64 form)
-  double* G;                // NGR planes (FP64 form)
+  double* P;                // NCURV planes (FP64 form)
+  double* G;                // five planes: a stage's state (direct plans; FP32-bulk: over Gf)
   float* Pf;                // NP planes (FP32-bulk form; same workspace region as P)
-  float* Gf;                // NGR planes (FP32-bulk form)
+  float* Gf;                // 4 G32_GROUPS planes (FP32-bulk form; same region as G)
   float* Sf[3];             // FP32-bulk form: float copies of S[d] (gradient kernel)
   float* volf;              // FP32-bulk form: float copy of vol
   double* Sb;               // CFL metric planes (NSB_PLANES: the cell means of the face vectors
@@ -103,8 +100,7 @@ struct NumDev {
 };
 
 constexpr int FLUX2_TILE_J = 15;   // cell rows of a flux-kernel tile (flux.hip)
-// i cells per thread of the gradient kernel (rhs.hip): 4 in FP32, 1 in FP64
-constexpr int grad_run(size_t rec_bytes) { return rec_bytes == 4 ? 4 : 1; }
+constexpr int GRAD_RUN = 4;        // i cells per thread of the FP32-bulk gradient kernel (rhs.hip)
 
 struct GhostOp {
   int blk;       // destination block
@@ -162,17 +158,20 @@ struct GradDt {
   const double* part = nullptr;    // CFL partials
   double* out = nullptr;           // dt per case
 };
-// What a stage of a box plan does before its flux launch, as one launch per sweep phase: the
-// phase's ghost fills and, where they are given, the Newton wall faces, the CFL partials (both
-// read interior states only) and the per-case dt mins of partials that an earlier launch took.
+// What a stage of a plan whose flux launch reads the state does before it, as one launch per
+// sweep phase: the phase's ghost fills and, where they are given, the Newton wall faces, the
+// sponge means, the CFL partials (all of interior states only) and the per-case dt mins of
+// partials that an earlier launch took.
 struct PreWork {
   const GhostOp* ops = nullptr;    // the phase's fill ops, `per` workgroups each
   int nops = 0, per = 0;
   const WallOp* wall = nullptr;    // wall ops, `wall_wgx` workgroups each
   int nwall = 0, wall_wgx = 0;
   const int* dt_pre = nullptr;     // CFL partials: workgroups per block (prefix)
-  int ndt = 0;
+  int ndt = 0, box = 0;            // (box: every block is one)
   double* part = nullptr;
+  const int* sponge = nullptr;     // sponge means: workgroups per block (prefix), 32 rows each
+  int nsponge = 0;
   GradDt fin;                      // the dt mins (ncases 0: none)
   int head = 0;                    // set by the launcher
 };
@@ -197,6 +196,11 @@ hipError_t launch_flux3(int mode, const BlockDev* d_blks, const int4* d_tiles, i
 hipError_t launch_box(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
                       const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
                       int zfuse, hipStream_t s);
+// FP64 plans with other blocks (curv.h), on the same terms
+hipError_t launch_curv(int mode, const BlockDev* d_blks, const int4* d_tiles, int ntiles, int ci_len,
+                       const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
+                       int zfuse, hipStream_t s);
+hipError_t launch_curv_geo(const BlockDev& hb, hipStream_t s);
 // fills a block's BoxEnt tables; *d_bad becomes non-zero if the block is no box
 hipError_t launch_box_check(const BlockDev& hb, unsigned* d_bad, hipStream_t s);
 hipError_t launch_shell_save(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,

@@ -37,20 +37,7 @@ struct ColGT {
   R th;
 };
 
-template <class R, class PT>
-__device__ __forceinline__ ColT<R> load_col(PT P, long long cells, long long c) {
-  ColT<R> o;
-  o.w.r = P[c];
-  o.w.u = P[cells + c];
-  o.w.v = P[2 * cells + c];
-  o.w.w = P[3 * cells + c];
-  o.w.p = P[4 * cells + c];
-  o.w.e = P[P_E * cells + c];
-  o.T = P[P_T * cells + c];
-  return o;
-}
-
-// the same from the FP32-bulk records (two / four 16-byte loads)
+// from the FP32-bulk records (two / four 16-byte loads)
 __device__ __forceinline__ ColT<float> load_col32(const float* P, size_t cells, size_t c) {
   const float4 a = ld4(P + 4 * c), b = ld4(P + 4 * (cells + c));
   ColT<float> o;
@@ -68,17 +55,6 @@ __device__ __forceinline__ ColGT<float> load_colg32(const float* G, size_t cells
   o.g.g[4] = b.x; o.g.g[5] = b.y; o.g.g[6] = b.z; o.g.g[7] = b.w;
   o.g.g[8] = d.x; o.g.g[9] = d.y; o.g.g[10] = d.z; o.g.g[11] = d.w;
   o.g.mu = e.x; o.g.k = e.y; o.th = e.z;
-  return o;
-}
-
-template <class R, class PT>
-__device__ __forceinline__ ColGT<R> load_colg(PT G, long long cells, long long c) {
-  ColGT<R> o;
-#pragma unroll
-  for (int i = 0; i < 12; ++i) o.g.g[i] = G[i * cells + c];
-  o.g.mu = G[G_MU * cells + c];
-  o.g.k = G[G_K * cells + c];
-  o.th = G[G_TH * cells + c];
   return o;
 }
 

@@ -103,7 +103,7 @@ __device__ __forceinline__ void grad32_block(const BlockDev* __restrict__ blks,
   const BlockDev& B = blks[b];
   const int ng = B.ng;
   const int b0 = B.n[0] + 2, b1 = B.n[1] + 2, b2 = B.n[2] + 2;
-  constexpr int RUN = grad_run(sizeof(float));
+  constexpr int RUN = GRAD_RUN;
   const int nrun = (b0 + RUN - 1) / RUN;
   const int l = (wg - wg_prefix[b]) * (int)blockDim.x + (int)threadIdx.x;
   if (l >= nrun * b1 * b2) return;

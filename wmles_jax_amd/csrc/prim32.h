@@ -221,46 +221,6 @@ __device__ __forceinline__ void dt_partial_block(const BlockDev* __restrict__ bl
   if (threadIdx.x == 0) part[wg] = r;
 }
 
-// Workgroup wgx of nwg of the work before a box plan's stage (PreWork): the dt mins, the wall
-// faces and the ghost fills first (w.head workgroups, a multiple of 8), then the CFL partials.
-__device__ __forceinline__ void pre_block(const BlockDev* __restrict__ blks, int nblk, const Ptrs& q,
-                                          const NumDev& nd, const PreWork& w, int wgx, int nwg) {
-  if (wgx >= w.head) {
-    dt_partial_block<true>(blks, w.dt_pre, nblk, q, nd, w.part, wgx - w.head, nwg - w.head);
-    return;
-  }
-  if (wgx < w.fin.ncases) {
-    const int lo = w.fin.off[wgx], hi = w.fin.off[wgx + 1];
-    double a = __builtin_huge_val();
-    for (int t0 = lo + (int)threadIdx.x; t0 < hi; t0 += 16 * (int)blockDim.x) {
-      double va[16];                             // clamped: a repeated element leaves a min unchanged
-#pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int t = min(t0 + u * (int)blockDim.x, hi - 1);
-        va[u] = w.fin.part[w.fin.list ? w.fin.list[t] : t];
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) a = nmin(a, va[u]);
-    }
-    a = block_reduce<true>(a);
-    if (threadIdx.x == 0) w.fin.out[wgx] = a;
-    return;
-  }
-  int h = wgx - w.fin.ncases;
-  if (h < w.wall_wgx * w.nwall) {
-    const int i = h / w.wall_wgx;
-    const WallOp op = w.wall[i];
-    const int idx = (h - i * w.wall_wgx) * (int)blockDim.x + (int)threadIdx.x;
-    if (idx < op.count) wall_face<false>(blks, op, idx, q, nd, nullptr, nullptr);
-    return;
-  }
-  h -= w.wall_wgx * w.nwall;
-  if (h < w.nops * w.per) {
-    const int i = h / w.per;
-    fill_cell(blks, w.ops[i], q, nd.gas, (h - i * w.per) * (int)blockDim.x + (int)threadIdx.x);
-  }
-}
-
 // Spanwise mean of sponge row `row` for rows of 9..129 cells (numpy's pairwise order for
 // the elements 1..nk-1 by eight lanes u of the row, combined by shuffles in that order);
 // every lane of the 8-lane group calls it.  smooth_ramp.py:214-216.
@@ -316,6 +276,53 @@ __device__ __forceinline__ void sponge_head(const BlockDev* __restrict__ blks, i
   const int ng = B.ng;
   const long long c0 = live ? cidx(B.N, ng + (int)(row / B.n[1]), ng + (int)(row % B.n[1]), ng) : 0;
   sponge_row_fast(B, row, u, live, c0, q.p[b]);
+}
+
+// Workgroup wgx of nwg of the work before a stage whose flux launch reads the state (PreWork):
+// the dt mins, the wall faces, the ghost fills and the sponge means first (w.head workgroups, a
+// multiple of 8), then the CFL partials.
+__device__ __forceinline__ void pre_block(const BlockDev* __restrict__ blks, int nblk, const Ptrs& q,
+                                          const NumDev& nd, const PreWork& w, int wgx, int nwg) {
+  if (wgx >= w.head) {
+    if (w.box) dt_partial_block<true>(blks, w.dt_pre, nblk, q, nd, w.part, wgx - w.head, nwg - w.head);
+    else dt_partial_block<false>(blks, w.dt_pre, nblk, q, nd, w.part, wgx - w.head, nwg - w.head);
+    return;
+  }
+  if (wgx < w.fin.ncases) {
+    const int lo = w.fin.off[wgx], hi = w.fin.off[wgx + 1];
+    double a = __builtin_huge_val();
+    for (int t0 = lo + (int)threadIdx.x; t0 < hi; t0 += 16 * (int)blockDim.x) {
+      double va[16];                             // clamped: a repeated element leaves a min unchanged
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const int t = min(t0 + u * (int)blockDim.x, hi - 1);
+        va[u] = w.fin.part[w.fin.list ? w.fin.list[t] : t];
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a = nmin(a, va[u]);
+    }
+    a = block_reduce<true>(a);
+    if (threadIdx.x == 0) w.fin.out[wgx] = a;
+    return;
+  }
+  int h = wgx - w.fin.ncases;
+  if (h < w.wall_wgx * w.nwall) {
+    const int i = h / w.wall_wgx;
+    const WallOp op = w.wall[i];
+    const int idx = (h - i * w.wall_wgx) * (int)blockDim.x + (int)threadIdx.x;
+    if (idx < op.count) wall_face<false>(blks, op, idx, q, nd, nullptr, nullptr);
+    return;
+  }
+  h -= w.wall_wgx * w.nwall;
+  if (h < w.nops * w.per) {
+    const int i = h / w.per;
+    fill_cell(blks, w.ops[i], q, nd.gas, (h - i * w.per) * (int)blockDim.x + (int)threadIdx.x);
+    return;
+  }
+  SpongeHead sh;
+  sh.pre = w.sponge;
+  sh.nwg = w.nsponge;
+  sponge_head(blks, nblk, q, sh, h - w.nops * w.per);
 }
 
 // ------------------------------------------------------------------------------ prim

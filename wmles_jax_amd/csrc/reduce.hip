@@ -17,52 +17,10 @@ __global__ __launch_bounds__(256) void k_dt_partial(const BlockDev* __restrict__
   dt_partial_block<BOX>(blks, wg_prefix, nblk, q, nd, part, (int)blockIdx.x, (int)gridDim.x);
 }
 
-// The work before a box plan's stage (pre_block)
+// The work before a stage whose flux launch reads the state (pre_block)
 __global__ __launch_bounds__(256) void k_pre(const BlockDev* __restrict__ blks, int nblk, Ptrs q, NumDev nd,
                                              PreWork w) {
   pre_block(blks, nblk, q, nd, w, (int)blockIdx.x, (int)gridDim.x);
-}
-
-// FP64 record (r, u, v, w, p, T, mu, e_int)
-template <bool DT>
-__global__ __launch_bounds__(256) void k_prim(const BlockDev* __restrict__ blks,
-                                              const int* __restrict__ wg_prefix, int nblk,
-                                              Ptrs q, NumDev nd, double* __restrict__ part,
-                                              int zfuse, SpongeHead sh) {
-  if ((int)blockIdx.x < sh.head) {
-    sponge_head(blks, nblk, q, sh, (int)blockIdx.x);
-    return;
-  }
-  // XCD-contiguous spans: the i faces one plane apart that the CFL partial reads twice
-  // stay in one L2
-  const int wg = xcd_span((int)blockIdx.x - sh.head, (int)gridDim.x - sh.head);
-  const int b = find_block_r(wg_prefix, nblk, wg);
-  const BlockDev& B = blks[b];
-  const long long c = (long long)(wg - wg_prefix[b]) * blockDim.x + threadIdx.x;
-  const long long cells = B.cells;
-  double dtc = __builtin_huge_val();
-  int I = 0, J = 0, K = 0;
-  if (c < cells) cell_ijk(B, (unsigned)c, &I, &J, &K);
-  if (c < cells && rec_read(B, I, J, K)) {
-    const GasC& gas = nd.gas;
-    double qv[5];
-    prim_state(blks, b, c, q, gas, zfuse, qv);
-    const Prim w = cons_to_prim(gas, qv[0], qv[1], qv[2], qv[3], qv[4]);
-    double* P = B.P;
-    P[c] = w.r;
-    P[cells + c] = w.u;
-    P[2 * cells + c] = w.v;
-    P[3 * cells + c] = w.w;
-    P[4 * cells + c] = w.p;
-    P[5 * cells + c] = w.T;
-    P[6 * cells + c] = mu_suth(gas, w.T);
-    P[7 * cells + c] = w.p / ((gas.gamma - 1.0) * w.r);
-    if (DT && interior_of(B, (unsigned)c, &I, &J, &K)) dtc = cell_dt(B, nd, (unsigned)c, I, J, K, w);
-  }
-  if (DT) {
-    const double r = block_reduce<true>(dtc);
-    if (threadIdx.x == 0) part[wg] = r;
-  }
 }
 
 template <bool DT>
@@ -337,7 +295,7 @@ hipError_t launch_dt_partial(const BlockDev* d_blks, const int* d_pre, int nblk,
 
 hipError_t launch_pre(const BlockDev* d_blks, int nblk, Ptrs q, const NumDev& nd, PreWork w, hipStream_t s) {
   if (!w.fin.out) w.fin.ncases = 0;
-  w.head = (w.fin.ncases + w.wall_wgx * w.nwall + w.nops * w.per + 7) / 8 * 8;   // (keeps the XCD spans)
+  w.head = (w.fin.ncases + w.wall_wgx * w.nwall + w.nops * w.per + w.nsponge + 7) / 8 * 8;   // (keeps the XCD spans)
   if (w.head + w.ndt <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_pre, dim3(w.head + w.ndt), dim3(256), 0, s, d_blks, nblk, q, nd, w);
   return hipGetLastError();
@@ -346,18 +304,12 @@ hipError_t launch_pre(const BlockDev* d_blks, int nblk, Ptrs q, const NumDev& nd
 hipError_t launch_prim(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
                        const NumDev& nd, double* d_part, int zfuse, SpongeHead sh, hipStream_t s) {
   if (nwg <= 0) return hipSuccess;
-  const bool f32 = nd.prec == WMX_PREC_FP32_BULK;
   if (!sh.pre) sh.nwg = 0;
   if (!sh.wall) sh.wall_wgx = sh.nwall = 0;
   sh.head = ((sh.nwg + sh.wall_wgx * sh.nwall) + 7) / 8 * 8;   // (keeps the XCD spans)
   const dim3 grid(nwg + sh.head);
-  if (d_part) {
-    if (f32) hipLaunchKernelGGL(k_prim32<true>, grid, dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part, zfuse, sh);
-    else hipLaunchKernelGGL(k_prim<true>, grid, dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part, zfuse, sh);
-  } else {
-    if (f32) hipLaunchKernelGGL(k_prim32<false>, grid, dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part, zfuse, sh);
-    else hipLaunchKernelGGL(k_prim<false>, grid, dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part, zfuse, sh);
-  }
+  hipLaunchKernelGGL(d_part ? k_prim32<true> : k_prim32<false>, grid, dim3(256), 0, s, d_blks, d_pre, nblk, q, nd, d_part,
+                     zfuse, sh);
   return hipGetLastError();
 }
 

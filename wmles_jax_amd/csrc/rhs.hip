@@ -14,88 +14,6 @@ namespace wmx {
 
 
 // ------------------------------------------------------------------------------ grad
-// FP64: one thread per cell.
-template <class R>
-__global__ __launch_bounds__(256) void k_grad_cell(const BlockDev* __restrict__ blks,
-                                              const int* __restrict__ wg_prefix, int nblk,
-                                              NumDev nd) {
-  const int wg = blockIdx.x;
-  const int b = find_block(wg_prefix, nblk, wg);
-  const BlockDev& B = blks[b];
-  const int ng = B.ng;
-  const int b0 = B.n[0] + 2, b1 = B.n[1] + 2, b2 = B.n[2] + 2;
-  long long l = (long long)(wg - wg_prefix[b]) * blockDim.x + threadIdx.x;
-  if (l >= (long long)b0 * b1 * b2) return;
-  const int K = ng - 1 + (int)(l % b2);
-  const int J = ng - 1 + (int)((l / b2) % b1);
-  const int I = ng - 1 + (int)(l / ((long long)b1 * b2));
-  const int* N = B.N;
-  const long long cells = B.cells;
-  const long long c = cidx(N, I, J, K);
-  const long long st[3] = {(long long)N[1] * N[2], (long long)N[2], 1};
-  const R* P = sizeof(R) == 8 ? (const R*)B.P : (const R*)B.Pf;
-  const int pl[4] = {P_U, P_V, P_W, P_T};
-  R phi0[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) phi0[v] = P[pl[v] * cells + c];
-  R acc[12];
-#pragma unroll
-  for (int i = 0; i < 12; ++i) acc[i] = R(0.0);
-  int cc[3] = {I, J, K};
-  const R h = R(0.5);
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double* S = B.S[d];
-    const long long fc = fcount(N, d);
-    int hi[3] = {cc[0], cc[1], cc[2]};
-    hi[d] += 1;
-    const long long flo = fidx(N, d, cc[0], cc[1], cc[2]);
-    const long long fhi = fidx(N, d, hi[0], hi[1], hi[2]);
-    R Slo[3] = {R(S[flo]), R(S[fc + flo]), R(S[2 * fc + flo])};
-    R Shi[3] = {R(S[fhi]), R(S[fc + fhi]), R(S[2 * fc + fhi])};
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      R pm = P[pl[v] * cells + c - st[d]];
-      R pp = P[pl[v] * cells + c + st[d]];
-      R flo_v = h * (pm + phi0[v]);
-      R fhi_v = h * (phi0[v] + pp);
-#pragma unroll
-      for (int x = 0; x < 3; ++x) acc[3 * v + x] = acc[3 * v + x] + (fhi_v * Shi[x] - flo_v * Slo[x]);
-    }
-  }
-  const double vol = B.vol[c];
-  const R volr = R(vol);
-  // one reciprocal of the volume (within an ulp of the reference's twelve divisions)
-  const R ivol = fdiv<R>(R(1.0), volr);
-  R g[12];
-#pragma unroll
-  for (int i = 0; i < 12; ++i) g[i] = acc[i] * ivol;
-  const R rho = P[c];
-  const R mu = P[P_MU * cells + c];
-  R mut = R(0.0);
-  if (nd.sgs != WMX_SGS_NONE) {
-    // filter width vol^(1/3) (solver.py:82); FP32-bulk: single-precision cube root
-    R delta;
-    if constexpr (sizeof(R) == 4) delta = cbrtf((float)vol);
-    else delta = R(cbrt(vol));                   // vol ** (1/3), within an ulp
-    const R cs = R(nd.sgs_c);
-    R nut;
-    if (nd.sgs == WMX_SGS_SMAGORINSKY) nut = nut_smagorinsky<R>(g, delta, cs);
-    else if (nd.sgs == WMX_SGS_WALE) nut = nut_wale<R>(g, delta, cs);
-    else nut = nut_vreman<R>(g, delta, cs);
-    mut = rho * nut;
-  } else {
-    mut = R(0.0) * rho;
-  }
-  R* G = sizeof(R) == 8 ? (R*)B.G : (R*)B.Gf;
-#pragma unroll
-  for (int i = 0; i < 12; ++i) G[i * cells + c] = g[i];
-  const GasC& gs = nd.gas;
-  G[G_MU * cells + c] = mu + mut;
-  G[G_K * cells + c] = R(gs.cp) * (fdiv<R>(mu, R(gs.Pr)) + fdiv<R>(mut, R(gs.Pr_t)));
-  G[G_TH * cells + c] = ducros<R>(g);
-}
-
 template <int SGS>
 __global__ __launch_bounds__(256) void k_grad32(const BlockDev* __restrict__ blks,
                                                 const int* __restrict__ wg_prefix, int nblk,
@@ -270,26 +188,23 @@ hipError_t launch_wm_eval(const NumDev& nd, int mode, long long n, const double*
 hipError_t launch_grad(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, const NumDev& nd,
                        const WallOp* d_wall, int nwall_ops, int wall_max, Ptrs q, const GradDt& gdt,
                        hipStream_t s) {
-  if (nd.prec == WMX_PREC_FP32_BULK) {
-    // side work in the same launch: per-case dt mins, then Newton wall faces (padded to 8);
-    // nwg == 0 (fused plans): the side work alone
-    const int wx = d_wall && nwall_ops > 0 && wall_max > 0 ? (wall_max + 255) / 256 : 0;
-    const int ndt = gdt.out ? gdt.ncases : 0;
-    const int head = ((ndt + wx * nwall_ops + 7) / 8) * 8;
-    if (nwg + head <= 0) return hipSuccess;
-    const dim3 grid(nwg + head);
+  // side work in the same launch: per-case dt mins, then Newton wall faces (padded to 8);
+  // nwg == 0 (fused plans): the side work alone
+  const int wx = d_wall && nwall_ops > 0 && wall_max > 0 ? (wall_max + 255) / 256 : 0;
+  const int ndt = gdt.out ? gdt.ncases : 0;
+  const int head = ((ndt + wx * nwall_ops + 7) / 8) * 8;
+  if (nwg + head <= 0) return hipSuccess;
+  const dim3 grid(nwg + head);
 #define WMX_GRAD32(S)                                                                          \
   hipLaunchKernelGGL(k_grad32<S>, grid, dim3(256), 0, s, d_blks, d_pre, nblk, nd, head, d_wall, \
-                     wx, nwall_ops, q, ndt, gdt.list, gdt.off, gdt.part, gdt.out)
-    switch (nd.sgs) {
-      case WMX_SGS_NONE: WMX_GRAD32(WMX_SGS_NONE); break;
-      case WMX_SGS_SMAGORINSKY: WMX_GRAD32(WMX_SGS_SMAGORINSKY); break;
-      case WMX_SGS_WALE: WMX_GRAD32(WMX_SGS_WALE); break;
-      default: WMX_GRAD32(WMX_SGS_VREMAN);
-    }
+                   wx, nwall_ops, q, ndt, gdt.list, gdt.off, gdt.part, gdt.out)
+  switch (nd.sgs) {
+    case WMX_SGS_NONE: WMX_GRAD32(WMX_SGS_NONE); break;
+    case WMX_SGS_SMAGORINSKY: WMX_GRAD32(WMX_SGS_SMAGORINSKY); break;
+    case WMX_SGS_WALE: WMX_GRAD32(WMX_SGS_WALE); break;
+    default: WMX_GRAD32(WMX_SGS_VREMAN);
+  }
 #undef WMX_GRAD32
-  } else if (nwg > 0)
-    hipLaunchKernelGGL(k_grad_cell<double>, dim3(nwg), dim3(256), 0, s, d_blks, d_pre, nblk, nd);
   return hipGetLastError();
 }
 

@@ -28,6 +28,7 @@ __device__ void st_pre(const StageStatic& s, double* __restrict__ part, int wgx)
   w.nwall = s.prim_wall_wgx > 0 ? s.nwall_ops : 0;
   w.head = s.prim_head;
   w.dt_pre = s.pre_all;
+  w.box = 1;
   w.part = part;
   pre_block(s.blks, s.nblk, s.pbuf[0], s.nd, w, wgx, s.prim_head + s.nprim);
 }

@@ -76,7 +76,7 @@ __device__ __forceinline__ void wall_face(const BlockDev* __restrict__ blks, con
   W[5 * nw + idx] = tau;
   W[6 * nw + idx] = qw;
 }
-// FP32-bulk gradient / SGS / Ducros.  One thread per run of grad_run(4) consecutive i
+// FP32-bulk gradient / SGS / Ducros.  One thread per run of GRAD_RUN consecutive i
 // cells of one (j, k) column: the i neighbours' phi and the shared i-face vectors stay in
 // registers from one cell of the run to the next, so the planes i-1 / i+1 (far apart in
 // memory) are read about once instead of three times.  Per cell the arithmetic is that
