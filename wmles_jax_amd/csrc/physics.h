@@ -117,10 +117,10 @@ WMX_HD void bc_farfield(const GasC& g, const double* src, const double* pinf, do
 template <class R>
 WMX_HD R fdiv(R a, R b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-#pragma clang fp contract(off)
   if constexpr (sizeof(R) == 4) {
-    return a * __builtin_amdgcn_rcpf(b);
+    return a * __builtin_amdgcn_rcpf(b);         // (its product contracts with what follows it)
   } else {
+#pragma clang fp contract(off)
     double y = __builtin_amdgcn_rcp(b);
     y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
     const double q = a * y;
@@ -133,10 +133,10 @@ WMX_HD R fdiv(R a, R b) {
 template <class R>
 WMX_HD R fsqrt(R a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-#pragma clang fp contract(off)
   if constexpr (sizeof(R) == 4) {
     return __builtin_amdgcn_sqrtf(a);
   } else {
+#pragma clang fp contract(off)
     const double y = __builtin_amdgcn_rsq(a), s = a * y, h = 0.5 * y, e = __builtin_fma(-h, s, 0.5);
     const double s1 = __builtin_fma(s, e, s), h1 = __builtin_fma(h, e, h);
     const double r = __builtin_fma(__builtin_fma(-s1, s1, a), h1, s1);
