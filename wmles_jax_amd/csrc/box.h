@@ -22,7 +22,7 @@
 // The state is read, not a primitive record: each thread forms the records of its column and
 // of a halo cell one plane ahead (rec_of), so no primitive launch writes 32 / 64 B per cell for
 // this one to read back with a halo.  Channel of 256 x 128 x 128 cells, Hybrid + Vreman, per
-// stage: FP32 307 us against 253 us on records and 78 us that wrote them; FP64 458 us against
+// stage: FP32 271 us against 253 us on records and 78 us that wrote them; FP64 423 us against
 // 461 us + 137 us.  It is bound by vector issue (about 200 us of the FP32 launch) and by the
 // state loads' latency at three (FP64: two) waves per SIMD.
 //
@@ -416,16 +416,15 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
   const BlockDev& B = blks[t.x];
   const int j0 = t.y, k0 = t.z, i0 = t.w;
   const int i1 = min(i0 + ci_len, B.n[0]);
-  const int tid = threadIdx.x;
-  const int tj = (tid >> 6) + 4 * ((tid >> 4) & 3), tk = tid & 15;   // tile_tid(tj, tk) == tid
+  int tid = threadIdx.x;
+  int tj = (tid >> 6) + 4 * ((tid >> 4) & 3), tk = tid & 15;         // tile_tid(tj, tk) == tid
   const int ng = B.ng;
   const int* N = B.N;
   const int n0 = B.n[0], n1 = B.n[1], n2 = B.n[2];
-  const int j = j0 + tj, k = k0 + tk;
   const bool own = tj < C2J;
-  const bool act = own && j < n1 && k < n2;
+  const bool act = own && j0 + tj < n1 && k0 + tk < n2;
   const int jl = min(j0 + C2J, n1) - j0, kl = min(k0 + TK, n2) - k0;
-  const int J = ng + j, K = ng + k;
+  int J = ng + j0 + tj, K = ng + k0 + tk;
   const unsigned cells = (unsigned)B.cells, sI = (unsigned)N[1] * N[2];
   const double dt = d_dt ? d_dt[B.case_id] : dt_host;
   const bool keep = SC == SC_ANY && (nd.scheme == WMX_SCHEME_KEEP ||
@@ -462,20 +461,39 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
 #pragma unroll
     for (int v = 0; v < 5; ++v) q[v] = ldu(qi + v * (size_t)cells, c);
   };
-  // own column (clamped into the array) and its slots
-  const unsigned cb = (unsigned)min(J, N[1] - 1) * N[2] + kcol(min(K, N[2] - 1));
+  // own column and its slots; halo job by ht, the thread index turned by a multiple of 64 that
+  // changes from one of an XCD's workgroups to the next (the jobs of two wavefronts would
+  // otherwise fall on the same two SIMDs of every CU), its cell in one word
   const bool own_p = p_ok(J, K), own_g = g_ok(J, K);
-  const int sp_own = (tj + 2) * H2K + (tk + 2), sg_own = (tj + 1) * GB<R>::P + (tk + 1);
-  // halo job by ht, the thread index turned by a multiple of 64 that changes from one of an
-  // XCD's workgroups to the next (the jobs of two wavefronts would otherwise fall on the same
-  // two SIMDs of every CU)
-  const int ht = (tid + 64 * ((tile >> 3) & 3)) & (NT - 1);
+  int sp_own = (tj + 2) * H2K + (tk + 2), sg_own = (tj + 1) * GB<R>::P + (tk + 1);
   int hj = 0, hk = 0, halo = 0;
-  box_halo_job(ht, &hj, &hk, &halo);
-  if (halo && !p_ok(J - tj + hj, K - tk + hk)) halo = 0;
-  const bool ring_g = halo == 2 && g_ok(J - tj + hj, K - tk + hk);
-  const unsigned hoff = halo ? (unsigned)(J - tj + hj) * N[2] + (unsigned)kcol(K - tk + hk) : 0;
-  const int hs = (hj + 2) * H2K + (hk + 2);
+  box_halo_job((tid + 64 * ((tile >> 3) & 3)) & (NT - 1), &hj, &hk, &halo);
+  if (halo && !p_ok(ng + j0 + hj, ng + k0 + hk)) halo = 0;
+  const bool halo1 = halo != 0, halo2 = halo == 2, ring_g = halo2 && g_ok(ng + j0 + hj, ng + k0 + hk);
+  const int hjob = (hj + 2) | (hk + 2) << 8;
+  // The thread's indices, in FP32 formed again from its number in each phase: kept through the
+  // march (or hoisted out of it) they took up to 20 registers of the face phases, which spilled,
+  // and a reload waits for every load issued before it (256 x 128 x 128 cells: 308 -> 271 us;
+  // FP64, which has the registers: 423 us as they are, 431 us formed again)
+  auto place = [&]() {
+    tid = threadIdx.x;
+    if constexpr (F32) asm volatile("" : "+v"(tid));
+    tj = (tid >> 6) + 4 * ((tid >> 4) & 3);
+    tk = tid & 15;
+    J = ng + j0 + tj;
+    K = ng + k0 + tk;
+    sp_own = (tj + 2) * H2K + (tk + 2);
+    sg_own = (tj + 1) * GB<R>::P + (tk + 1);
+  };
+  int ht, hs;
+  auto hplace = [&]() {
+    int w = hjob;
+    if constexpr (F32) asm volatile("" : "+v"(w));
+    hj = (w & 255) - 2;
+    hk = (w >> 8) - 2;
+    ht = ((int)threadIdx.x + 64 * ((tile >> 3) & 3)) & (NT - 1);
+    hs = (hj + 2) * H2K + (hk + 2);
+  };
   // metric tables of the tile's rows and columns (index 0: row j0 - 1 / column k0 - 1)
   if (tid < 2 * G2K) {
     const int a = tid < G2K ? 0 : 1, x = tid - a * G2K;
@@ -503,19 +521,22 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
 #pragma unroll
   for (int x = 0; x < 4; ++x) Hx[x] = Hn[x] = R(0);
   auto request = [&](int p) {                    // the states of plane p
-    load_q((unsigned)p * sI + cb, qn);
-    if (halo) load_q((unsigned)p * sI + hoff, hq);
+    // (the own column clamped into the array)
+    load_q((unsigned)p * sI + (unsigned)min(J, N[1] - 1) * N[2] + kcol(min(K, N[2] - 1)), qn);
+    hplace();
+    if (halo1) load_q((unsigned)p * sI + (unsigned)(ng + j0 + hj) * N[2] + (unsigned)kcol(ng + k0 + hk), hq);
   };
   auto arrive = [&]() {                          // their records
     R a[4], b[4];
     rec_of(nd, qn, B.p_ref, B.T_gauge, B.e_ref, a, b);
     mu1 = b[2];
-    if (halo) rec_of(nd, hq, B.p_ref, B.T_gauge, B.e_ref, Hx, Hn);
+    if (halo1) rec_of(nd, hq, B.p_ref, B.T_gauge, B.e_ref, Hx, Hn);
     return cell_of(a, b);
   };
   auto stage_plane = [&](R (*P)[NP2], const BCell<R>& c) {
     if (own_p) stage(P, sp_own, c);
-    if (halo) stage(P, hs, cell_of(Hx, Hn));
+    hplace();
+    if (halo1) stage(P, hs, cell_of(Hx, Hn));
     mu0 = mu1;
     Hr = Hn[0];
     Hm = Hn[2];
@@ -524,7 +545,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
   W0 = W1 = arrive();
   if constexpr (F32) {
     stage_plane(sP[NB - 1], W1);
-  } else if (halo == 2) {
+  } else if (halo2) {
 #pragma unroll
     for (int x = 0; x < 3; ++x) sH0[x][ht] = Hx[x];
   }
@@ -558,6 +579,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     const bool inner = I >= I0 && I < Iend;      // plane owned by the tile: j / k faces
     const bool fin = act && I >= I0 + 1;         // cell I-1 is finished at this plane
     R (*P)[NP2] = sP[buf];
+    place();
     const BCell<R> Pn = arrive();                // own record of I+1
     auto cell = [&](const R (*Q)[NP2], int s) {
       BCell<R> w;
@@ -645,8 +667,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
 #pragma unroll
       for (int v = 0; v < GB<R>::N; ++v) sG[v][sg_own] = G[v];
     }
-    W0 = W1;
-    if (!F32 && own_p) W1 = cell(P, sp_own);
+    if (F32) W0 = W1;
     if (fin) {
       // outward sums in FP64; the FP32-bulk energy gets the gauge terms
       const double ivol = iwi_p * iyz;
@@ -658,7 +679,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       for (int v = 0; v < 5; ++v) r[v] = a[v] * ivol;
       if (nd.n_sponge > 0) {
         const double xcv = ldu(B.xc, c);
-        const long long mrow = (long long)(I - 1 - ng) * n1 + j;
+        const long long mrow = (long long)(I - 1 - ng) * n1 + (J - ng);
         const long long mplane = (long long)n0 * n1;
         for (int sp = 0; sp < nd.n_sponge; ++sp) {
           const double sigma = sponge_sigma(nd.sponge[sp], xcv);
@@ -675,7 +696,9 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     }
     if (I == Iend) break;
     __builtin_amdgcn_sched_barrier(0);
+    place();
     if (inner && ring_g) {
+      hplace();
       R Gr[GB<R>::N], m[4];
 #pragma unroll
       for (int x = 0; x < GB<R>::NV; ++x) {
@@ -704,6 +727,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
         for (int v = 0; v < NF; ++v) sFj[v][tid] = F[v];
       }
       __builtin_amdgcn_sched_barrier(0);
+      place();
       const int rj = own ? tj : tk, rk = own ? tk : kl;   // k face left of (tj, tk) / upper edge of row tk
       if (rj < jl && (own ? rk < kl : true)) {
         R F[6];
@@ -722,6 +746,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       }
     }
     __builtin_amdgcn_sched_barrier(0);
+    place();
     // ---- FP32: plane I+1 staged in the other buffer and the records of I+2 requested before
     //      the exchange barrier, which then covers both
     if (F32) {
@@ -735,6 +760,9 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     __syncthreads();                             // j / k face exchange
     __builtin_amdgcn_s_setprio(0);
     if (!F32) {                                  // FP64: one buffer, free after the exchange barrier
+      W0 = W1;
+      if (own_p) W1 = cell(P, sp_own);
+      hplace();
       if (ring_g) {
 #pragma unroll
         for (int x = 0; x < 3; ++x) sH0[F32 ? 0 : x][F32 ? 0 : ht] = P[1 + x][hs];
