@@ -115,7 +115,8 @@ struct WallOp {
 
 struct InflowDev {
   int n_tab, n_modes;
-  int coop;                 // set by the launcher: phases evaluated cooperatively in LDS
+  int coop;                 // set by the launcher: 1 phases evaluated cooperatively in LDS, 2 with the
+                            // table's y column there too
   const double* table;
   const double* modes;
   double U_inf, L, rho_inf, p_inf;

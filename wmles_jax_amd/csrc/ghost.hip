@@ -148,6 +148,15 @@ __device__ double interp_col(InterpAt at, double x, const double* xp, const doub
 
 // Synthetic inflow ghost fill, reference smooth_ramp.py:150-197.  One workgroup per
 // (ghost layer m, row J); threads over K (full ghosted extent, <= blockDim).
+//
+// A few hundred workgroups: bound by the FP64 cosines (134 x 3 rows of 70 cells, 64 modes: 5.4
+// million, 17 us of issue) and by each row's serial chain.  So a workgroup has 512 threads (two
+// cosine chains to hide each other on every SIMD), the table's y column is searched in LDS (in
+// memory each of its steps was a round trip), and a row mean is taken by eight lanes of every
+// wavefront in the pairwise sum's own order after one barrier (one thread and three barriers
+// before): 41.5 -> 35.8 us; 69 x 3 rows of 39 cells 24.6 -> 19.6 us.  (A cosine of a quarter of the
+// instructions, the modes' coefficients requested first, and a third of the code each left it
+// as it is or slowed it.)
 __global__ void k_inflow(const BlockDev* __restrict__ blks, int blk, InflowDev in, Ptrs q,
                          GasC gas, double time, const double* __restrict__ d_dt, double t_coef) {
   extern __shared__ double red[];
@@ -167,33 +176,36 @@ __global__ void k_inflow(const BlockDev* __restrict__ blks, int blk, InflowDev i
   double z_l = B.xc[2 * cells + ci] / in.L;
   double X0 = in.U_inf * t / in.L;
   const bool inner = valid && K >= ng && K < ng + nk;
-  // the profile columns at y_l, loaded before the mode sums (one search of the y column)
   const double* tb = in.table;
-  const InterpAt at = interp_at(y_l, tb, 7, in.n_tab);
-  double tcol[6];
-  for (int c = 0; c < 6; ++c) tcol[c] = interp_col(at, y_l, tb, tb + 1 + c, 7);
   const int nm = in.n_modes;
   // cos of every (cell, mode) phase, computed by all threads of the workgroup into LDS
   // (when the row fits), then summed per cell in mode order: the same values and the same
   // sum as one thread per cell doing its modes in turn.  Mode-major with an odd pitch, so
   // that lanes of one mode (the sums) or of one cell (the phases) fall in distinct banks.
   const int P2 = N2 | 1;
-  double* cosb = red + blockDim.x + 1;                  // [nm][P2] when cooperative
+  double* cosb = red + 2 * blockDim.x + 1;              // [nm][P2] when cooperative
   double* yz = cosb + (long long)P2 * nm;               // [2][N2]
-  const bool coop = in.coop;
+  double* ys = yz + 2 * N2;                             // [n_tab] the table's y column
+  const bool coop = in.coop, ytab = in.coop == 2;
   if (coop) {
+    for (int i = ytab ? threadIdx.x : in.n_tab; i < in.n_tab; i += blockDim.x) ys[i] = tb[(long long)7 * i];
     for (int kk = threadIdx.x; kk < N2; kk += blockDim.x) {
       const long long cj = cidx(B.N, gi, J, kk);
       yz[kk] = B.xc[cells + cj] / in.L;
       yz[N2 + kk] = B.xc[2 * cells + cj] / in.L;
     }
+    __syncthreads();
   }
+  // the profile columns at y_l, loaded before the mode sums (one search of the y column)
+  const InterpAt at = ytab ? interp_at(y_l, ys, 1, in.n_tab) : interp_at(y_l, tb, 7, in.n_tab);
+  double tcol[6];
+  for (int c = 0; c < 6; ++c) tcol[c] = interp_col(at, y_l, tb, tb + 1 + c, 7);
   double fld[3];
   for (int comp = 0; comp < 3; ++comp) {
     const double* md = in.modes + (long long)comp * 4 * nm;
     double f = 0.0;
     if (coop) {
-      __syncthreads();                                   // yz staged / previous sums done
+      if (comp > 0) __syncthreads();                     // previous sums done
       if ((int)blockDim.x % nm == 0) {
         // every element of this thread has the same mode k: its coefficients (and the
         // time term) are loaded once; the phase keeps its operation order
@@ -226,16 +238,29 @@ __global__ void k_inflow(const BlockDev* __restrict__ blks, int blk, InflowDev i
     }
     fld[comp] = f;
   }
-  if (coop) __syncthreads();                             // the row statistics reuse red[]
-  // row statistics over the interior span, summed in numpy's add.reduce order
+  // row statistics over the interior span, summed in numpy's add.reduce order (the first element
+  // plus the pairwise sum of the rest, whose runs of <= 128 use 8 interleaved accumulators);
+  // two buffers in turn, so that one barrier a mean is enough
+  int turn = 0;
   auto row_mean = [&](double val) {
-    red[K] = inner ? val : 0.0;
+    double* buf = red + (turn ^= 1) * blockDim.x;
+    buf[K] = inner ? val : 0.0;
     __syncthreads();
-    if (K == 0) red[blockDim.x] = np_sum([&](int i) { return red[ng + i]; }, nk) / nk;
-    __syncthreads();
-    double r = red[blockDim.x];
-    __syncthreads();
-    return r;
+    const double* e = buf + ng;
+    const int n = nk - 1;
+    if (n < 8 || n > 128) {                              // short or long rows: one thread
+      double* sum = red + 2 * blockDim.x;
+      if (K == 0) *sum = np_sum([&](int i) { return e[i]; }, nk) / nk;
+      __syncthreads();
+      return *sum;
+    }
+    const int u = K & 7, nfull = n - n % 8;
+    double a = e[1 + u];
+    for (int i = 8; i < nfull; i += 8) a = a + e[1 + i + u];
+#pragma unroll
+    for (int m = 1; m <= 4; m <<= 1) a = a + __shfl_xor(a, m, 8);
+    for (int i = nfull; i < n; ++i) a = a + e[1 + i];
+    return (e[0] + a) / nk;
   };
   double mean0 = row_mean(fld[0]);
   fld[0] = fld[0] - mean0;
@@ -293,9 +318,14 @@ hipError_t launch_inflow(const BlockDev* d_blks, int blk, int N1, int N2, int ng
   dim3 grid(N1, ng);
   // cooperative phase evaluation when a row's (cell, mode) table fits in 56 KB of LDS
   const size_t coop_bytes = sizeof(double) * ((size_t)(N2 | 1) * in.n_modes + 2 * (size_t)N2);
+  const size_t tab_bytes = sizeof(double) * (size_t)in.n_tab, lds = 64 * 1024;
   in.coop = coop_bytes <= 56 * 1024 ? 1 : 0;
-  if (in.coop && threads < 256) threads = 256;           // more lanes for the phase table
-  size_t shm = sizeof(double) * (threads + 1) + (in.coop ? coop_bytes : 0);
+  auto shm_of = [&](int th, size_t extra) { return sizeof(double) * (2 * (size_t)th + 1) + extra; };
+  // more lanes for the phase table, and the table's y column, where the 64 KB hold them
+  if (in.coop && threads < 256) threads = 256;
+  if (in.coop && threads < 512 && shm_of(512, coop_bytes) <= lds) threads = 512;
+  if (in.coop && shm_of(threads, coop_bytes + tab_bytes) <= lds) in.coop = 2;
+  size_t shm = shm_of(threads, in.coop ? coop_bytes + (in.coop == 2 ? tab_bytes : 0) : 0);
   hipLaunchKernelGGL(k_inflow, grid, dim3(threads), shm, s, d_blks, blk, in, q, gas, time, d_dt,
                      coef);
   return hipGetLastError();
