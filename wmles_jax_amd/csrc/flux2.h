@@ -96,7 +96,7 @@ template <int ORDER>
 __device__ __forceinline__ void kep_pairs_f32(const CellWT<float>& L2, const CellWT<float>& L,
                                               const CellWT<float>& Rc, const CellWT<float>& R2, float Sx,
                                               float Sy, float Sz, float* F, float* un4) {
-  auto ek = [](const CellWT<float>& c) { return c.e + 0.5f * ((c.u * c.u + c.v * c.v) + c.w * c.w); };
+  auto ek = [](const CellWT<float>& c) { return __builtin_fmaf(0.5f, __builtin_fmaf(c.w, c.w, __builtin_fmaf(c.v, c.v, c.u * c.u)), c.e); };
   const float EL = ek(L), ER = ek(Rc);
   auto pair = [&](const CellWT<float>& a, const CellWT<float>& b, float Ea, float Eb, float* A, float* w) {
     const float sr = a.r + b.r, su = a.u + b.u, sv = a.v + b.v, sw = a.w + b.w;
@@ -104,11 +104,12 @@ __device__ __forceinline__ void kep_pairs_f32(const CellWT<float>& L2, const Cel
     const float ww = (su * Sx + sv * Sy) + sw * Sz;
     const float M = sr * ww, sp4 = 4.f * sp;
     A[0] = M;
-    A[1] = M * su + sp4 * Sx;
-    A[2] = M * sv + sp4 * Sy;
-    A[3] = M * sw + sp4 * Sz;
-    A[4] = M * sE + (2.f * sp) * ww;
+    A[1] = __builtin_fmaf(sp4, Sx, M * su);
+    A[2] = __builtin_fmaf(sp4, Sy, M * sv);
+    A[3] = __builtin_fmaf(sp4, Sz, M * sw);
+    A[4] = __builtin_fmaf(2.f * sp, ww, M * sE);
     *w = ww;
+    return sr;
   };
   float A[5], w;
   pair(L, Rc, EL, ER, A, &w);
@@ -120,9 +121,9 @@ __device__ __forceinline__ void kep_pairs_f32(const CellWT<float>& L2, const Cel
     return;
   }
   float Aa[5], wa, Ab[5], wb;
-  pair(L, R2, EL, ek(R2), Aa, &wa);
+  const float sra = pair(L, R2, EL, ek(R2), Aa, &wa);
   pair(L2, Rc, ek(L2), ER, Ab, &wb);
-  F[0] = (8.f * A[0] - (Aa[0] + Ab[0])) * (1.f / 24.f);
+  F[0] = (8.f * A[0] - __builtin_fmaf(sra, wa, Ab[0])) * (1.f / 24.f);
 #pragma unroll
   for (int c = 1; c < 5; ++c) F[c] = (8.f * A[c] - (Aa[c] + Ab[c])) * (1.f / 48.f);
   *un4 = (8.f * w - (wa + wb)) * (1.f / 12.f);

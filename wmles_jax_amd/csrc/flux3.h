@@ -9,21 +9,22 @@
 //   1. stages (u, v, w, T') of plane I+1 (three rolling slots hold planes I-1, I, I+1),
 //      (rho, p', mu, e') and the centroids of plane I, own columns from registers loaded
 //      one plane ahead, the halo ring from loads issued during the previous plane;
-//   2. evaluates the gradient records of plane I on the tile + 1-cell ring (306 cells; at
-//      the chunk's two end planes, which feed only the i faces, the 240 own cells);
-//   3. evaluates the j / k faces of plane I (exchanged through LDS) and the i face I-1/2 of
-//      the own column (registers);
-//   4. finishes cell I-1: its i faces I-3/2 and I-1/2 (registers) and its j / k faces,
-//      kept from the previous plane in the other half of the double-buffered exchange.
-// The march runs over planes I0-1 .. I0+len, one plane more at each end than the tile's
-// cells.  Three barriers per plane (staging, gradients, face exchange; the last is skipped
-// at the end planes, which have no j / k faces).
+//   2. evaluates the gradient record of the own column's cell (rows 0..15; the ring's other 50
+//      cells are a second pass of one wavefront) and with it the own i face I-1/2 (registers),
+//      which finishes cell I-1: its i faces I-3/2 and I-1/2 and its j / k faces, kept from the
+//      previous plane;
+//   3. evaluates the j / k faces of plane I, exchanged through LDS.
+// The march runs over planes I0-1 .. I0+len, one plane more at each end than the tile's cells.
+// Three barriers per plane (staging, gradients, face exchange; the end planes, which have no
+// j / k faces, need the first alone).  The i face and the epilogue stand before the gradient
+// barrier: they need no other thread's record, and the wavefronts without a second pass have
+// them to do (512 x 128 x 64-cell ramp: 485 us per launch with both after it, 450 us).
 //
 // Wavefront priorities (s_setprio) by phase: two workgroups share each CU, one wavefront of
 // each per SIMD, and the launch is bound by latency at the barriers, not by issue.  A
 // wavefront in its gradient phase issues first (its workgroup's next barrier waits for the
 // slowest wavefront's gradient cells, whose geometry loads carry a memory round trip), then
-// one in its face tasks; the epilogue and the staging run at the base priority.
+// one in its face tasks; the staging runs at the base priority.
 #pragma once
 #include "flux2.h"
 
@@ -150,7 +151,7 @@ __device__ __forceinline__ void flux3_tile(const BlockDev* __restrict__ blks, co
   __shared__ float sPr[4][NP2];                  // (rho, p', mu, e') of the current plane
   __shared__ float sG[NGW][NG2S];                // gradient records of the current plane
   __shared__ double sX[3][NG2S];                 // centroids of the current plane
-  __shared__ float sS[3][3][NG2S];               // lower i / j / k face vectors of the gradient cells
+  __shared__ float sS[2][3][NG2S];               // lower j / k face vectors of the gradient cells
   __shared__ float sFj[NFX][NT];                 // slot tile_tid(r, c)
   __shared__ float sFk[NFX][NT + C2J + 1];       // slot kface_slot(r, c)
   const int4 t = tiles[tile];
@@ -280,38 +281,26 @@ __device__ __forceinline__ void flux3_tile(const BlockDev* __restrict__ blks, co
     }
     __syncthreads();
     __builtin_amdgcn_s_setprio(PRIO_GRAD);
-    // ---- gradient records of plane I: the tile + ring (306 cells) at owned planes, the own
-    //      cells at the two end planes
-    {
-      int rr[2] = {-1, -1};
-      if (inner) {
-        rr[0] = tid;
-        rr[1] = tid + NT < NG2 ? tid + NT : -1;
-      } else if (own) {
-        rr[0] = (tj + 1) * G2K + (tk + 1);
-      }
+    // ---- gradient records of plane I: the own column's here, the 50 ring cells' below
+    float G[NGW], Slo[9];
+    auto gradient = [&](int gj, int gk, float* Gv, float* Sv) {
+      grad_cell3(B, nd, sPh[s_m], sPh[s_0], sPh[s_p], sPr, (gj + 1) * H2K + (gk + 1), I, ng + j0 - 1 + gj, ng + k0 - 1 + gk,
+                 Gv, Sv);
+    };
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int r = rr[u];
-        if (r < 0) continue;
-        const int gj = r / G2K, gk = r - gj * G2K;
-        const int JJ = ng + j0 - 1 + gj, KK = ng + k0 - 1 + gk;
-        if (!g_ok(JJ, KK)) continue;
-        float Gv[NGW], Slo[9];
-        grad_cell3(B, nd, sPh[s_m], sPh[s_0], sPh[s_p], sPr, (gj + 1) * H2K + (gk + 1), I, JJ, KK, Gv, Slo);
-        const int gsl = gj * G2P + gk;
+    for (int v = 0; v < NGW; ++v) G[v] = 0.f;
 #pragma unroll
-        for (int v = 0; v < NGW; ++v) sG[v][gsl] = Gv[v];
+    for (int v = 0; v < 9; ++v) Slo[v] = 0.f;
+    const bool own_gi = g_ok(J, K) && (own || inner);
+    if (own_gi) gradient(tj + 1, tk + 1, G, Slo);
+    // (rounded here: the i face must not contract the record's last products, which the ring's
+    // and the neighbours' copies hold rounded)
 #pragma unroll
-        for (int v = 0; v < 9; ++v) sS[v / 3][v % 3][gsl] = Slo[v];
-      }
-    }
+    for (int v = 0; v < NGW; ++v) asm volatile("" : "+v"(G[v]));
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(PRIO_FACE);
-    __syncthreads();
-    // ---- face fluxes: 0 j face below row tj, 1 k face left of column tk (or the upper
-    //      edge k face of row tk), 2 the own i face I-1/2
-    // ---- cell I-1: its state and volume loads go out before the face tasks, whose
-    //      arithmetic covers their latency
+    // ---- cell I-1: its state and volume loads go out before the i face, whose arithmetic
+    //      covers their latency
     const bool fin = act && I >= I0 + 1;
     const unsigned c = (unsigned)(I - 1) * sI + (unsigned)J * N[2] + K;
     const double* qi = qin.p[t.x];
@@ -321,104 +310,56 @@ __device__ __forceinline__ void flux3_tile(const BlockDev* __restrict__ blks, co
 #pragma unroll
       for (int v = 0; v < 5; ++v) vq[v] = ldu(qi + v * cells, c);
     }
-    float Fin[NFX] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int task = inner ? 0 : 2; task < (I >= I0 ? 3 : 0); ++task) {
-      bool doit = act;
-      int d = 0, fI = I, fJ = J, fK = K;
-      int rj = tj, rk = tk;
-      CellWT<float> L2, L, Rc, R2;
-      CellGT<float> gL, gR;
-      float thL, thR, TL, TR;
-      float dx[3] = {0.f, 0.f, 0.f};           // centroid difference, FP64 then rounded
-      if (task == 2) {
-        L2 = rec_w(Pw[0]); L = rec_w(Pw[1]); Rc = rec_w(Pw[2]); R2 = rec_w(Pw[3]);
-        TL = Pw[1].T; TR = Pw[2].T;
+    // flux through a face of direction d with lower cell index f along it, or its wall model's
+    auto face = [&](int d, int fI, int fJ, int fK, const CellWT<float>& L2, const CellWT<float>& L,
+                    const CellWT<float>& Rc, const CellWT<float>& R2, float thL, float thR, const CellGT<float>& gL,
+                    const CellGT<float>& gR, float TL, float TR, const float* dx, const float* S, float* F) {
+      const int cf = d == 0 ? fI : (d == 1 ? fJ : fK);
+      int side = -1;
+      if (cf == ng) side = 0;
+      else if (cf == ng + B.n[d]) side = 1;
+      if (side >= 0 && B.faces[2 * d + side].kind == WMX_BC_WALLMODEL) {
+        int t1, t2;
+        tangents(d, &t1, &t2);
+        const int cc[3] = {fI, fJ, fK};
+        const unsigned nw = (unsigned)B.n[t1] * B.n[t2];
+        const unsigned w = (unsigned)(cc[t1] - ng) * B.n[t2] + (cc[t2] - ng);
+        const double* W = B.wall[2 * d + side];   // gauge form (p - p_ref) S, no mass flux
 #pragma unroll
-        for (int i = 0; i < 12; ++i) gL.g[i] = Gp[i];
-        gL.mu = Gp[12]; gL.k = Gp[13]; thL = Gp[14];
-        gR = sg_g<float>(sG, sg_own); thR = sG[14][sg_own];
-#pragma unroll
-        for (int x = 0; x < 3; ++x) dx[x] = float(sX[x][sg_own] - Xp[x]);
+        for (int v = 0; v < 5; ++v) F[v] = (float)ldu(W + v * nw, w);
+        F[5] = 0.f;
       } else {
-        if (task == 0) {
-          d = 1;
-          doit = rj <= jl && rk < kl;
-        } else if (own) {
-          d = 2;
-          doit = rj < jl && rk < kl;
-        } else {
-          d = 2;
-          rj = tk; rk = kl;
-          doit = rj < jl;
-        }
-        fJ = ng + j0 + rj;
-        fK = ng + k0 + rk;
-        const int dj = d == 1, dk = d == 2;
-        const int pR = (rj + 2) * H2K + (rk + 2), gR_ = (rj + 1) * G2P + (rk + 1);
-        const int pst = dj * H2K + dk, gst = dj * G2P + dk;
-        if (doit) {
-          auto cw = [&](int s) {
-            CellWT<float> w;
-            w.r = sPr[0][s]; w.u = sPh[s_0][0][s]; w.v = sPh[s_0][1][s]; w.w = sPh[s_0][2][s];
-            w.p = sPr[1][s]; w.e = sPr[3][s];
-            return w;
-          };
-          L2 = cw(pR - 2 * pst); L = cw(pR - pst); Rc = cw(pR); R2 = cw(pR + pst);
-          TL = sPh[s_0][3][pR - pst]; TR = sPh[s_0][3][pR];
-          gL = sg_g<float>(sG, gR_ - gst); gR = sg_g<float>(sG, gR_);
-          thL = sG[14][gR_ - gst]; thR = sG[14][gR_];
-#pragma unroll
-          for (int x = 0; x < 3; ++x) dx[x] = float(sX[x][gR_] - sX[x][gR_ - gst]);
-        }
+        flux_core_f32<SC>(nd, L2, L, Rc, R2, thL, thR, gL, gR, TL, TR, dx[0], dx[1], dx[2], S[0], S[1], S[2],
+                          float(B.p_ref), float(B.e_ref), F, &F[5]);
       }
-      float F[NFX] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (doit) {
-        const int cf = d == 0 ? fI : (d == 1 ? fJ : fK);
-        int side = -1;
-        if (cf == ng) side = 0;
-        else if (cf == ng + B.n[d]) side = 1;
-        if (side >= 0 && B.faces[2 * d + side].kind == WMX_BC_WALLMODEL) {
-          int t1, t2;
-          tangents(d, &t1, &t2);
-          const int cc[3] = {fI, fJ, fK};
-          const unsigned nw = (unsigned)B.n[t1] * B.n[t2];
-          const unsigned w = (unsigned)(cc[t1] - ng) * B.n[t2] + (cc[t2] - ng);
-          const double* W = B.wall[2 * d + side];   // gauge form (p - p_ref) S, no mass flux
+    };
+    // ---- the own i face I-1/2
+    float Fin[NFX] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (act && I >= I0) {
+      CellGT<float> gL, gR;
 #pragma unroll
-          for (int v = 0; v < 5; ++v) F[v] = (float)ldu(W + v * nw, w);
-        } else {
-          // the face vector, staged by the gradient cell whose lower face it is
-          const int ss = task == 2 ? sg_own : (rj + 1) * G2P + (rk + 1);
-          flux_core_f32<SC>(nd, L2, L, Rc, R2, thL, thR, gL, gR, TL, TR, dx[0], dx[1], dx[2], sS[d][0][ss], sS[d][1][ss],
-                            sS[d][2][ss], float(B.p_ref), float(B.e_ref), F, &F[5]);
-        }
-        if (task == 2) {
-#pragma unroll
-          for (int v = 0; v < NFX; ++v) Fin[v] = F[v];
-        } else if (d == 1) {
-#pragma unroll
-          for (int v = 0; v < NFX; ++v) sFj[v][tile_tid(rj, rk)] = F[v];
-        } else {
-#pragma unroll
-          for (int v = 0; v < NFX; ++v) sFk[v][kface_slot(rj, rk)] = F[v];
-        }
+      for (int i = 0; i < 12; ++i) {
+        gL.g[i] = Gp[i];
+        gR.g[i] = G[i];
       }
-    }
-    // ---- prefetch for plane I+1 (own record of I+2, own centroid of I+1, the ring), issued
-    //      before the exchange barrier so that the epilogue and the barrier cover its
-    //      latency (this plane's staging consumed the registers it overwrites)
-    if (I < Iend) {
-      Pn = load_rec32(P, cells, (size_t)(I + 2) * sI + cb);
+      gL.mu = Gp[12]; gL.k = Gp[13];
+      gR.mu = G[12]; gR.k = G[13];
+      float dx[3];                               // centroid difference, FP64 then rounded
 #pragma unroll
-      for (int x = 0; x < 3; ++x) Xn[x] = ldu(XC + x * (size_t)cells, (unsigned)(I + 1) * sI + cb);
-      ring_load(I + 2, I + 1);
+      for (int x = 0; x < 3; ++x) dx[x] = float(sX[x][sg_own] - Xp[x]);
+      face(0, I, J, K, rec_w(Pw[0]), rec_w(Pw[1]), rec_w(Pw[2]), rec_w(Pw[3]), Gp[14], G[14], gL, gR, Pw[1].T, Pw[2].T, dx,
+           Slo, Fin);
     }
-    if (inner) __syncthreads();                  // (uniform) j / k face exchange
-    __builtin_amdgcn_s_setprio(PRIO_REST);
+    if (own_gi && inner) {
+#pragma unroll
+      for (int v = 0; v < NGW; ++v) sG[v][sg_own] = G[v];
+#pragma unroll
+      for (int v = 0; v < 6; ++v) sS[v / 3][v % 3][sg_own] = Slo[3 + v];
+    }
+#pragma unroll
+    for (int v = 0; v < NGW; ++v) Gp[v] = G[v];
+    __builtin_amdgcn_sched_barrier(0);
     if (fin) {
-      // stages 2 and 3: the base-state loads go out first, so the sums below overlap their
-      // latency (before the barrier their registers would spill)
       if (MODE >= 2) {
         const double* qz = q0.p[t.x];
 #pragma unroll
@@ -463,6 +404,77 @@ __device__ __forceinline__ void flux3_tile(const BlockDev* __restrict__ blks, co
         for (int v = 0; v < 5; ++v) stu(o + v * cells, c, a0 * vz[v] + a1 * (vq[v] + dt * r[v]));
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    if (inner) {
+      // ring cells (row 0, columns 0 and 17) as a second pass of one wavefront: which one changes
+      // from one of an XCD's workgroups to the next, so that no SIMD gets all of them
+      const int g = (tid + 64 * ((tile >> 3) & 3)) & (NT - 1);
+      if (g < G2K + 2 * TK) {
+        const int gj = g < G2K ? 0 : 1 + ((g - G2K) & 15), gk = g < G2K ? g : (g < G2K + TK ? 0 : G2K - 1);
+        if (g_ok(ng + j0 - 1 + gj, ng + k0 - 1 + gk)) {
+          float Gv[NGW], Sv[9];
+          gradient(gj, gk, Gv, Sv);
+          const int gsl = gj * G2P + gk;
+#pragma unroll
+          for (int v = 0; v < NGW; ++v) sG[v][gsl] = Gv[v];
+#pragma unroll
+          for (int v = 0; v < 6; ++v) sS[v / 3][v % 3][gsl] = Sv[3 + v];
+        }
+      }
+      __syncthreads();
+      // ---- j face below row tj, k face left of column tk (or the upper edge k face of row tk)
+#pragma unroll 1
+      for (int task = 0; task < 2; ++task) {
+        int rj = tj, rk = tk;
+        bool doit;
+        const int d = 1 + task;
+        if (task == 0) {
+          doit = rj <= jl && rk < kl;
+        } else if (own) {
+          doit = rj < jl && rk < kl;
+        } else {
+          rj = tk; rk = kl;
+          doit = rj < jl;
+        }
+        if (doit) {
+          const int pR = (rj + 2) * H2K + (rk + 2), gR_ = (rj + 1) * G2P + (rk + 1);
+          const int pst = task == 0 ? H2K : 1, gst = task == 0 ? G2P : 1;
+          auto cw = [&](int q) {
+            CellWT<float> w;
+            w.r = sPr[0][q]; w.u = sPh[s_0][0][q]; w.v = sPh[s_0][1][q]; w.w = sPh[s_0][2][q];
+            w.p = sPr[1][q]; w.e = sPr[3][q];
+            return w;
+          };
+          float dx[3], S[3], F[NFX];
+#pragma unroll
+          for (int x = 0; x < 3; ++x) {
+            dx[x] = float(sX[x][gR_] - sX[x][gR_ - gst]);
+            S[x] = sS[task][x][gR_];             // staged by the gradient cell whose lower face it is
+          }
+          face(d, I, ng + j0 + rj, ng + k0 + rk, cw(pR - 2 * pst), cw(pR - pst), cw(pR), cw(pR + pst), sG[14][gR_ - gst],
+               sG[14][gR_], sg_g<float>(sG, gR_ - gst), sg_g<float>(sG, gR_), sPh[s_0][3][pR - pst], sPh[s_0][3][pR], dx, S,
+               F);
+          if (task == 0) {
+#pragma unroll
+            for (int v = 0; v < NFX; ++v) sFj[v][tile_tid(rj, rk)] = F[v];
+          } else {
+#pragma unroll
+            for (int v = 0; v < NFX; ++v) sFk[v][kface_slot(rj, rk)] = F[v];
+          }
+        }
+      }
+    }
+    // ---- prefetch for plane I+1 (own record of I+2, own centroid of I+1, the ring), issued
+    //      before the exchange barrier so that the epilogue and the barrier cover its
+    //      latency (this plane's staging consumed the registers it overwrites)
+    if (I < Iend) {
+      Pn = load_rec32(P, cells, (size_t)(I + 2) * sI + cb);
+#pragma unroll
+      for (int x = 0; x < 3; ++x) Xn[x] = ldu(XC + x * (size_t)cells, (unsigned)(I + 1) * sI + cb);
+      ring_load(I + 2, I + 1);
+    }
+    if (inner) __syncthreads();                  // (uniform) j / k face exchange
+    __builtin_amdgcn_s_setprio(PRIO_REST);
     // ---- carry: the partial sum (lower i face minus the j / k faces of this plane's
     //      exchange), gradient record and centroid of the own cell I
     if (act && inner) {
@@ -473,8 +485,6 @@ __device__ __forceinline__ void flux3_tile(const BlockDev* __restrict__ blks, co
                                   ((double)sFk[v][kup] - (double)sFk[v][tid]));
     }
     if (own_g) {
-#pragma unroll
-      for (int v = 0; v < NGW; ++v) Gp[v] = sG[v][sg_own];
 #pragma unroll
       for (int x = 0; x < 3; ++x) Xp[x] = sX[x][sg_own];
     }

@@ -147,6 +147,14 @@ WMX_HD R fsqrt(R a) {
 #endif
 }
 
+// a b + c rounded once, where a sum of two products has its multiply-add written out: either
+// product could go into it, and every copy of a face flux has to round the same way
+template <class R>
+WMX_HD R ffma(R a, R b, R c) {
+  if constexpr (sizeof(R) == 4) return __builtin_fmaf(a, b, c);
+  else return __builtin_fma(a, b, c);
+}
+
 // Primitive record of one cell as the face kernels read it: rho, u, v, w, p, e_int.
 template <class R>
 struct CellWT {
@@ -253,8 +261,10 @@ WMX_HD void hllc_flux(R gamma, const R* wl, const R* wr, R Sx, R Sy, R Sz, R* F)
   R ss = fdiv<R>(((pr - pl) + (rl * unl) * (sL - unl)) - (rr * unr) * (sR - unr),
                  rl * (sL - unl) - rr * (sR - unr));
   const R gm1 = gamma - R(1.0), h = R(0.5);
-  R El = fdiv<R>(pl, gm1) + (h * rl) * ((ul * ul + vl * vl) + zl * zl);
-  R Er = fdiv<R>(pr, gm1) + (h * rr) * ((ur * ur + vr * vr) + zr * zr);
+  // (FP32: the quotients' products go into the multiply-adds)
+  auto div_add = [](R a, R b, R c) { return sizeof(R) == 4 ? ffma<R>(a, fdiv<R>(R(1), b), c) : fdiv<R>(a, b) + c; };
+  R El = div_add(pl, gm1, (h * rl) * (ffma<R>(ul, ul, vl * vl) + zl * zl));
+  R Er = div_add(pr, gm1, (h * rr) * (ffma<R>(ur, ur, vr * vr) + zr * zr));
   R r, u, v, z, p, un, E, s;
   int branch;  // 0: FL, 1: F*L, 2: F*R, 3: FR
   if (sL >= R(0)) branch = 0;
@@ -267,7 +277,7 @@ WMX_HD void hllc_flux(R gamma, const R* wl, const R* wr, R Sx, R Sy, R Sz, R* F)
   R Fp[5] = {m, m * u + p * nx, m * v + p * ny, m * z + p * nz, (E + p) * un};
   if (branch == 1 || branch == 2) {
     R f = fdiv<R>(r * (s - un), s - ss);
-    R e = fdiv<R>(E, r) + (ss - un) * (ss + fdiv<R>(p, r * (s - un)));
+    R e = div_add(E, r, (ss - un) * div_add(p, r * (s - un), ss));
     R d = ss - un;
     R st[5] = {f, f * (u + d * nx), f * (v + d * ny), f * (z + d * nz), f * e};
     R U[5] = {r, r * u, r * v, r * z, E};
@@ -348,7 +358,7 @@ WMX_HD void viscous_face_e(const CellGT<R>& a, const CellGT<R>& b, const R* phiL
   F[1] = F[1] + (-ts0);
   F[2] = F[2] + (-ts1);
   F[3] = F[3] + (-ts2);
-  F[4] = F[4] + ((-((uf0 * ts0 + uf1 * ts1) + uf2 * ts2)) - kf * dTdn);
+  F[4] = F[4] + ((-(ffma<R>(uf0, ts0, uf1 * ts1) + uf2 * ts2)) - kf * dTdn);
 }
 
 WMX_HD void viscous_face(const CellG& a, const CellG& b, const double* phiL, const double* phiR,
