@@ -18,7 +18,7 @@
 // Three barriers per plane (staging, gradients, face exchange; the end planes, which have no
 // j / k faces, need the first alone).  The i face and the epilogue stand before the gradient
 // barrier: they need no other thread's record, and the wavefronts without a second pass have
-// them to do (512 x 128 x 64-cell ramp: 485 us per launch with both after it, 450 us).
+// them to do (512 x 128 x 64-cell ramp: 485 us per launch with both after it, 450 us before it).
 //
 // Wavefront priorities (s_setprio) by phase: two workgroups share each CU, one wavefront of
 // each per SIMD, and the launch is bound by latency at the barriers, not by issue.  A
@@ -422,9 +422,12 @@ __device__ __forceinline__ void flux3_tile(const BlockDev* __restrict__ blks, co
         }
       }
       __syncthreads();
-      // ---- j face below row tj, k face left of column tk (or the upper edge k face of row tk)
-#pragma unroll 1
+      // ---- j face below row tj, k face left of column tk (or the upper edge k face of row tk),
+      //      a copy of the face flux each (one copy with the strides chosen at run time: 450 us,
+      //      so 440 us)
+#pragma unroll
       for (int task = 0; task < 2; ++task) {
+        __builtin_amdgcn_sched_barrier(0);
         int rj = tj, rk = tk;
         bool doit;
         const int d = 1 + task;
