@@ -10,7 +10,7 @@ MUSCL-HLLC) with the Ducros switch, Vreman SGS, isothermal equilibrium wall mode
 both walls, periodic x / z, constant mass flux, CFL 0.8, seeded synthetic initial state
 (bulk profile + 5% Gaussian velocity noise).  A step is the reference's driver step:
 max_dt + advance (3 RHS + 3 stage updates + constraint), dt kept on the device, run as
-Solver.step (the CFL min is taken in the first stage's primitive pass, the same value
+Solver.step (the CFL min is taken in the first stage's launches, the same value
 as max_dt; eager launches, --graph replays captured hipGraphs instead).  The
 timed region holds exactly K steps bracketed by device synchronisations.  Both
 arithmetic forms run; the FP32-bulk form is the headline value, the FP64 form and the
@@ -48,7 +48,9 @@ HBM_PEAK_GBS = 8000.0                      # MI355X HBM3E, datasheet
 # Geometry per stage: FP64 plain form 3 owned face vectors (9 words) + xc (3) + vol (1)
 # = 104 B; FP32-bulk form float face vectors (36 B) + FP64 xc (24 B) + FP64 vol (8 B)
 # = 68 B.  The fused flux kernel moves one third per launch.
+# Blocks whose metrics are tensor products (the channels and the ensemble) read no geometry per cell.
 B_ALG_STEP = {"fp64": 320.0 + 3 * 104.0, "fp32": 320.0 + 3 * 68.0}   # 632 / 524 B
+B_ALG_BOX = 320.0
 
 
 def make_case(nx, ny, nz, ns):
@@ -177,9 +179,9 @@ def form_errors(r64, r32):
             "q_w": float(abs(qw(st32) - qw(st64)) / abs(qw(st64)))}
 
 
-FLUX_KERNEL = {True: "k_flux3 (gradient records in the march + face fluxes + divergence + RK stage)",
+FLUX_KERNEL = {True: "k_box, curvilinear blocks k_flux3 (gradients in the march + face fluxes + divergence + RK stage)",
                False: "k_flux2 (face fluxes + divergence + RK stage; gradient records from k_grad32)",
-               None: "k_flux1 (FP64: face fluxes + divergence + RK stage)"}
+               None: "k_box, curvilinear blocks k_curv (FP64: gradients in the march + face fluxes + divergence + RK stage)"}
 
 
 _COPY_PEAK = []
@@ -259,18 +261,18 @@ def bench_channel(args, wmx):
     el = r["elapsed"]
     value = cells * args.steps / el / 1e6
     flux_ms, flux_n = r["prof"]["flux"]
-    b_launch = B_ALG_STEP[head] / 3.0 * cells
+    b_launch = B_ALG_BOX / 3.0 * cells
     workload = f"channel {nx}x{ny}x{nz} Hybrid(KEP4+MUSCL-HLLC) Vreman WM {head}"
     rec = _record(args, value, el * 1e3 / args.steps, "f32-bulk+f64" if head == "fp32" else "f64",
                   workload, {"cells": cells, "blocks": 1, "ng": 3,
                              "step": "Solver.step = max_dt + advance (SSP-RK3, 3 RHS, mass-flux "
-                                     "constraint; the CFL min taken in the first stage's primitive pass)",
+                                     "constraint; the CFL min taken in the first stage's launches)",
                              "graph": bool(args.graph),
                              "form": head,
                              "fused_gradients": r["solver"]._fused if head == "fp32" else None},
-                  _roofline(flux_ms / flux_n / 1e3, b_launch, workload, B_ALG_STEP[head],
+                  _roofline(flux_ms / flux_n / 1e3, b_launch, workload, B_ALG_BOX,
                             r["solver"]._fused if head == "fp32" else None))
-    rec["step_hbm_frac"] = round(B_ALG_STEP[head] * cells / (el / args.steps) / 1e9 / HBM_PEAK_GBS, 4)
+    rec["step_hbm_frac"] = round(B_ALG_BOX * cells / (el / args.steps) / 1e9 / HBM_PEAK_GBS, 4)
     ci, order, ntiles = r["solver"].tiling()
     rec["config"]["tiling"] = {"ci_len": ci, "xcd_order": order, "tiles": ntiles}
     if "fp64" in res and "fp32" in res:
@@ -374,8 +376,8 @@ def bench_ensemble(args, wmx):
     rec = _record(args, cells * args.steps / el_e / 1e6, el_e * 1e3 / args.steps, "f32-bulk+f64", workload,
                   {"cells": cells, "cases": 16, "blocks": nblk, "form": "fp32",
                    "tiling": {"ci_len": best[0], "xcd_order": best[1]}},
-                  _roofline(flux_ms / flux_n / 1e3, B_ALG_STEP["fp32"] / 3.0 * cells, workload,
-                            B_ALG_STEP["fp32"]))
+                  _roofline(flux_ms / flux_n / 1e3, B_ALG_BOX / 3.0 * cells, workload,
+                            B_ALG_BOX))
     rec["state_finite"] = all(bool(torch.isfinite(q).all()) for Q in Qe for q in Q)
     rec["autotune_flux_ms"] = {k: round(v, 4) for k, v in timings.items()}
     if args.ens_forms == "eager":
@@ -478,8 +480,8 @@ def bench_wm(args, wmx):
                   {"cells": cells, "blocks": 1, "form": "fp32", "wall_faces": n_faces,
                    "network": "3-64-64-2 ISRU, BF16 MFMA inference, 3 Newton polish steps",
                    "n_match": n_match},
-                  _roofline(flux_ms / flux_n / 1e3, B_ALG_STEP["fp32"] / 3.0 * cells, workload,
-                            B_ALG_STEP["fp32"]))
+                  _roofline(flux_ms / flux_n / 1e3, B_ALG_BOX / 3.0 * cells, workload,
+                            B_ALG_BOX))
     # FP32-bulk plans evaluate the Newton faces in another launch's head (no launch of
     # their own); the learned model keeps its wall launch.  Both step times are reported.
     per = lambda pr: round(pr["wall"][0] / pr["wall"][1], 5) if "wall" in pr else None

@@ -23,8 +23,8 @@
 // of a halo cell one plane ahead (rec_of), so no primitive launch writes 32 / 64 B per cell for
 // this one to read back with a halo.  Channel of 256 x 128 x 128 cells, Hybrid + Vreman, per
 // stage: FP32 271 us against 253 us on records and 78 us that wrote them; FP64 423 us against
-// 461 us + 137 us.  It is bound by vector issue (about 200 us of the FP32 launch) and by the
-// state loads' latency at three (FP64: two) waves per SIMD.
+// 461 us + 137 us.  It is bound by vector issue (86% of the
+// FP32 launch's cycles, 67% of the lanes active: the Hybrid's upwind branch).
 //
 // March.  At plane I the tile evaluates the gradient records of plane I, the own i face I-1/2,
 // which completes cell I-1, and then the j / k faces of plane I.  The records of planes I-1 and

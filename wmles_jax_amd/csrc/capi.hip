@@ -382,16 +382,18 @@ int auto_ci_len(int nb, const int* dims, int prec, int cu_count, long long* ntil
 // FP32-bulk plan of box blocks that evaluates its gradients in the march (box.h).
 bool direct(const wmx_plan* p) { return p->nd.prec != WMX_PREC_FP32_BULK || (p->box && p->fuse_grad); }
 
-// i-planes per tile of the box kernels when none is requested.  W workgroups share a CU (3 in
+// i-planes per tile of the kernels that read the state when none is requested.  W workgroups share a CU (3 in
 // FP32, 2 in FP64), so T tiles are r full rounds of W CUs slots and a remainder.  A full round
-// of ci planes takes ci + 1 units (11.3 us FP32, 12.1 us FP64); a remainder that puts at most k
+// of ci planes takes ci + 1 units (9.8 us FP32, 11.1 us FP64); a remainder that puts at most k
 // workgroups on a CU takes t(k) of one: 0.55 / 0.78 / 1 (FP32), 0.6 / 1 (FP64).  Fitted to the
 // 256 x 128 x 128-cell, 128 x 96 x 96-cell and ensemble launches at ci of 2..64 (within 13%).
 // Short chunks are allowed down to one plane: below one workgroup per CU a launch is the
 // serial march of one tile (24 x 16 x 12 cells, FP64: 29.4 us at four planes, 15.0 us at one).
 // The shortest estimate over ci in [1, 64] wins, ties to the shorter chunk, whose tiles leave
-// and refill the slots more often (256 planes, FP32: 8 per tile, three full rounds, 307 us; 26
-// per tile, one round, 319 us; 24 per tile, one round and 24 tiles, 422 us).
+// and refill the slots more often (256 planes, FP32: 8 per tile, three full rounds, 265 us; 26
+// per tile, one round, 278 us; 24 per tile, one round and 24 tiles, 372 us).  The curvilinear
+// FP64 kernel takes the same model (190 x 63 x 33 ramp, step: 6 planes, its choice, 493 us; 4
+// planes 544 us, 8 planes 581 us).
 int box_ci_len(const wmx_plan* p) {
   const bool f32 = p->nd.prec == WMX_PREC_FP32_BULK;
   const double t32[4] = {0.0, 0.55, 0.78, 1.0}, t64[3] = {0.0, 0.6, 1.0};
@@ -1029,8 +1031,8 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
     // (half reciprocal volumes and filter widths of the curvilinear FP64 kernel)
     if (!p->box && p->nd.prec != WMX_PREC_FP32_BULK)
       for (int b = 0; b < p->nb; ++b) WMX_CHECK(launch_curv_geo(p->hb[b], nullptr));
-    // those kernels and the box kernels read a fused side's k ghosts at their periodic images: a side that is no
-    // plain periodic face of its own block is filled by a launch
+    // the kernels that read the state read a fused side's k ghosts at their periodic images: a
+    // side that is no plain periodic face of its own block is filled by a launch
     bool image = true;
     for (int b = 0; b < p->nb; ++b)
       for (int sd = 0; sd < 2; ++sd)

@@ -393,7 +393,7 @@ class Solver:
     def step(self, Q, time=0.0, graph=False):
         """The reference driver's step, max_dt then advance (examples/channel_wmles.py:
         124-125), with dt kept on the device (the CFL min is taken in the first stage's
-        primitive pass; same value as max_dt).  Launches go to the caller's stream;
+        launches; same value as max_dt).  Launches go to the caller's stream;
         graph=True instead replays the whole launch sequence as one captured hipGraph
         when the state pointers repeat (the usual `Q, dt = solver.step(Q)` loop alternates
         two buffers).  Returns (Q_new, dt)."""
