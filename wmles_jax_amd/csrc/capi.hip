@@ -1295,12 +1295,21 @@ int wmx_mass_flux(wmx_plan* p, double* const* q, void* stream) {
   WMX_CHECK(timed(p, K_MF, s, [&] {
     hipError_t e = launch_mf_partial(p->d_blks, p->d_pre_int, p->nb, nwg_of(p->pre_int), pq,
                                      p->d_case_dir, p->d_part, s);
-    if (e == hipSuccess)
-      e = launch_case_final(1, p->n_cases, p->case_wg_ident ? nullptr : p->d_case_wg, p->d_case_off, p->d_part,
-                            p->d_case_target, p->d_delta, s);
+    const int* list = p->case_wg_ident ? nullptr : p->d_case_wg;
+    int most = 0;                                // partials of a case: up to a wavefront's lanes
+    for (int c = 0; c < p->n_cases; ++c) most = std::max(most, p->case_off[c + 1] - p->case_off[c]);
+    MfFinal fin;
+    if (most <= 64) {
+      fin.list = list;
+      fin.off = p->d_case_off;
+      fin.part = p->d_part;
+      fin.target = p->d_case_target;
+    } else if (e == hipSuccess) {
+      e = launch_case_final(1, p->n_cases, list, p->d_case_off, p->d_part, p->d_case_target, p->d_delta, s);
+    }
     if (e == hipSuccess)
       e = launch_mf_apply(p->d_blks, p->d_pre_all, p->nb, nwg_of(p->pre_all), pq, p->d_case_dir,
-                          p->d_delta, s);
+                          p->d_delta, fin, s);
     return e;
   }));
   return 0;

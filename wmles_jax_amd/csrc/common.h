@@ -220,8 +220,15 @@ hipError_t launch_mf_partial(const BlockDev* d_blks, const int* d_pre, int nblk,
 hipError_t launch_case_final(int mode, int ncases, const int* d_case_wg, const int* d_case_off,
                              const double* d_part, const double* d_target, double* d_out,
                              hipStream_t s);
+// fin.off != nullptr: the deltas are formed from the partials by the launch itself
+struct MfFinal {
+  const int* list = nullptr;       // as GradDt's
+  const int* off = nullptr;
+  const double* part = nullptr;
+  const double* target = nullptr;
+};
 hipError_t launch_mf_apply(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
-                           const int* d_case_dir, const double* d_delta, hipStream_t s);
+                           const int* d_case_dir, const double* d_delta, MfFinal fin, hipStream_t s);
 hipError_t launch_wm_eval(const NumDev& nd, int mode, long long n, const double* a, const double* b,
                           const double* c, const double* d, double T_wall, double* o0, double* o1,
                           hipStream_t s);
