@@ -230,8 +230,7 @@ int wmx_advance(wmx_plan* plan, double* const* q0, double* const* qout, double d
                 const double* d_dt, double time, void* stream);
 /* The reference driver's step (examples/channel_wmles.py:124-125: max_dt then advance)
    with dt kept on the device: d_dt[case] <- CFL dt of q0, then qout = advance(q0).
-   The dt partials come from the first stage's primitive launch (same values as
-   wmx_max_dt, one pass over q0 fewer).
+   The dt partials come from the first stage's launches (same values as wmx_max_dt).
    use_graph != 0 (and a non-default stream, and no time-dependent inflow): the launch
    sequence is captured once per (q0, qout, d_dt, time) into a hipGraph (at most 4
    kept per plan) and replayed on later calls with the same pointers. */
@@ -244,10 +243,9 @@ int wmx_step(wmx_plan* plan, double* const* q0, double* const* qout, double* d_d
 int wmx_plan_set_tiling(wmx_plan* plan, int32_t ci_len, int32_t order);
 /* FP32-bulk kernel form (no reference counterpart): on != 0 (the default) the flux kernel
    evaluates the Green-Gauss gradients, SGS viscosity and Ducros sensor of each plane in
-   LDS as it marches, so no gradient records go through HBM and the separate gradient launch
-   keeps only its side work (per-case dt min, Newton wall faces); on == 0 runs the separate
+   LDS as it marches, so no gradient records go through HBM; on == 0 runs the separate
    gradient kernel and the flux kernel that reads its records.  Persistent stages follow
-   the same choice; FP64 plans ignore it. */
+   the same choice; FP64 plans, which always evaluate them in the march, ignore it. */
 int wmx_plan_set_fused_gradients(wmx_plan* plan, int32_t on);
 /* Persistent stages (the batching form's launch structure; no reference counterpart):
    on != 0 runs every RK stage of wmx_advance / wmx_step as ONE cooperative launch -- a

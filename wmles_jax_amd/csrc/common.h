@@ -320,10 +320,6 @@ template <class T>
 using gconst = const __attribute__((address_space(1))) T*;
 template <class T>
 using gmut = __attribute__((address_space(1))) T*;
-template <class T>
-__device__ __forceinline__ gconst<T> gmem(const T* p) { return (gconst<T>)p; }
-template <class T>
-__device__ __forceinline__ gmut<T> gmem_w(T* p) { return (gmut<T>)p; }
 
 // Load / store at element `i` of an array whose base pointer is wave-uniform, with the
 // byte offset formed in 32 bits: the access compiles to the scalar-base global form

@@ -170,56 +170,6 @@ __device__ __forceinline__ void flux_core_f32(const NumDev& nd, const CellWT<flo
   viscous_face_e<float>(gL, gR, phL, phR, d0 * id, d1 * id, d2 * id, id, sx, sy, sz, Ff);
 }
 
-template <class R>
-__device__ __forceinline__ void flux_core(const NumDev& nd, const CellWT<R>& L2, const CellWT<R>& L,
-                                          const CellWT<R>& Rc, const CellWT<R>& R2, R thL, R thR,
-                                          const CellGT<R>& gL, const CellGT<R>& gR, R TL, R TR,
-                                          const double* xL, const double* xR, double Sx, double Sy,
-                                          double Sz, double* F) {
-  static_assert(sizeof(R) == 8, "the FP32-bulk face flux is flux_core_f32");
-  const R sx = R(Sx), sy = R(Sy), sz = R(Sz);
-  const int sch = nd.scheme;
-  double Fc[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, Fu[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  double s = sch == WMX_SCHEME_MUSCLHLLC ? 1.0 : 0.0;
-  if (sch == WMX_SCHEME_HYBRID) {
-    const R th = fmax(thL, thR);
-    s = (double)fmin(fmax((th - R(nd.th0)) / R(nd.th1 - nd.th0), R(0.0)), R(1.0));
-  }
-  if (s < 1.0) {
-    R Fr[5], un4;
-    const bool keep = sch == WMX_SCHEME_KEEP || (sch == WMX_SCHEME_HYBRID && nd.central == WMX_SCHEME_KEEP);
-    if (keep) central_flux<true, R>(nd.order, L2, L, Rc, R2, sx, sy, sz, Fr, &un4);
-    else central_flux<false, R>(nd.order, L2, L, Rc, R2, sx, sy, sz, Fr, &un4);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) Fc[v] = (double)Fr[v];
-  }
-  if (s > 0.0) {
-    R Fr[5];
-    muscl_hllc_flux<R>(R(nd.gas.gamma), nd.limiter, L2, L, Rc, R2, sx, sy, sz, R(0), Fr);
-#pragma unroll
-    for (int v = 0; v < 5; ++v) Fu[v] = (double)Fr[v];
-  }
-  if (sch == WMX_SCHEME_HYBRID) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) F[v] = (1.0 - s) * Fc[v] + s * Fu[v];
-  } else if (sch == WMX_SCHEME_MUSCLHLLC) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) F[v] = Fu[v];
-  } else {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) F[v] = Fc[v];
-  }
-  const double dx0 = xR[0] - xL[0], dx1 = xR[1] - xL[1], dx2 = xR[2] - xL[2];
-  const double idist = 1.0 / sqrt((dx0 * dx0 + dx1 * dx1) + dx2 * dx2);
-  const R phL[4] = {L.u, L.v, L.w, TL};
-  const R phR[4] = {Rc.u, Rc.v, Rc.w, TR};
-  R Fv[5] = {R(0), R(0), R(0), R(0), R(0)};
-  viscous_face_e<R>(gL, gR, phL, phR, R(dx0 * idist), R(dx1 * idist), R(dx2 * idist), R(idist), sx, sy,
-                    sz, Fv);
-#pragma unroll
-  for (int v = 0; v < 5; ++v) F[v] = F[v] + (double)Fv[v];
-}
-
 // FP32-bulk tile: 15 rows (j) x 16 columns (k) of cells on a 16 x 16 thread grid.
 // Per plane the tile has 240 i faces, 16 x 16 j faces (incl. the upper edge row) and
 // 15 x 17 k faces (incl. the upper edge column): thread (tj, tk) evaluates the i face

@@ -361,14 +361,6 @@ WMX_HD void viscous_face_e(const CellGT<R>& a, const CellGT<R>& b, const R* phiL
   F[4] = F[4] + ((-(ffma<R>(uf0, ts0, uf1 * ts1) + uf2 * ts2)) - kf * dTdn);
 }
 
-WMX_HD void viscous_face(const CellG& a, const CellG& b, const double* phiL, const double* phiR,
-                         const double* xcL, const double* xcR, double Sx, double Sy, double Sz,
-                         double* F) {
-  double dx0 = xcR[0] - xcL[0], dx1 = xcR[1] - xcL[1], dx2 = xcR[2] - xcL[2];
-  double idist = 1.0 / sqrt((dx0 * dx0 + dx1 * dx1) + dx2 * dx2);
-  viscous_face_e<double>(a, b, phiL, phiR, dx0 * idist, dx1 * idist, dx2 * idist, idist, Sx, Sy, Sz, F);
-}
-
 // Plain-form KEP/KEEP wrappers used by the FP64 kernels (no gauge).
 template <bool KEEP>
 WMX_HD void central_flux(int order, const CellW& L2, const CellW& L, const CellW& R, const CellW& R2,
