@@ -141,22 +141,27 @@ __device__ __forceinline__ double cell_dt(const BlockDev& B, const NumDev& nd, u
   return cell_dt_eval(nd, w, m, vol);
 }
 
-// 1 / dt of a box cell but for the factor cfl, within 1e-10 of cell_dt's (BoxEnt's reciprocal
-// widths, one reciprocal of rho and one square root; the box check admits metrics that are
-// within 3e-11 of the tables).  cv = 4 max(4/3, gamma / Pr) mu(T) (T + S) / (T c).  NaN where
-// the terms may cancel.
+// 1 / dt of a box cell but for the factor cfl, within 2e-10 of cell_dt's: BoxEnt's reciprocal
+// widths (the box check admits metrics within 3e-11 of the tables), one reciprocal of rho, one
+// root of two corrections (1e-12 from the 2^-14 that fdiv takes the hardware estimates to have),
+// and a pressure that is the difference of total and kinetic energy, whose roundings grow by
+// their ratio.  Below 1e-4 of the total energy (Mach 190) the difference is not relied on: two
+// ways of rounding could even disagree on its sign.  There, and where density or pressure are
+// not positive, NaN comes back.  cv = 4 max(4/3, gamma / Pr) mu(T) (T + S) / (T c).
 __device__ __forceinline__ double box_rate(const NumDev& nd, const double* q, double cv, const double* iw) {
   const GasC& gas = nd.gas;
   const double ir = rcp64(q[0]);
   const double u = q[1] * ir, v = q[2] * ir, w = q[3] * ir;
-  const double pr = ((gas.gamma - 1.0) * ir) * (q[4] - (0.5 * q[0]) * ((u * u + v * v) + w * w));   // p / rho
+  const double ei = q[4] - (0.5 * q[0]) * ((u * u + v * v) + w * w);   // p / (gamma - 1)
+  const double pr = ((gas.gamma - 1.0) * ir) * ei;                     // p / rho
   const double c2 = gas.gamma * pr, T = pr * nd.rc.iR;
   const double y = __builtin_amdgcn_rsq(c2), s0 = c2 * y;
-  const double cs = s0 + (0.5 * y) * (c2 - s0 * s0);
+  const double s1 = s0 + (0.5 * y) * (c2 - s0 * s0);
+  const double cs = s1 + (0.5 * y) * (c2 - s1 * s1);
   const double nu4 = ((cv * (T * cs)) * rcp64(T + gas.S_suth)) * ir;
   const double x = ((fabs(u) + cs) * iw[0] + (fabs(v) + cs) * iw[1]) + (fabs(w) + cs) * iw[2];
   const double r = x + nu4 * ((iw[0] * iw[0] + iw[1] * iw[1]) + iw[2] * iw[2]);
-  return q[0] > 0.0 && nu4 >= 0.0 ? r : __builtin_nan("");
+  return q[0] > 0.0 && nu4 >= 0.0 && ei > 1e-4 * fabs(q[4]) ? r : __builtin_nan("");
 }
 
 // CFL partial of workgroup wgx of nwg: INT_CELLS interior cells per thread, blockDim.x apart
