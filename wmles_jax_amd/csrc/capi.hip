@@ -1021,7 +1021,7 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
   WMX_CHECK(hipMemset(d_nz, 0, sizeof(unsigned) * (p->nb + 1)));
   for (int b = 0; b < p->nb; ++b) {
     WMX_CHECK(launch_cell_sb(p->hb[b], d_nz + b, nullptr));
-    WMX_CHECK(launch_box_check(p->hb[b], d_bad, nullptr));
+    WMX_CHECK(launch_box_check(p->hb[b], p->nd.prec, d_bad, nullptr));
   }
   WMX_CHECK(hipDeviceSynchronize());
   {

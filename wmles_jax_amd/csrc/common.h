@@ -202,8 +202,9 @@ hipError_t launch_curv(int mode, const BlockDev* d_blks, const int4* d_tiles, in
                        const NumDev& nd, Ptrs qin, Ptrs q0, Ptrs out, const double* d_dt, double dt,
                        int zfuse, hipStream_t s);
 hipError_t launch_curv_geo(const BlockDev& hb, hipStream_t s);
-// fills a block's BoxEnt tables; *d_bad becomes non-zero if the block is no box
-hipError_t launch_box_check(const BlockDev& hb, unsigned* d_bad, hipStream_t s);
+// fills a block's BoxEnt tables; *d_bad becomes non-zero if the block is no box for plans of
+// precision prec
+hipError_t launch_box_check(const BlockDev& hb, int prec, unsigned* d_bad, hipStream_t s);
 hipError_t launch_shell_save(const BlockDev* d_blks, const int* d_pre, int nblk, int nwg, Ptrs q,
                              hipStream_t s);
 hipError_t launch_shell_finish(int mode, const BlockDev* d_blks, const int* d_pre, int nblk, int nwg,
