@@ -215,10 +215,11 @@ int wmx_apply_bcs_phases(wmx_plan* plan, double* const* q, int32_t first, int32_
                          void* stream);
 /* R = RHS(q) with zero ghosts, for a q whose ghosts the caller has filled (no sweep; q is
    not modified).  The RHS part of Solver._rhs after apply_bcs (wmles/solver.py:97-106);
-   the callers' own sources are added by the caller. */
+   the callers' own sources are added by the caller.  r may be q itself or overlap it (one
+   copy more, and q is then not kept). */
 int wmx_rhs_filled(wmx_plan* plan, double* const* q, double* const* r, void* stream);
-/* R = RHS(q) with zero ghosts; q's ghost cells are overwritten by the sweep.
-   Replaces Solver.rhs / _rhs (wmles/solver.py:97-106,159-160). */
+/* R = RHS(q) with zero ghosts; q's ghost cells are overwritten by the sweep.  r may be q
+   itself or overlap it (one copy more).  Replaces Solver.rhs / _rhs (wmles/solver.py:97-106,159-160). */
 int wmx_rhs(wmx_plan* plan, double* const* q, double* const* r, double time, void* stream);
 /* One SSP-RK3 step + constraints: qout = step(q0).  The three stages run in place
    in qout (qout must not alias q0).  q0 is returned unchanged (its ghosts are saved

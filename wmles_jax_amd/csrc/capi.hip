@@ -642,6 +642,25 @@ hipError_t plan_flux(const wmx_plan* p, int mode, const BlockDev* d_blks, const 
   return launch_flux(mode, d_blks, d_tiles, ntiles, ci_len, nd, qin, q0, out, d_dt, dt, s);
 }
 
+// r = RHS of the filled state q, zero ghosts.  A flux launch that reads its neighbours' states must
+// not write over them: where some r overlaps some q, its output is formed in the stage buffer.
+int rhs_of_filled(wmx_plan* p, Ptrs q, Ptrs r, hipStream_t s) {
+  auto bytes = [&](int b) { return (uintptr_t)(5 * sizeof(double)) * (uintptr_t)p->hb[b].cells; };
+  bool over = false;
+  for (int i = 0; direct(p) && i < p->nb; ++i)
+    for (int j = 0; j < p->nb; ++j) {
+      const uintptr_t a = (uintptr_t)r.p[i], b = (uintptr_t)q.p[j];
+      over = over || (a < b + bytes(j) && b < a + bytes(i));
+    }
+  const Ptrs out = over ? stage_buffer(p) : r;
+  WMX_CHECK(plan_flux(p, 0, p->d_blks, p->d_tiles, (int)p->tiles.size(), p->ci_len, p->nd, q, q, out, nullptr, 0.0,
+                      false, s));
+  WMX_CHECK(launch_shell_finish(0, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), q, out, nullptr, 0.0, s));
+  for (int b = 0; over && b < p->nb; ++b)
+    WMX_CHECK(hipMemcpyAsync(r.p[b], out.p[b], bytes(b), hipMemcpyDeviceToDevice, s));
+  return 0;
+}
+
 int check_plan(const wmx_plan* p) {
   if (!p) return fail("null plan");
   if (!p->ws) return fail("plan has no workspace bound (wmx_plan_bind_workspace)");
@@ -1268,11 +1287,7 @@ int wmx_rhs_filled(wmx_plan* p, double* const* q, double* const* r, void* stream
   hipStream_t s = as_stream(stream);
   Ptrs pq = make_ptrs(p, q), pr = make_ptrs(p, r);
   if (run_cells(p, pq, 0.0, nullptr, 0.0, s, nullptr, false, false)) return 1;
-  WMX_CHECK(plan_flux(p, 0, p->d_blks, p->d_tiles, (int)p->tiles.size(), p->ci_len, p->nd, pq, pq, pr,
-                        nullptr, 0.0, false, s));
-  WMX_CHECK(launch_shell_finish(0, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), pq, pr,
-                                nullptr, 0.0, s));
-  return 0;
+  return rhs_of_filled(p, pq, pr, s);
 }
 
 int wmx_rhs(wmx_plan* p, double* const* q, double* const* r, double time, void* stream) {
@@ -1280,11 +1295,7 @@ int wmx_rhs(wmx_plan* p, double* const* q, double* const* r, double time, void* 
   hipStream_t s = as_stream(stream);
   Ptrs pq = make_ptrs(p, q), pr = make_ptrs(p, r);
   if (run_cells(p, pq, time, nullptr, 0.0, s)) return 1;
-  WMX_CHECK(plan_flux(p, 0, p->d_blks, p->d_tiles, (int)p->tiles.size(), p->ci_len, p->nd, pq, pq, pr,
-                        nullptr, 0.0, false, s));
-  WMX_CHECK(launch_shell_finish(0, p->d_blks, p->d_pre_shell, p->nb, nwg_of(p->pre_shell), pq, pr,
-                                nullptr, 0.0, s));
-  return 0;
+  return rhs_of_filled(p, pq, pr, s);
 }
 
 int wmx_mass_flux(wmx_plan* p, double* const* q, void* stream) {
