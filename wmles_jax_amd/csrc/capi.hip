@@ -1624,6 +1624,7 @@ int wmx_step(wmx_plan* p, double* const* q0, double* const* qout, double* d_dt, 
 
 int wmx_wall_stats(wmx_plan* p, double* const* q, double* d_tau, double* d_qw, void* stream) {
   if (check_plan(p)) return 1;
+  if (!q || (!p->wall.empty() && (!d_tau || !d_qw))) return fail("null argument");   // (the kernel writes both)
   hipStream_t s = as_stream(stream);
   Ptrs pq = make_ptrs(p, q);
   WMX_CHECK(launch_wall(p->d_blks, p->d_wall, (int)p->wall.size(), p->wall_max, pq, p->nd, s, d_tau, d_qw));
