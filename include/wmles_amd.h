@@ -155,7 +155,8 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks,
                     const wmx_numerics_desc* numerics, int32_t ninflow,
                     const wmx_inflow_desc* inflows, wmx_plan** out);
 int wmx_plan_destroy(wmx_plan* plan);
-/* Device workspace the plan needs (bytes, 256-aligned); bind it once. */
+/* Device workspace the plan needs (bytes, 256-aligned); bind it once.  Binding another drops the
+   steps that wmx_step captured with the former one. */
 int wmx_plan_workspace_bytes(const wmx_plan* plan, size_t* bytes);
 int wmx_plan_bind_workspace(wmx_plan* plan, void* d_workspace, size_t bytes);
 /* Number of WallModel faces and their (block, axis, side, n_t1, n_t2) records. */

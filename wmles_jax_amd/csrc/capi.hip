@@ -1064,6 +1064,7 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
       p->fuse_last = false;
       for (BlockDev& B : p->hb) B.zfuse = 0;
     }
+    drop_graphs(p);                              // (captured steps hold the tile table and the workspace)
     if (retile(p)) return 1;
     for (int b = 0; b < p->nb; ++b)
       p->hb[b].sb_zero = p->hb[b].Sb ? (int)(~nz[b] & ((1u << NSB_PLANES) - 1u)) : 0;
