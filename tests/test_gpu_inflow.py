@@ -27,3 +27,9 @@ def test_inflow_rows_match_the_oracle(nz, n_modes):
     A = s1.apply_bcs(Q, s1.geoms, t)[0].cpu().numpy()
     B = np.asarray(s0.apply_bcs([q.cpu().numpy() for q in Q], s0.geoms, t)[0])
     assert golden_io.rel_err(A[:, :ng], B[:, :ng]) <= 1e-13
+
+
+@pytest.mark.parametrize("nz,n_modes", [(694, 8), (1017, 5), (536, 11)])
+def test_wide_rows_with_a_large_phase_table_match_the_oracle(nz, n_modes):
+    """Rows of more than 512 cells whose phase table leaves room for one row buffer."""
+    test_inflow_rows_match_the_oracle(nz, n_modes)

@@ -799,7 +799,7 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
       delete p;
       return fail("inflow needs a profile table and at least one mode");
     }
-    p->inflows.push_back(InflowDev{in.n_tab, in.n_modes, 0, in.table, in.modes, in.U_inf, in.L,
+    p->inflows.push_back(InflowDev{in.n_tab, in.n_modes, 0, 2, in.table, in.modes, in.U_inf, in.L,
                                    in.rho_inf, in.p_inf});
   }
   // (what a caller's fill writes is unknown: every pass of such a plan is kept)

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "../../include/wmles_amd.h"
+#include "inflow.h"
 #include "physics.h"
 
 namespace wmx {
@@ -115,8 +116,7 @@ struct WallOp {
 
 struct InflowDev {
   int n_tab, n_modes;
-  int coop;                 // set by the launcher: 1 phases evaluated cooperatively in LDS, 2 with the
-                            // table's y column there too
+  int coop, rows;           // set by the launcher (InflowForm)
   const double* table;
   const double* modes;
   double U_inf, L, rho_inf, p_inf;

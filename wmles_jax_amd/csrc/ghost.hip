@@ -183,7 +183,7 @@ __global__ void k_inflow(const BlockDev* __restrict__ blks, int blk, InflowDev i
   // sum as one thread per cell doing its modes in turn.  Mode-major with an odd pitch, so
   // that lanes of one mode (the sums) or of one cell (the phases) fall in distinct banks.
   const int P2 = N2 | 1;
-  double* cosb = red + 2 * blockDim.x + 1;              // [nm][P2] when cooperative
+  double* cosb = red + in.rows * blockDim.x + 1;        // [nm][P2] when cooperative
   double* yz = cosb + (long long)P2 * nm;               // [2][N2]
   double* ys = yz + 2 * N2;                             // [n_tab] the table's y column
   const bool coop = in.coop, ytab = in.coop == 2;
@@ -240,16 +240,18 @@ __global__ void k_inflow(const BlockDev* __restrict__ blks, int blk, InflowDev i
   }
   // row statistics over the interior span, summed in numpy's add.reduce order (the first element
   // plus the pairwise sum of the rest, whose runs of <= 128 use 8 interleaved accumulators);
-  // two buffers in turn, so that one barrier a mean is enough
+  // two buffers in turn, so that one barrier a mean is enough (one buffer: a second barrier)
   int turn = 0;
   auto row_mean = [&](double val) {
-    double* buf = red + (turn ^= 1) * blockDim.x;
+    if (in.rows == 1) __syncthreads();                   // the previous mean's reads
+    else turn ^= 1;
+    double* buf = red + turn * blockDim.x;
     buf[K] = inner ? val : 0.0;
     __syncthreads();
     const double* e = buf + ng;
     const int n = nk - 1;
     if (n < 8 || n > 128) {                              // short or long rows: one thread
-      double* sum = red + 2 * blockDim.x;
+      double* sum = red + in.rows * blockDim.x;
       if (K == 0) *sum = np_sum([&](int i) { return e[i]; }, nk) / nk;
       __syncthreads();
       return *sum;
@@ -313,20 +315,12 @@ hipError_t launch_fill_cells(const BlockDev* d_blks, const GhostOp* d_ops, int n
 hipError_t launch_inflow(const BlockDev* d_blks, int blk, int N1, int N2, int ng, InflowDev in,
                          Ptrs q, GasC gas, double time, const double* d_dt, double coef,
                          hipStream_t s) {
-  int threads = ((N2 + 63) / 64) * 64;
-  if (threads > 1024) return hipErrorInvalidValue;
+  if (N2 > 1024) return hipErrorInvalidValue;
   dim3 grid(N1, ng);
-  // cooperative phase evaluation when a row's (cell, mode) table fits in 56 KB of LDS
-  const size_t coop_bytes = sizeof(double) * ((size_t)(N2 | 1) * in.n_modes + 2 * (size_t)N2);
-  const size_t tab_bytes = sizeof(double) * (size_t)in.n_tab, lds = 64 * 1024;
-  in.coop = coop_bytes <= 56 * 1024 ? 1 : 0;
-  auto shm_of = [&](int th, size_t extra) { return sizeof(double) * (2 * (size_t)th + 1) + extra; };
-  // more lanes for the phase table, and the table's y column, where the 64 KB hold them
-  if (in.coop && threads < 256) threads = 256;
-  if (in.coop && threads < 512 && shm_of(512, coop_bytes) <= lds) threads = 512;
-  if (in.coop && shm_of(threads, coop_bytes + tab_bytes) <= lds) in.coop = 2;
-  size_t shm = shm_of(threads, in.coop ? coop_bytes + (in.coop == 2 ? tab_bytes : 0) : 0);
-  hipLaunchKernelGGL(k_inflow, grid, dim3(threads), shm, s, d_blks, blk, in, q, gas, time, d_dt,
+  const InflowForm f = inflow_form(N2, in.n_modes, in.n_tab);
+  in.coop = f.coop;
+  in.rows = f.rows;
+  hipLaunchKernelGGL(k_inflow, grid, dim3(f.threads), f.lds, s, d_blks, blk, in, q, gas, time, d_dt,
                      coef);
   return hipGetLastError();
 }
