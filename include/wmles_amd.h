@@ -249,6 +249,15 @@ int wmx_plan_set_tiling(wmx_plan* plan, int32_t ci_len, int32_t order);
    gradient kernel and the flux kernel that reads its records.  Persistent stages follow
    the same choice; FP64 plans, which always evaluate them in the march, ignore it. */
 int wmx_plan_set_fused_gradients(wmx_plan* plan, int32_t on);
+/* Which flux kernel the plan's right-hand sides run (no counterpart in the reference); settled by
+   the bound geometry, the precision and wmx_plan_set_fused_gradients. */
+enum {
+  WMX_FORM_SPLIT = 0,   /* FP32-bulk: primitive and gradient records, then the face fluxes */
+  WMX_FORM_FUSED = 1,   /* FP32-bulk: primitive records, gradients in the flux march */
+  WMX_FORM_BOX = 2,     /* both precisions: from the state, metrics as three one-dimensional tables */
+  WMX_FORM_CURV = 3     /* FP64: from the state, metrics per cell */
+};
+int wmx_plan_kernel_form(const wmx_plan* plan, int32_t* form);
 /* Persistent stages (the batching form's launch structure; no reference counterpart):
    on != 0 runs every RK stage of wmx_advance / wmx_step as ONE cooperative launch -- a
    grid of the kernel's co-resident maximum walks the stage's ghost-sweep phases, the

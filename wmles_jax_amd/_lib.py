@@ -107,6 +107,7 @@ def _load():
         "wmx_plan_set_tiling": ([P, C.c_int32, C.c_int32], C.c_int),
         "wmx_plan_set_persistent": ([P, C.c_int32], C.c_int),
         "wmx_plan_set_fused_gradients": ([P, C.c_int32], C.c_int),
+        "wmx_plan_kernel_form": ([P, C.POINTER(C.c_int32)], C.c_int),
         "wmx_tile_model": ([C.c_int32, P, C.c_int32, C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32)], C.c_int),
         "wmx_plan_tiling": ([P, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32)], C.c_int),
         "wmx_mass_flux": ([P, PP, P], C.c_int),
@@ -145,6 +146,12 @@ class WmxError(RuntimeError):
 def check(rc):
     if rc != 0:
         raise WmxError(lib.wmx_last_error().decode())
+
+
+def kernel_form(plan):
+    form = C.c_int32()
+    check(lib.wmx_plan_kernel_form(plan, C.byref(form)))
+    return ("split", "fused", "box", "curvilinear")[form.value]
 
 
 def ptr_array(tensors):

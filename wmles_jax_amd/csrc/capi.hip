@@ -1553,6 +1553,13 @@ int wmx_plan_set_fused_gradients(wmx_plan* p, int32_t on) {
   return 0;
 }
 
+int wmx_plan_kernel_form(const wmx_plan* p, int32_t* form) {
+  if (check_plan(p)) return 1;
+  if (!form) return fail("null argument");
+  *form = direct(p) ? (p->box ? WMX_FORM_BOX : WMX_FORM_CURV) : (p->fuse_grad ? WMX_FORM_FUSED : WMX_FORM_SPLIT);
+  return 0;
+}
+
 int wmx_plan_set_persistent(wmx_plan* p, int32_t on) {
   if (check_plan(p)) return 1;
   if (!on) {

@@ -215,6 +215,13 @@ class EnsembleSolver:
         _lib.check(_lib.lib.wmx_plan_set_persistent(self._plan, 1 if on else 0))
         self.persistent = bool(on)
 
+    def kernel_form(self):
+        """The flux kernel in use: "box" (metrics as three one-dimensional tables) or "curvilinear"
+        (FP64, metrics per cell), both from the state itself; FP32-bulk plans with other blocks
+        "fused" (primitive records, gradients in the march), and without fused gradients
+        "split"."""
+        return _lib.kernel_form(self._plan)
+
     def set_tiling(self, ci_len=0, order=1):
         """Flux-kernel tiling: i-planes per marching tile (0: automatic), XCD-interleaved
         order (1) or not (0)."""
