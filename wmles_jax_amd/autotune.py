@@ -3,15 +3,21 @@
 Times a few steps of a solver (or ensemble) for each candidate tiling -- i-planes per
 marching tile (0: the plan's makespan model) x XCD-interleaved tile order -- with HIP
 events around the flux kernel,
-keeps the fastest, and caches the choice per (device, form, block sizes) in a JSON file
-(default ~/.cache/wmles_jax_amd/tiling.json, override with WMX_TUNE_CACHE).
+keeps the fastest, and caches the choice per (device, precision, flux kernel and its
+revision, scheme, block sizes) in a JSON file (default ~/.cache/wmles_jax_amd/tiling.json, override with WMX_TUNE_CACHE).
 """
 import json
 import os
 
 import torch
 
-CANDIDATES = ((0, 1), (0, 0), (8, 1), (12, 1), (16, 1), (24, 1), (32, 1))
+# Short chunks fill the chip on small blocks (24 x 16 x 12 cells in the box kernel: one plane per
+# tile 15 us, four 29 us), long ones save start-up planes on large blocks.
+CANDIDATES = ((0, 1), (0, 0), (1, 1), (2, 1), (4, 1), (6, 1), (8, 1), (12, 1), (16, 1), (24, 1), (32, 1))
+# Raised when a flux kernel changes enough to move its best chunk (256 x 128 x 128 box, FP32: 8
+# planes 265 us, 24 planes 372 us; the kernel before it was best at 37): entries of other
+# revisions are timed anew.
+REVISION = 2
 
 
 def _cache_path():
@@ -23,7 +29,7 @@ def _key(obj):
     solvers = getattr(obj, "solvers", [obj])
     dims = [tuple(b.n) for s in solvers for b in s.blocks]
     scheme = type(solvers[0].scheme).__name__
-    return f"{torch.cuda.get_device_name()}|{solvers[0].precision}|{scheme}|{dims}"
+    return f"{torch.cuda.get_device_name()}|{solvers[0].precision}|{obj.kernel_form()}.{REVISION}|{scheme}|{dims}"
 
 
 def tune(obj, Q, steps=4, candidates=CANDIDATES, use_cache=True, rounds=2, warmup=10):
