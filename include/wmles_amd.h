@@ -270,8 +270,13 @@ int wmx_plan_kernel_form(const wmx_plan* plan, int32_t* form);
    (wmx_step's use_graph is ignored while it is on).  on == 0 restores the separate
    launches. */
 int wmx_plan_set_persistent(wmx_plan* plan, int32_t on);
-/* The automatic choice without a plan (host only): i-planes per tile and tile count
-   for blocks of interior sizes dims[3 * nblocks] in the given form on cu_count CUs. */
+/* The automatic choice without a plan (host only): i-planes per tile and tile count for
+   blocks of interior sizes dims[3 * nblocks] in the given kernel form (WMX_FORM_*) and
+   precision on cu_count CUs. */
+int wmx_tile_model_form(int32_t nblocks, const int32_t* dims, int32_t form, int32_t precision,
+                        int32_t cu_count, int32_t* ci_len, int32_t* ntiles);
+/* The same for the kernels that read stored records (FP32-bulk: WMX_FORM_SPLIT and
+   WMX_FORM_FUSED; their model with the FP64 start-up cost, which no plan runs). */
 int wmx_tile_model(int32_t nblocks, const int32_t* dims, int32_t precision, int32_t cu_count,
                    int32_t* ci_len, int32_t* ntiles);
 /* The tiling in use: i-planes per tile, order, number of tiles. */

@@ -108,6 +108,8 @@ def _load():
         "wmx_plan_set_persistent": ([P, C.c_int32], C.c_int),
         "wmx_plan_set_fused_gradients": ([P, C.c_int32], C.c_int),
         "wmx_plan_kernel_form": ([P, C.POINTER(C.c_int32)], C.c_int),
+        "wmx_tile_model_form": ([C.c_int32, P, C.c_int32, C.c_int32, C.c_int32, C.POINTER(C.c_int32),
+                                 C.POINTER(C.c_int32)], C.c_int),
         "wmx_tile_model": ([C.c_int32, P, C.c_int32, C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32)], C.c_int),
         "wmx_plan_tiling": ([P, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int32)], C.c_int),
         "wmx_mass_flux": ([P, PP, P], C.c_int),

@@ -352,8 +352,8 @@ hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 // Flux tiles: per block (i-chunk, j-tile, k-tile).  Order 1 interleaves contiguous
 // spans of the tile list across the 8 XCDs (workgroup w runs on XCD w % 8), so the
 // tiles one XCD runs are neighbours and share its L2.
-// i-planes per tile when none is requested: both flux kernels run two 256-thread
-// workgroups per CU, so a launch of T tiles takes ceil(T / (2 CUs)) rounds of
+// i-planes per tile when none is requested, for the kernels that read records: both run two
+// 256-thread workgroups per CU, so a launch of T tiles takes ceil(T / (2 CUs)) rounds of
 // (ci + alpha) plane times, alpha being the per-tile start-up (the FP32-bulk kernel's
 // register window costs about 1.5 planes, the FP64 kernel's about 0.5).  The shortest
 // estimate over ci in [4, 64] wins (ties: the longer chunk).  dims: n[3] per block.
@@ -394,21 +394,25 @@ bool direct(const wmx_plan* p) { return p->nd.prec != WMX_PREC_FP32_BULK || (p->
 // per tile, one round, 278 us; 24 per tile, one round and 24 tiles, 372 us).  The curvilinear
 // FP64 kernel takes the same model (190 x 63 x 33 ramp, step: 6 planes, its choice, 493 us; 4
 // planes 544 us, 8 planes 581 us).
-int box_ci_len(const wmx_plan* p) {
-  const bool f32 = p->nd.prec == WMX_PREC_FP32_BULK;
+int direct_ci_len(int nb, const int* dims, int prec, int cu_count, long long* ntiles) {
+  const bool f32 = prec == WMX_PREC_FP32_BULK;
   const double t32[4] = {0.0, 0.55, 0.78, 1.0}, t64[3] = {0.0, 0.6, 1.0};
   const double* t = f32 ? t32 : t64;
-  const long long cus = std::max(1, p->cu_count), W = f32 ? 3 : 2;
+  const long long cus = std::max(1, cu_count), W = f32 ? 3 : 2;
   int best = 1;
+  long long best_T = 0;
   double best_cost = 1e300;
   for (int ci = 1; ci <= 64; ++ci) {
     long long T = 0;
-    for (const BlockDev& B : p->hb)
-      T += (long long)((B.n[0] + ci - 1) / ci) * ((B.n[1] + FLUX2_TILE_J - 1) / FLUX2_TILE_J) * ((B.n[2] + 15) / 16);
+    for (int b = 0; b < nb; ++b) {
+      const int* n = dims + 3 * b;
+      T += (long long)((n[0] + ci - 1) / ci) * ((n[1] + FLUX2_TILE_J - 1) / FLUX2_TILE_J) * ((n[2] + 15) / 16);
+    }
     const long long r = T / (W * cus), m = T - r * W * cus;
     const double cost = ((double)r + t[(m + cus - 1) / cus]) * (ci + 1);
-    if (cost < best_cost - 1e-9) { best_cost = cost; best = ci; }
+    if (cost < best_cost - 1e-9) { best_cost = cost; best = ci; best_T = T; }
   }
+  if (ntiles) *ntiles = best_T;
   return best;
 }
 
@@ -418,12 +422,10 @@ void build_tiles(wmx_plan* p) {
   const int tjr = FLUX2_TILE_J;
   if (p->ci_req > 0) {
     p->ci_len = p->ci_req;
-  } else if (direct(p)) {
-    p->ci_len = box_ci_len(p);
   } else {
     std::vector<int> dims;
     for (int b = 0; b < p->nb; ++b) dims.insert(dims.end(), p->hb[b].n, p->hb[b].n + 3);
-    p->ci_len = auto_ci_len(p->nb, dims.data(), p->nd.prec, p->cu_count, nullptr);
+    p->ci_len = (direct(p) ? direct_ci_len : auto_ci_len)(p->nb, dims.data(), p->nd.prec, p->cu_count, nullptr);
   }
   for (int b = 0; b < p->nb; ++b) {
     const BlockDev& B = p->hb[b];
@@ -1522,6 +1524,17 @@ int wmx_tile_model(int32_t nblocks, const int32_t* dims, int32_t precision, int3
   if (nblocks < 1 || !dims || !ci_len || !ntiles) return fail("bad argument");
   long long T = 0;
   *ci_len = auto_ci_len(nblocks, dims, precision, cu_count, &T);
+  *ntiles = (int32_t)T;
+  return 0;
+}
+
+int wmx_tile_model_form(int32_t nblocks, const int32_t* dims, int32_t form, int32_t precision, int32_t cu_count,
+                        int32_t* ci_len, int32_t* ntiles) {
+  if (nblocks < 1 || !dims || !ci_len || !ntiles) return fail("bad argument");
+  if (form < WMX_FORM_SPLIT || form > WMX_FORM_CURV) return fail("unknown kernel form");
+  const bool reads_state = form == WMX_FORM_BOX || form == WMX_FORM_CURV;
+  long long T = 0;
+  *ci_len = (reads_state ? direct_ci_len : auto_ci_len)(nblocks, dims, precision, cu_count, &T);
   *ntiles = (int32_t)T;
   return 0;
 }
