@@ -233,6 +233,9 @@ constexpr int bgrad_plane(int i) {
   return i == 0 ? 3 * D + t : i == 1 ? 3 * D + s : i == 2 ? 4 * t : i == 3 ? 4 * s : 3 * (i - 4) + D;
 }
 
+// (FP64) the gradient planes that faces of normal 0 do not read: du/dx, dv/dx, dv/dz, dw/dx, dw/dy
+constexpr int djk_plane(int v) { return v == 0 ? 0 : v == 1 ? 3 : v + 3; }
+
 // Viscous flux (viscous.py:28-51) through a face of normal D and area S, id = 1 / distance of
 // the two centroids: V[0..2] the viscous stress times the area, V[3] the energy flux.  The
 // face gradient's normal component g_n + ((phi_R - phi_L) id - g_n) is (phi_R - phi_L) id;
@@ -552,7 +555,10 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
   request(I0 - 1);
   stage_plane(sP[0], arrive());
   request(I0);
-  // partial outward sum of the own cell I-1 in FP64: its lower i face minus its j / k face sums
+  // Outward sum of the own cell I-1 so far, in FP64.  FP32: its lower i face minus its j / k face
+  // sums; FP64: the lower i face alone, so that the difference of the two i faces is formed before
+  // the smaller sums go in (their sum would round at the size of the flux); those wait in the
+  // planes of the own gradient slot that no i face reads, free after the exchange barrier.
   double Cp[NF];
 #pragma unroll
   for (int v = 0; v < NF; ++v) Cp[v] = 0.0;
@@ -663,6 +669,10 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       if (side >= 0) wall_flux(0, side, I, J, K, Fin);
       else face_axis<0, SC, R>(nd, W0, W1, cell(P, sp_own), Pn, sG[GB<R>::TH][sg_own], G[GB<R>::TH], grad_i, idi, dxi, R(sW[0][tj + 1] * sW[1][tk + 1]), pr, er, Fin);
     }
+    if (!F32 && fin) {
+#pragma unroll
+      for (int v = 0; v < NF; ++v) Cp[v] = (Cp[v] - (double)Fin[v]) - (double)sG[djk_plane(v)][sg_own];
+    }
     if (own_g) {
 #pragma unroll
       for (int v = 0; v < GB<R>::N; ++v) sG[v][sg_own] = G[v];
@@ -673,7 +683,7 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       const double ivol = iwi_p * iyz;
       double a[NF], r[5];
 #pragma unroll
-      for (int v = 0; v < NF; ++v) a[v] = Cp[v] - (double)Fin[v];
+      for (int v = 0; v < NF; ++v) a[v] = F32 ? Cp[v] - (double)Fin[v] : Cp[v];
       if (F32) a[4] = fm(B.p_ref, a[NF - 1], fm(B.e_ref, a[0], a[4]));
 #pragma unroll
       for (int v = 0; v < 5; ++v) r[v] = a[v] * ivol;
@@ -770,13 +780,15 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       stage_plane(sP[0], Pn);
       request(I + 2);
     }
-    // ---- carry: the partial outward sum of the own cell I
+    // ---- carry: the outward sum of the own cell I so far
     if (act && inner) {
       const int jup = tile_tid(tj + 1, tk), kup = kface_slot(tj, tk + 1);
 #pragma unroll
-      for (int v = 0; v < NF; ++v)
-        Cp[v] = (double)Fin[v] - (((double)sFj[v][jup] - (double)sFj[v][tid]) +
-                                  ((double)sFk[v][kup] - (double)sFk[v][tid]));
+      for (int v = 0; v < NF; ++v) {
+        const double d = ((double)sFj[v][jup] - (double)sFj[v][tid]) + ((double)sFk[v][kup] - (double)sFk[v][tid]);
+        Cp[v] = F32 ? (double)Fin[v] - d : (double)Fin[v];
+        if (!F32) sG[djk_plane(v)][sg_own] = (R)d;
+      }
     }
     if (F32) buf ^= 1;
     else __syncthreads();                        // plane I+1 staged

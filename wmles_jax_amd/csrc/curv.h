@@ -69,16 +69,15 @@ __device__ __forceinline__ CellWT<double> cell_wt(const BCell<double>& c) {
   return w;
 }
 
-// Numerical flux (times area) of a face with vector S; dx the centroid difference; gsum(i) the
-// sum of component i of the two cells' gradient records, evaluated after the inviscid part.
-template <int SC, class GS>
-__device__ __forceinline__ void face_curv(const NumDev& nd, const BCell<double>& L2, const BCell<double>& L,
-                                          const BCell<double>& Rc, const BCell<double>& R2, double thL, double thR,
-                                          GS gsum, const double* dx, const double* S, double* F) {
+// Inviscid part of the numerical flux (times area) of a face with vector S; th the larger of its
+// cells' sensors.
+template <int SC>
+__device__ __forceinline__ void inviscid_curv(const NumDev& nd, const BCell<double>& L2, const BCell<double>& L,
+                                              const BCell<double>& Rc, const BCell<double>& R2, double th,
+                                              const double* S, double* F) {
   const int scheme = SC == SC_ANY ? nd.scheme : (SC == SC_HYB_KEP4_ALBADA ? WMX_SCHEME_HYBRID : WMX_SCHEME_KEP);
   double s = scheme == WMX_SCHEME_MUSCLHLLC ? 1.0 : 0.0;
-  if (scheme == WMX_SCHEME_HYBRID)
-    s = fmin(fmax(fdiv<double>(fmax(thL, thR) - nd.th0, nd.th1 - nd.th0), 0.0), 1.0);
+  if (scheme == WMX_SCHEME_HYBRID) s = fmin(fmax(fdiv<double>(th - nd.th0, nd.th1 - nd.th0), 0.0), 1.0);
   // (a part whose weight is exactly 0 is not evaluated)
 #pragma unroll
   for (int v = 0; v < 5; ++v) F[v] = 0.0;
@@ -99,9 +98,14 @@ __device__ __forceinline__ void face_curv(const NumDev& nd, const BCell<double>&
 #pragma unroll
     for (int v = 0; v < 5; ++v) F[v] = F[v] + s * Fu[v];
   }
-  __builtin_amdgcn_sched_barrier(0);
-  // viscous part (viscous.py:28-51): gradients at the face with the component along the
-  // centroid line corrected
+}
+
+// Viscous part (viscous.py:28-51): gradients at the face with the component along the centroid line
+// corrected.  V[0..2] the stress times the area, V[3] heat flux and work; dx the centroid
+// difference, gsum(i) the sum of component i of the two cells' gradient records.
+template <class GS>
+__device__ __forceinline__ void viscous_curv(const BCell<double>& L, const BCell<double>& Rc, GS gsum,
+                                             const double* dx, const double* S, double* V) {
   const double id = rsq64((dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2]);
   const double e[3] = {dx[0] * id, dx[1] * id, dx[2] * id};
   double gf[9];
@@ -126,15 +130,27 @@ __device__ __forceinline__ void face_curv(const NumDev& nd, const BCell<double>&
   const double td = (2.0 / 3.0) * ((gf[0] + gf[4]) + gf[8]);
   const double t00 = muf * ((gf[0] + gf[0]) - td), t11 = muf * ((gf[4] + gf[4]) - td), t22 = muf * ((gf[8] + gf[8]) - td);
   const double t01 = muf * (gf[1] + gf[3]), t02 = muf * (gf[2] + gf[6]), t12 = muf * (gf[5] + gf[7]);
-  const double ts[3] = {(t00 * S[0] + t01 * S[1]) + t02 * S[2], (t01 * S[0] + t11 * S[1]) + t12 * S[2],
-                        (t02 * S[0] + t12 * S[1]) + t22 * S[2]};
+  V[0] = (t00 * S[0] + t01 * S[1]) + t02 * S[2];
+  V[1] = (t01 * S[0] + t11 * S[1]) + t12 * S[2];
+  V[2] = (t02 * S[0] + t12 * S[1]) + t22 * S[2];
   double w = kf * dTdn;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    F[1 + c] = F[1 + c] - ts[c];
-    w = w + (0.5 * (L.u[c] + Rc.u[c])) * ts[c];
-  }
-  F[4] = F[4] - w;
+  for (int c = 0; c < 3; ++c) w = w + (0.5 * (L.u[c] + Rc.u[c])) * V[c];
+  V[3] = w;
+}
+
+// Numerical flux of a face: the viscous part after the inviscid one, so that the records it reads
+// are not held through that
+template <int SC, class GS>
+__device__ __forceinline__ void face_curv(const NumDev& nd, const BCell<double>& L2, const BCell<double>& L,
+                                          const BCell<double>& Rc, const BCell<double>& R2, double th, GS gsum,
+                                          const double* dx, const double* S, double* F) {
+  inviscid_curv<SC>(nd, L2, L, Rc, R2, th, S, F);
+  __builtin_amdgcn_sched_barrier(0);
+  double V[4];
+  viscous_curv(L, Rc, gsum, dx, S, V);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) F[1 + c] = F[1 + c] - V[c];
 }
 
 // A cell's metrics as the gradient reads them: lower and upper face vectors (S[2 d], S[2 d + 1]),
@@ -346,7 +362,11 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
   request(I0 - 1);
   stage_plane(arrive());
   request(I0);
-  double Cp[5], Xp[3];     // partial outward sum of the own cell I-1 (lower i face minus j / k faces); its centroid
+  // Lower i face of the own cell I-1, and its centroid.  The sum of its j / k faces waits in LDS: the
+  // difference of the two i faces is formed first, since a sum through either would round at the
+  // size of the flux (where the flow does not change along i, the j and k faces alone are the sum;
+  // in a laminar shear they are 1e-9 of the pressure).  In registers it would be spilled.
+  double Cp[5], Xp[3];
 #pragma unroll
   for (int v = 0; v < 5; ++v) Cp[v] = 0.0;
 #pragma unroll
@@ -393,13 +413,34 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
       }
       grad_curv(nd, o, u, m, p, rho, mu, put);
     };
-    // the own record waits in the thread's own slots of the exchange (free here) and in G[10..14]
-    // until the i face has read that of plane I-1
-    double G[NGC - 10] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    auto park = [&](int x) -> double& { return x < 5 ? sFj[x][tid] : (x < 10 ? sFk[x - 5][tid] : G[x - 10]); };
+    // The own record, and with it the viscous part of the own i face I-1/2 while its velocity
+    // gradients are in registers (the own slot still holds the record of plane I-1).  The
+    // temperature's gradient waits in the thread's own slots of the j exchange, the viscous part in
+    // the same slots until the inviscid part is there.
+    const bool iface = act && I >= I0;
+    const int iwall = iface ? wall_of(0, I) : -1;
     if (own_g) {
       const double mi[4] = {W1.u[0], W1.u[1], W1.u[2], W1.T}, pi[4] = {Pn.u[0], Pn.u[1], Pn.u[2], Pn.T};
-      grads(geo, mi, pi, sp_own, sP[0][sp_own], mu0, [&](int x, double g) { park(x) = g; });
+      double g[9], m[3];
+      grads(geo, mi, pi, sp_own, sP[0][sp_own], mu0, [&](int x, double q) {
+        if (x < 9) g[x] = q;
+        else if (x < 12) sFj[x - 9][tid] = q;
+        else m[x - 12] = q;
+      });
+      __builtin_amdgcn_sched_barrier(0);
+      double V[4] = {0.0, 0.0, 0.0, 0.0}, th = 0.0;
+      if (iface && iwall < 0) {
+        const double dx[3] = {Xc[0] - Xp[0], Xc[1] - Xp[1], Xc[2] - Xp[2]};
+        viscous_curv(W1, cell(sp_own), [&](int x) {
+          return sG[x][sg_own] + (x < 9 ? g[x] : x < 12 ? sFj[x - 9][tid] : m[x - 12]);
+        }, dx, geo.S[0], V);
+        th = fmax(sG[14][sg_own], m[2]);
+      }
+#pragma unroll
+      for (int v = 0; v < NGC; ++v) sG[v][sg_own] = v < 9 ? g[v] : v < 12 ? sFj[v - 9][tid] : m[v - 12];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sFj[v][tid] = V[v];
+      sFj[4][tid] = th;
     }
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
@@ -407,14 +448,13 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
     double Fin[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) Fin[v] = 0.0;
-    if (act && I >= I0) {
-      const int side = wall_of(0, I);
-      if (side >= 0) {
-        wall_flux(0, side, I, J, K, Fin);
-      } else {                                   // (the own slot still holds the record of plane I-1)
-        const double dx[3] = {Xc[0] - Xp[0], Xc[1] - Xp[1], Xc[2] - Xp[2]};
-        auto gsum = [&](int x) { return sG[x][sg_own] + park(x); };
-        face_curv<SC>(nd, W0, W1, cell(sp_own), Pn, sG[14][sg_own], G[4], gsum, dx, geo.S[0], Fin);
+    if (iface) {
+      if (iwall >= 0) {
+        wall_flux(0, iwall, I, J, K, Fin);
+      } else {
+        inviscid_curv<SC>(nd, W0, W1, cell(sp_own), Pn, sFj[4][tid], geo.S[0], Fin);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Fin[1 + v] = Fin[1 + v] - sFj[v][tid];
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -432,10 +472,6 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
         for (int v = 0; v < 5; ++v) vz[v] = ldu(qz + v * (size_t)cells, c);
       }
     }
-    if (own_g) {
-#pragma unroll
-      for (int v = 0; v < NGC; ++v) sG[v][sg_own] = park(v);
-    }
     __builtin_amdgcn_sched_barrier(0);
     if (MODE >= 2 && fin) {
 #pragma unroll
@@ -445,7 +481,7 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
       const double ivol = hiv_p + hiv_p;
       double r[5];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) r[v] = (Cp[v] - Fin[v]) * ivol;
+      for (int v = 0; v < 5; ++v) r[v] = ((Cp[v] - Fin[v]) - sFk[v][kface_slot(tj, tk)]) * ivol;
       if (nd.n_sponge > 0) {                     // SmoothRampSponge, smooth_ramp.py:212-221
         const double xcv = ldu(B.xc, c);
         const long long mrow = (long long)(I - 1 - ng) * n1 + (J - ng);
@@ -509,7 +545,7 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
           const double dx[3] = {Xp[0] - xj[0], Xp[1] - xj[1], Xp[2] - xj[2]};
           auto gsum = [&](int x) { return sG[x][sg_own - G2K] + sG[x][sg_own]; };
           face_curv<SC>(nd, cell(sp_own - 2 * H2K), cell(sp_own - H2K), cell(sp_own), cell(sp_own + H2K),
-                        sG[14][sg_own - G2K], sG[14][sg_own], gsum, dx, Sj, F);
+                        fmax(sG[14][sg_own - G2K], sG[14][sg_own]), gsum, dx, Sj, F);
         }
 #pragma unroll
         for (int v = 0; v < 5; ++v) sFj[v][tid] = F[v];
@@ -529,7 +565,7 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
           const int sp = (rj + 2) * H2K + (rk + 2), sg = (rj + 1) * G2K + (rk + 1);
           const double dx[3] = {xr[0] - xk[0], xr[1] - xk[1], xr[2] - xk[2]};
           auto gsum = [&](int x) { return sG[x][sg - 1] + sG[x][sg]; };
-          face_curv<SC>(nd, cell(sp - 2), cell(sp - 1), cell(sp), cell(sp + 1), sG[14][sg - 1], sG[14][sg], gsum, dx, Sk, F);
+          face_curv<SC>(nd, cell(sp - 2), cell(sp - 1), cell(sp), cell(sp + 1), fmax(sG[14][sg - 1], sG[14][sg]), gsum, dx, Sk, F);
         }
         const int slot = kface_slot(rj, rk);
 #pragma unroll
@@ -549,12 +585,17 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
     if (own_p) W1 = cell(sp_own);
     stage_plane(Pn);
     request(I + 2);
-    // ---- carry: the partial outward sum of the own cell I
+    // ---- carry: the lower i face of the own cell I; the sum of its j / k faces takes the own k
+    //      face's slot, whose other reader is the row's lane before: in this wavefront, and the sum
+    //      that is stored needs the load that reads it
     if (act && inner) {
-      const int jup = tile_tid(tj + 1, tk), kup = kface_slot(tj, tk + 1);
+      const int jup = tile_tid(tj + 1, tk), kown = kface_slot(tj, tk), kup = kface_slot(tj, tk + 1);
 #pragma unroll
-      for (int v = 0; v < 5; ++v)
-        Cp[v] = Fin[v] - ((sFj[v][jup] - sFj[v][tid]) + (sFk[v][kup] - sFk[v][tid]));
+      for (int v = 0; v < 5; ++v) {
+        const double d = (sFj[v][jup] - sFj[v][tid]) + (sFk[v][kup] - sFk[v][kown]);
+        Cp[v] = Fin[v];
+        sFk[v][kown] = d;
+      }
     }
     __syncthreads();                             // plane I+1 staged
   }
