@@ -69,7 +69,9 @@ struct GB {
 };
 
 // Kennedy-Gruber flux of order 2 / 4 as pair sums (kep_pairs_f32) across a face of normal D:
-// the mass flux is k[0] F[0], the others k[1] F[1..4].
+// the mass flux is k[0] F[0], the others k[1] F[1..4].  FP64 of order 4 takes the factors into the
+// combination (1/6 of the inner pair, 1/48 of the outer ones): a factor after it would round the
+// pressure-sized sum once more.
 template <int D, int ORDER, class R>
 __device__ __forceinline__ void kep_axis(const BCell<R>& L2, const BCell<R>& L, const BCell<R>& Rc,
                                          const BCell<R>& R2, R S, R* F, R* un4, R* k) {
@@ -100,10 +102,17 @@ __device__ __forceinline__ void kep_axis(const BCell<R>& L2, const BCell<R>& L, 
   pair(L, Rc, A, &sr, &w);
   pair(L, R2, Aa, &sra, &wa);
   pair(L2, Rc, Ab, &srb, &wb);
+  *un4 = fm(R(8), w, -(wa + wb)) * R(1.0 / 12.0);
+  if constexpr (sizeof(R) == 8) {
+    F[0] = fm(R(1.0 / 3.0), A[0], -((Aa[0] + Ab[0]) * R(1.0 / 24.0)));
+#pragma unroll
+    for (int c = 1; c < 5; ++c) F[c] = fm(R(1.0 / 6.0), A[c], -((Aa[c] + Ab[c]) * R(1.0 / 48.0)));
+    k[0] = k[1] = R(1);
+    return;
+  }
   F[0] = fm(R(8), A[0], -fm(sra, wa, Ab[0]));
 #pragma unroll
   for (int c = 1; c < 5; ++c) F[c] = fm(R(8), A[c], -(Aa[c] + Ab[c]));
-  *un4 = fm(R(8), w, -(wa + wb)) * R(1.0 / 12.0);
   k[0] = R(1.0 / 24.0);
   k[1] = R(1.0 / 48.0);
 }
@@ -197,7 +206,13 @@ __device__ __forceinline__ void upwind_axis(R gamma, int limiter, const BCell<R>
   R u[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) u[c] = left ? wl[1 + c] : wr[1 + c];
-  const R E = fm(p, fdiv<R>(R(1), gamma - R(1.0)), (h * r) * fm(u[2], u[2], fm(u[0], u[0], u[1] * u[1])));
+  // (a / b + c: FP32 as the multiply-add of the reciprocal that the compiler forms, FP64 the quotient)
+  auto div_add = [](R a, R b, R c) {
+#pragma clang fp contract(off)
+    return sizeof(R) == 4 ? fm(a, fdiv<R>(R(1), b), c) : fdiv<R>(a, b) + c;
+  };
+  const R kin = fm(u[2], u[2], fm(u[0], u[0], u[1] * u[1]));
+  const R E = sizeof(R) == 4 ? div_add(p, gamma - R(1.0), (h * r) * kin) : fm(h * r, kin, fdiv<R>(p, gamma - R(1.0)));
   R G[5];
   G[0] = r * un;
 #pragma unroll
@@ -205,9 +220,9 @@ __device__ __forceinline__ void upwind_axis(R gamma, int limiter, const BCell<R>
   G[4] = (E + p) * un;
   if (left ? sL < R(0) : sR > R(0)) {           // a star state lies on the face
     const R a = r * (s - un), d = ss - un, is = fdiv<R>(R(1), s - ss);
-    const R f = a * is;
-    const R e = fm(E, fdiv<R>(R(1), r), d * fm(p, fdiv<R>(R(1), a), ss));
-    G[0] = fm(s, fm(a, is, -r), G[0]);
+    const R f = sizeof(R) == 4 ? a * is : fdiv<R>(a, s - ss);
+    const R ed = div_add(p, a, ss), e = sizeof(R) == 4 ? div_add(E, r, d * ed) : fm(d, ed, fdiv<R>(E, r));
+    G[0] = fm(s, sizeof(R) == 4 ? fm(a, is, -r) : f - r, G[0]);
 #pragma unroll
     for (int c = 0; c < 3; ++c) G[1 + c] = fm(s, fm(f, c == D ? fm(d, n, u[c]) : u[c], -(r * u[c])), G[1 + c]);
     G[4] = fm(s, fm(f, e, -E), G[4]);

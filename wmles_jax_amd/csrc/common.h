@@ -402,22 +402,21 @@ __device__ __forceinline__ void rec32_store(float* Pb, size_t cells, size_t c, c
   st4(Pb + 4 * (cells + c), make_float4(b[0], b[1], b[2], b[3]));
 }
 
-// The same record in FP64, without gauge (box kernels): one reciprocal of rho, within an ulp
-// or two of k_prim's divisions.
+// The same record in FP64, without gauge: cons_to_prim's and mu_suth's quotients, the five by rho
+// and its multiples from one reciprocal (quot64), so the bits of the divisions.
 __device__ __forceinline__ void rec_of(const NumDev& nd, const double* q, double, double, double, double* a,
                                        double* b) {
 #pragma clang fp contract(off)
+  const GasC& g = nd.gas;
   const RecC& rc = nd.rc;
-  const double r = q[0];
-  const double ir = rcp64(r);
-  a[0] = q[1] * ir; a[1] = q[2] * ir; a[2] = q[3] * ir;
+  const double r = q[0], y = rcp_step64(r);
+  a[0] = quot64(q[1], r, y); a[1] = quot64(q[2], r, y); a[2] = quot64(q[3], r, y);
   const double k = (a[0] * a[0] + a[1] * a[1]) + a[2] * a[2];
-  const double p = (nd.gas.gamma - 1.0) * (q[4] - (0.5 * r) * k);
-  const double pr = p * ir;
-  const double T = pr * rc.iR, t = T * rc.iTref64;
+  const double p = (g.gamma - 1.0) * (q[4] - (0.5 * r) * k);
+  const double T = quot64(p, r * g.R, y * rc.iR), t = quot64(T, g.T_ref, rc.iTref64);
   a[3] = T;
-  b[0] = r; b[1] = p; b[3] = pr * rc.igm1;
-  b[2] = (rc.muc64 * (t * sqrt(t))) * rcp64(T + nd.gas.S_suth);
+  b[0] = r; b[1] = p; b[3] = quot64(p, (g.gamma - 1.0) * r, y * rc.igm1);
+  b[2] = fdiv<double>((g.mu_ref * (t * fsqrt<double>(t))) * (g.T_ref + g.S_suth), T + g.S_suth);
 }
 
 // SmoothRampSponge weight at a cell centre x (smooth_ramp.py:212-221); pr = (x_start_l,

@@ -25,13 +25,6 @@ namespace {
 constexpr int NGC = 15;                        // g[12], mu_eff, k_eff, theta
 constexpr int GCS = (G2J - 1) * G2K + G2K;     // gradient slots (17 x 18)
 
-// 1 / sqrt(x) within an ulp or two: the hardware estimate and two Newton steps
-__device__ __forceinline__ double rsq64(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y + (0.5 * y) * (1.0 - (x * y) * y);
-  return y + (0.5 * y) * (1.0 - (x * y) * y);
-}
-
 // Kennedy-Gruber flux of order 2 / 4 as pair sums (kep_pairs_f32 in FP64; E = e + |u|^2 / 2)
 template <int ORDER>
 __device__ __forceinline__ void kep_curv(const BCell<double>& L2, const BCell<double>& L, const BCell<double>& Rc,
@@ -58,9 +51,9 @@ __device__ __forceinline__ void kep_curv(const BCell<double>& L2, const BCell<do
   double Aa[5], Ab[5];
   pair(L, R2, Aa);
   pair(L2, Rc, Ab);
-  F[0] = (8.0 * A[0] - (Aa[0] + Ab[0])) * (1.0 / 24.0);
+  F[0] = (1.0 / 3.0) * A[0] - (Aa[0] + Ab[0]) * (1.0 / 24.0);
 #pragma unroll
-  for (int v = 1; v < 5; ++v) F[v] = (8.0 * A[v] - (Aa[v] + Ab[v])) * (1.0 / 48.0);
+  for (int v = 1; v < 5; ++v) F[v] = (1.0 / 6.0) * A[v] - (Aa[v] + Ab[v]) * (1.0 / 48.0);
 }
 
 __device__ __forceinline__ CellWT<double> cell_wt(const BCell<double>& c) {
@@ -106,7 +99,7 @@ __device__ __forceinline__ void inviscid_curv(const NumDev& nd, const BCell<doub
 template <class GS>
 __device__ __forceinline__ void viscous_curv(const BCell<double>& L, const BCell<double>& Rc, GS gsum,
                                              const double* dx, const double* S, double* V) {
-  const double id = rsq64((dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2]);
+  const double id = fdiv<double>(1.0, fsqrt<double>((dx[0] * dx[0] + dx[1] * dx[1]) + dx[2] * dx[2]));
   const double e[3] = {dx[0] * id, dx[1] * id, dx[2] * id};
   double gf[9];
 #pragma unroll

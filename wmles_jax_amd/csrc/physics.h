@@ -114,17 +114,33 @@ WMX_HD void bc_farfield(const GasC& g, const double* src, const double* pinf, do
 // instructions instead of eleven and seventeen: a third of the FP64 face kernels' issue was
 // IEEE divisions (box launch of 256 x 128 x 128 cells, Hybrid + Vreman: 458 -> 424 us).  Four
 // million quotients and roots of random operands over 60 decades equalled the IEEE ones.
+// The reciprocal of b after its Newton step, and a / b from it: several quotients by one divisor share
+// the first, and a rounded multiple of it serves that multiple of b.
+WMX_HD double rcp_step64(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma clang fp contract(off)
+  const double y = __builtin_amdgcn_rcp(b);
+  return __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+#else
+  return 1.0 / b;
+#endif
+}
+WMX_HD double quot64(double a, double b, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma clang fp contract(off)
+  const double q = a * y;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
+#else
+  return a / b;
+#endif
+}
 template <class R>
 WMX_HD R fdiv(R a, R b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   if constexpr (sizeof(R) == 4) {
     return a * __builtin_amdgcn_rcpf(b);         // (its product contracts with what follows it)
   } else {
-#pragma clang fp contract(off)
-    double y = __builtin_amdgcn_rcp(b);
-    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
-    const double q = a * y;
-    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
+    return quot64(a, b, rcp_step64(b));
   }
 #else
   return a / b;
