@@ -1,8 +1,9 @@
-"""Rounding of the FP64 right-hand sides: their distance from the oracle evaluated in long double (80
-bits) on the same stored nodes and states, as the rms over the block relative to the rms of the
-value.  FORMER holds what the kernels that formed every record with divisions, each central flux
-with one factor a pair and each cell's sum face by face measured here, with 2% for the last digit
-printed: arithmetic that replaces theirs rounds no more."""
+"""Rounding of the FP64 right-hand sides and steps: their distance from the oracle evaluated in long
+double (80 bits) on the same stored nodes and states, as the rms over the block relative to the rms
+of the value.  FORMER and FORMER_STEP hold what the kernels measured here that formed every record
+with divisions, each central flux with one factor a pair, each cell's sum face by face and each
+stage as a0 q0 + a1 (q + dt r), with 2% for the last digit printed: arithmetic that replaces theirs
+rounds no more."""
 import numpy as np
 import pytest
 
@@ -32,6 +33,15 @@ FORMER = {("box", "hybrid"): (3.33e-15, 1.85e-14, 3.05e-14, 2.97e-14, 3.01e-15),
           ("curvilinear", "kep"): (2.78e-15, 2.44e-14, 9.15e-14, 1.32e-13, 2.82e-15),
           ("curvilinear", "muscl"): (1.49e-14, 9.33e-15, 8.58e-15, 9.01e-15, 1.30e-14),
           ("curvilinear", "keep"): (2.36e-15, 3.20e-14, 6.48e-14, 1.24e-13, 2.39e-15)}
+# the state after one step of 1e-6 s (rounding of the stages; one seed)
+FORMER_STEP = {("box", "hybrid"): (8.137e-17, 7.493e-17, 1.388e-16, 1.083e-16, 5.842e-17),
+               ("box", "kep"): (8.144e-17, 7.475e-17, 1.394e-16, 1.085e-16, 5.826e-17),
+               ("box", "muscl"): (8.119e-17, 7.457e-17, 1.020e-16, 9.848e-17, 5.774e-17),
+               ("box", "keep"): (8.127e-17, 7.481e-17, 1.081e-16, 1.052e-16, 5.822e-17),
+               ("curvilinear", "hybrid"): (8.139e-17, 7.553e-17, 1.554e-16, 1.258e-16, 5.808e-17),
+               ("curvilinear", "kep"): (8.136e-17, 7.507e-17, 1.559e-16, 1.255e-16, 5.824e-17),
+               ("curvilinear", "muscl"): (8.089e-17, 7.515e-17, 1.183e-16, 1.217e-16, 5.790e-17),
+               ("curvilinear", "keep"): (8.156e-17, 7.522e-17, 1.192e-16, 1.222e-16, 5.830e-17)}
 
 
 def in_long_double(solver):
@@ -43,8 +53,8 @@ def in_long_double(solver):
     return solver
 
 
-@pytest.mark.parametrize("form,name", list(FORMER))
-def test_right_hand_sides_round_no_more_than_before(form, name):
+def build(form, name):
+    """(block, solver, long double oracle, noisy state by seed)."""
     n, scheme, sgs = CASES[name]
     spec, arrays = box_spec(n, (None, SLIP, None), scheme, sgs)
     if form == "curvilinear":
@@ -55,12 +65,31 @@ def test_right_hand_sides_round_no_more_than_before(form, name):
     mesh, sol = cases.build(wmx, spec, arrays)
     assert sol.kernel_form() == form
     ref = in_long_double(cases.build(oracle, spec, arrays)[1])
-    blk, err = mesh.blocks[0], np.zeros(5)
-    for seed in range(3):
-        Q = cases.interior_noise(mesh.blocks, [np.asarray(q.cpu()) for q in sol.init_state(cases.prim_fn)], seed,
-                                 amp=0.05)
-        got = blk.interior(sol.rhs(Q)[0].cpu().numpy())
-        want = blk.interior(ref.rhs([np.asarray(q, np.longdouble) for q in Q])[0])
-        assert want.dtype == np.longdouble
-        err += np.sqrt(((got - want) ** 2).mean(axis=(1, 2, 3)) / (want ** 2).mean(axis=(1, 2, 3))).astype(float) / 3
+    q0 = [np.asarray(q.cpu()) for q in sol.init_state(cases.prim_fn)]
+    return mesh.blocks[0], sol, ref, lambda seed: cases.interior_noise(mesh.blocks, q0, seed, amp=0.05)
+
+
+def rms_error(got, want):
+    assert want.dtype == np.longdouble
+    return np.sqrt(((got - want) ** 2).mean(axis=(1, 2, 3)) / (want ** 2).mean(axis=(1, 2, 3))).astype(float)
+
+
+def wide(Q):
+    return [np.asarray(q, np.longdouble) for q in Q]
+
+
+@pytest.mark.parametrize("form,name", list(FORMER))
+def test_right_hand_sides_round_no_more_than_before(form, name):
+    blk, sol, ref, noisy = build(form, name)
+    err = np.mean([rms_error(blk.interior(sol.rhs(Q)[0].cpu().numpy()), blk.interior(ref.rhs(wide(Q))[0]))
+                   for Q in map(noisy, range(3))], axis=0)
     assert np.all(err <= 1.02 * np.array(FORMER[form, name])), err
+
+
+@pytest.mark.parametrize("form,name", list(FORMER_STEP))
+def test_steps_round_no_more_than_before(form, name):
+    blk, sol, ref, noisy = build(form, name)
+    Q = noisy(0)
+    err = rms_error(blk.interior(sol.advance(Q, 1e-6)[0].cpu().numpy()),
+                    blk.interior(ref.advance(wide(Q), np.longdouble(1e-6))[0]))
+    assert np.all(err <= 1.02 * np.array(FORMER_STEP[form, name])), err

@@ -618,7 +618,8 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     __builtin_amdgcn_sched_barrier(0);
     // ---- cell I-1: its state loads go out first, covered by the gradients and the i face
     const unsigned c = (unsigned)(I - 1) * sI + (unsigned)J * N[2] + K;
-    // the stage is base + a1 dt r with base = a0 q0 + a1 q: one value per component is kept
+    // the stage is a0 q0 + a1 (q + dt r).  FP32 keeps one value per component, base = a0 q0 + a1 q,
+    // and adds a1 dt r; FP64, where the state's roundings are its largest, keeps q and parks q0
     const double a0 = MODE == 2 ? 0.75 : 1.0 / 3.0, a1 = MODE == 1 ? 1.0 : (MODE == 2 ? 0.25 : 2.0 / 3.0);
     double base[5], vz[5];
     if (MODE >= 1 && fin) {
@@ -665,7 +666,10 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
     // ---- own i face I-1/2, which completes cell I-1
     if (MODE >= 2 && fin) {
 #pragma unroll
-      for (int v = 0; v < 5; ++v) base[v] = fm(a0, vz[v], a1 * base[v]);
+      for (int v = 0; v < 5; ++v) {
+        if (F32) base[v] = fm(a0, vz[v], a1 * base[v]);
+        else sFj[v][tid] = (R)vz[v];             // (own slot: free until the plane's j faces)
+      }
     }
     R Fin[6];
 #pragma unroll
@@ -717,7 +721,12 @@ __device__ __forceinline__ void box_tile(const BlockDev* __restrict__ blks, cons
       }
       double* o = out.p[t.x];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) stu(o + v * (size_t)cells, c, MODE == 0 ? r[v] : fm(a1 * dt, r[v], base[v]));
+      for (int v = 0; v < 5; ++v) {
+        double w = MODE == 0 ? r[v] : fm(F32 ? a1 * dt : dt, r[v], base[v]);
+        if (!F32 && MODE == 2) w = fm(a0, (double)sFj[v][tid], a1 * w);      // (a1 w is exact)
+        if (!F32 && MODE == 3) w = fm(a1, w, a0 * (double)sFj[v][tid]);
+        stu(o + v * (size_t)cells, c, w);
+      }
     }
     if (I == Iend) break;
     __builtin_amdgcn_sched_barrier(0);

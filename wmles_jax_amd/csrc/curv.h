@@ -453,8 +453,8 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
     __builtin_amdgcn_sched_barrier(0);
     // ---- cell I-1: its state loads covered by the i face
     const unsigned c = (unsigned)(I - 1) * sI + (unsigned)J * N[2] + K;
-    // the stage is base + a1 dt r with base = a0 q0 + a1 q: one value per component is kept
-    const double a0 = MODE == 2 ? 0.75 : 1.0 / 3.0, a1 = MODE == 1 ? 1.0 : (MODE == 2 ? 0.25 : 2.0 / 3.0);
+    // the stage is a0 q0 + a1 (q + dt r)
+    const double a0 = MODE == 2 ? 0.75 : 1.0 / 3.0, a1 = MODE == 2 ? 0.25 : 2.0 / 3.0;
     double base[5], vz[5];
     if (MODE >= 1 && fin) {
 #pragma unroll
@@ -466,10 +466,6 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (MODE >= 2 && fin) {
-#pragma unroll
-      for (int v = 0; v < 5; ++v) base[v] = a0 * vz[v] + a1 * base[v];
-    }
     if (fin) {
       const double ivol = hiv_p + hiv_p;
       double r[5];
@@ -490,7 +486,12 @@ __device__ __forceinline__ void curv_tile(const BlockDev* __restrict__ blks, con
       }
       double* o = out.p[t.x];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) stu(o + v * (size_t)cells, c, MODE == 0 ? r[v] : base[v] + (a1 * dt) * r[v]);
+      for (int v = 0; v < 5; ++v) {
+        double w = MODE == 0 ? r[v] : __builtin_fma(dt, r[v], base[v]);
+        if (MODE == 2) w = __builtin_fma(a0, vz[v], a1 * w);                 // (a1 w is exact)
+        if (MODE == 3) w = __builtin_fma(a1, w, a0 * vz[v]);
+        stu(o + v * (size_t)cells, c, w);
+      }
     }
     if (I == Iend) break;
     __builtin_amdgcn_sched_barrier(0);
