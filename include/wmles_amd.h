@@ -185,7 +185,17 @@ int wmx_plan_set_case_gauge(wmx_plan* plan, int32_t case_id, double p_ref, doubl
    brackets every later
    launch of a class whose bit is set in `mask` with hipEvents on the launch stream
    (mask 0 stops and clears); wmx_plan_profile_read synchronises the recorded events
-   and returns per-class summed milliseconds and launch counts (10 entries each). */
+   and returns per-class summed milliseconds and launch counts (10 entries each).
+   A launch that carries several kinds of work counts under one class:
+   - WMX_FORM_BOX and WMX_FORM_CURV stages: class 3 holds the ghost fills and, in the stage's
+     first launches, the Newton wall faces, the sponge means (rows of 9..129 cells) and the CFL
+     partials and mins of wmx_step; classes 1 and 2 are empty;
+   - WMX_FORM_FUSED stages: class 2 holds the Newton wall faces, those sponge means and the CFL
+     partials, class 1 the CFL mins;
+   - WMX_FORM_SPLIT stages: class 2 holds those sponge means and the CFL partials, class 1 the
+     Newton wall faces and the CFL mins.
+   Class 4 is then the learned wall model's launch, class 5 wmx_max_dt (and a min that no later
+   launch of the stage could take), class 9 the means of other rows. */
 int wmx_plan_profile(wmx_plan* plan, int32_t mask);
 int wmx_plan_profile_read(wmx_plan* plan, double* ms, int32_t* counts);
 

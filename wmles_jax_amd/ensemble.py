@@ -189,7 +189,8 @@ class EnsembleSolver:
 
     def profile(self, classes=("flux",)):
         """Start HIP-event timing of the named kernel classes (empty: stop).  Launches
-        replayed from a captured graph are not timed."""
+        replayed from a captured graph are not timed.  A launch that carries several kinds of
+        work counts once (Solver.profile)."""
         mask = 0
         for c in classes:
             mask |= 1 << self.KERNEL_CLASSES.index(c)

@@ -251,7 +251,10 @@ class Solver:
     KERNEL_CLASSES = ("flux", "grad", "prim", "fill", "wall", "dt", "massflux", "shell", "inflow", "sponge")
 
     def profile(self, classes=("flux",)):
-        """Start event timing of the named kernel classes (empty: stop)."""
+        """Start event timing of the named kernel classes (empty: stop).  A launch that carries
+        several kinds of work counts once: "fill" holds the Newton wall faces, sponge means and
+        CFL partials of box and FP64 plans, "prim" and "grad" those of the others
+        (include/wmles_amd.h)."""
         mask = 0
         for c in classes:
             mask |= 1 << self.KERNEL_CLASSES.index(c)
