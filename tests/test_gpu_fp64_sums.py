@@ -1,6 +1,6 @@
 """FP64 outward sums where the flow does not change along i: the two i faces of a cell carry the same
 pressure-sized flux, and what is left of the x momentum is the viscous force, 1e-9 of it.  Summed
-through the pressure it would keep six digits; the bar is the form's 1e-12."""
+through the pressure it would keep eight digits; the bar is the form's 1e-12."""
 import numpy as np
 import pytest
 

@@ -17,14 +17,16 @@
 // One body for both arithmetic forms (R = float: FP32-bulk records in gauge form with the
 // FP64 epilogue of flux2.h; R = double: the plain form's eight record planes).  Contraction
 // is off in the functions below and the fused multiply-adds are written out, so every
-// instance (kernel, mode, scheme, persistent stage) rounds the same way.
+// instance (kernel, mode, scheme, persistent stage) rounds the same way.  FP64 divides, scales and
+// sums so that it rounds no more than a form with a division per quotient and each face's flux
+// summed by itself; FP32, whose fluxes are 1e-7, takes the cheaper forms.
 //
 // The state is read, not a primitive record: each thread forms the records of its column and
 // of a halo cell one plane ahead (rec_of), so no primitive launch writes 32 / 64 B per cell for
-// this one to read back with a halo.  Channel of 256 x 128 x 128 cells, Hybrid + Vreman, per
-// stage: FP32 271 us against 253 us on records and 78 us that wrote them; FP64 423 us against
-// 461 us + 137 us.  It is bound by vector issue (86% of the
-// FP32 launch's cycles, 67% of the lanes active: the Hybrid's upwind branch).
+// this one to read back with a halo.  Channel of 256 x 128 x 128 cells, Hybrid + Vreman, mean of the
+// three stages by events: FP32 274 us against 253 us on records and 78 us that wrote them; FP64
+// 427 us against 461 us + 137 us (a kernel trace reads 282 and 444).  It is bound by vector issue
+// (86% of the FP32 launch's cycles, 67% of the lanes active: the Hybrid's upwind branch).
 //
 // March.  At plane I the tile evaluates the gradient records of plane I, the own i face I-1/2,
 // which completes cell I-1, and then the j / k faces of plane I.  The records of planes I-1 and

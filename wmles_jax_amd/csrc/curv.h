@@ -10,9 +10,9 @@
 // plane before is kept in registers.  Per plane and column 19 geometry words are read for the
 // gradients, requested before the records of the next plane are formed; the lower face vectors
 // among them serve the i face.  Bound by the latency of the state and geometry loads and by FP64
-// issue at two waves per SIMD.  190 x 63 x 33 ramp, Hybrid + Vreman: 128 us per stage (114 in
+// issue at two waves per SIMD.  190 x 63 x 33 ramp, Hybrid + Vreman: 134 us per stage (125 in
 // stage 1) where primitive, gradient and flux launches on stored records took 12 + 28 + 131;
-// 128 x 72 x 56 skewed box, MUSCL + Smagorinsky: 110 us, was 13 + 37 + 132.  Every spilled
+// 128 x 72 x 56 skewed box, MUSCL + Smagorinsky: 113 us, was 13 + 37 + 132.  Every spilled
 // register costs twice, since its reload waits for all loads issued before it: with 127 of them
 // the ramp's stage took 182 us.
 #pragma once

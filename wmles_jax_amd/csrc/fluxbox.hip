@@ -6,9 +6,9 @@ namespace wmx {
 
 // Occupancy: FP32 161 VGPRs and 52.9 KB of LDS, three workgroups per CU; FP64 256 VGPRs and
 // 77 KB, two.  Measured per launch on the 256 x 128 x 128 channel (Hybrid KEP4 + MUSCL-HLLC,
-// Vreman): FP32 461 us + 78 us of primitive launch with the general fused kernel, 271 us here;
-// FP64 920 us + 300 us of gradient launch + 137 us, 423 us here.  VALU issue and the latency of
-// three dependent LDS phases per plane bound both; HBM does not.
+// Vreman; events, mean of the stages): FP32 461 us + 78 us of primitive launch with the general
+// fused kernel, 274 us here; FP64 920 us + 300 us of gradient launch + 137 us, 427 us here.  VALU
+// issue and the latency of three dependent LDS phases per plane bound both; HBM does not.
 template <class R, int MODE, int SC>
 __global__ __launch_bounds__(256, sizeof(R) == 4 ? 3 : 2) void k_box(
     const BlockDev* __restrict__ blks, const int4* __restrict__ tiles, int ci_len, NumDev nd, Ptrs qin, Ptrs q0,
