@@ -79,6 +79,8 @@ struct wmx_plan {
   bool has_external = false;          // some face is WMX_BC_EXTERNAL: the caller runs the sweep
   bool fuse_last = false;   // the last phase is k-face fills only: a step's primitive launches
                             // evaluate those ghosts (BlockDev::zfuse) and skip its fill launch
+  std::vector<int> fuse_sides;        // ... the sides of each block that could be (empty: none)
+  bool fuse_image = true;             // ... all of them plain periodic faces of their own block
   // sponge row means in head workgroups of the primitive launch (every block's rows of
   // 9..129 cells): per-block first workgroup, 32 rows each
   std::vector<int> sponge_pre;
@@ -381,6 +383,21 @@ int auto_ci_len(int nb, const int* dims, int prec, int cu_count, long long* ntil
 // every FP64 plan (box.h where its blocks' metrics are tensor products, else curv.h), and an
 // FP32-bulk plan of box blocks that evaluates its gradients in the march (box.h).
 bool direct(const wmx_plan* p) { return p->nd.prec != WMX_PREC_FP32_BULK || (p->box && p->fuse_grad); }
+
+// Whether a step leaves the sweep's last phase to the kernels of its stages (the primitive kernel
+// evaluates any such ghost; the kernels that read the state read a k ghost at its periodic image,
+// so there a side that is no plain periodic face of its own block is filled by a launch).  True
+// where that changed BlockDev::zfuse.
+bool choose_fusion(wmx_plan* p) {
+  p->fuse_last = !p->fuse_sides.empty() && (!direct(p) || p->fuse_image);
+  bool changed = false;
+  for (int b = 0; b < p->nb; ++b) {
+    const int z = p->fuse_last ? p->fuse_sides[b] : 0;
+    changed = changed || p->hb[b].zfuse != z;
+    p->hb[b].zfuse = z;
+  }
+  return changed;
+}
 
 // i-planes per tile of the kernels that read the state when none is requested.  W workgroups share a CU (3 in
 // FP32, 2 in FP64), so T tiles are r full rounds of W CUs slots and a remainder.  A full round
@@ -823,10 +840,17 @@ int wmx_plan_create(int32_t nblocks, const wmx_block_desc* blocks, const wmx_num
         for (int e = 0; ok && e < p->phase_off[nph - 1]; ++e)
           if (p->ops[e].axis == 2 && p->ops[e].blk == op.blk && p->ops[e].side == op.side) ok = false;
       }
-    p->fuse_last = ok;
-    if (ok)
-      for (int o = p->phase_off[nph - 1]; o < p->phase_off[nph]; ++o)
-        p->hb[p->ops[o].blk].zfuse |= 1 << p->ops[o].side;
+    if (ok) {
+      p->fuse_sides.assign(nblocks, 0);
+      for (int o = p->phase_off[nph - 1]; o < p->phase_off[nph]; ++o) {
+        const GhostOp& op = p->ops[o];
+        const wmx_face_desc& f = p->hb[op.blk].faces[4 + op.side];
+        p->fuse_sides[op.blk] |= 1 << op.side;
+        p->fuse_image = p->fuse_image && f.kind == WMX_FACE_INTERFACE && f.nb == op.blk && f.src_axis == 2 &&
+                        f.src_side == 1 - op.side && f.mapping[0] == 0 && f.mapping[1] == 1 && !f.flip[0] && !f.flip[1];
+      }
+    }
+    choose_fusion(p);
   }
   // wall faces
   for (int b = 0; b < nblocks; ++b)
@@ -1052,20 +1076,7 @@ int wmx_plan_bind_workspace(wmx_plan* p, void* ws, size_t bytes) {
     // (half reciprocal volumes and filter widths of the curvilinear FP64 kernel)
     if (!p->box && p->nd.prec != WMX_PREC_FP32_BULK)
       for (int b = 0; b < p->nb; ++b) WMX_CHECK(launch_curv_geo(p->hb[b], nullptr));
-    // the kernels that read the state read a fused side's k ghosts at their periodic images: a
-    // side that is no plain periodic face of its own block is filled by a launch
-    bool image = true;
-    for (int b = 0; b < p->nb; ++b)
-      for (int sd = 0; sd < 2; ++sd)
-        if ((p->hb[b].zfuse >> sd) & 1) {
-          const wmx_face_desc& f = p->hb[b].faces[4 + sd];
-          image = image && f.kind == WMX_FACE_INTERFACE && f.nb == b && f.src_axis == 2 && f.src_side == 1 - sd &&
-                  f.mapping[0] == 0 && f.mapping[1] == 1 && !f.flip[0] && !f.flip[1];
-        }
-    if ((p->box || p->nd.prec != WMX_PREC_FP32_BULK) && !image) {
-      p->fuse_last = false;
-      for (BlockDev& B : p->hb) B.zfuse = 0;
-    }
+    choose_fusion(p);
     drop_graphs(p);                              // (captured steps hold the tile table and the workspace)
     if (retile(p)) return 1;
     for (int b = 0; b < p->nb; ++b)
@@ -1561,6 +1572,11 @@ int wmx_plan_set_tiling(wmx_plan* p, int32_t ci_len, int32_t order) {
 int wmx_plan_set_fused_gradients(wmx_plan* p, int32_t on) {
   if (check_plan(p)) return 1;
   p->fuse_grad = on != 0;
+  if (choose_fusion(p)) {
+    // the descriptors are read by kernels that may still be in flight on any stream
+    WMX_CHECK(hipDeviceSynchronize());
+    WMX_CHECK(hipMemcpy(p->d_blks, p->hb.data(), sizeof(BlockDev) * p->nb, hipMemcpyHostToDevice));
+  }
   if (retile(p)) return 1;
   drop_graphs(p);
   return 0;
